@@ -71,9 +71,13 @@ struct PrefillScratch {
     // q2: rows [q hi | q lo] of 2 head_dim halves; p2: rows [P hi | P lo] of 2 t_pad halves (one GEMM sums both parts)
     void *xn = nullptr, *qkv = nullptr, *q2 = nullptr, *v_t = nullptr, *p2 = nullptr, *a = nullptr;
     void *g = nullptr, *u = nullptr, *mm = nullptr;
-    void *gemm_ws = nullptr; // fp32 partial sums of split-K products (short prompts)
+    void *gemm_ws = nullptr; // fp32 partial sums of split-K products (short prompts); f32 mode: also the parts of one operand
+    size_t gemm_ws_bytes = 0;
     bool gemm_attention = false; // the buffers of the two-GEMM form of attention (scores, p2) exist
     static constexpr size_t kGemmWsBytes = (size_t)64 << 20;
+    // f32 mode: three bf16 parts of an activation matrix (6 bytes per element: 85 MB for 1024 rows of 13824) beside the partial
+    // sums; a product whose rows need more runs in several passes over the weights
+    static constexpr size_t kGemmWsBytesF32 = (size_t)192 << 20;
     void release() {
         void *all[] = {x, h, scores, xn, qkv, q2, v_t, p2, a, g, u, mm, gemm_ws};
         for (void *b : all)
@@ -166,13 +170,14 @@ bool tunables_set(Tunables &t, const char *name, const char *value) {
     if (n == "GEMM_ROPE") return flag_off(t.gemm.no_rope_epilogue);
     if (n == "FINISH_NORM") return flag_off(t.gemm.no_finish_norm);
     if (n == "GEMM_KGROUP") return flag_off(t.gemm.no_kgroup);
+    if (n == "GEMM_SPLIT3") return flag_off(t.gemm.no_split3);
     return false;
 }
 
 void tunables_from_env(Tunables &t) {
     static const char *const names[] = {"GEMV_BURST", "ATTN_CHUNK", "ATTN_SINGLE_MAX", "ATTN_MERGE", "ATTN_LDS", "PREFILL_ATTN", "PREFILL_ATTN_ORDER",
                                         "DECODE_GRAPH", "DECODE_FOLD", "GEMM_TILE", "GEMM_SPLIT_K", "GEMM_SPLIT_HALF", "GEMM_DUAL", "GEMM_DUAL_CUT",
-                                        "GEMM_ROPE", "FINISH_NORM", "GEMM_KGROUP"};
+                                        "GEMM_ROPE", "FINISH_NORM", "GEMM_KGROUP", "GEMM_SPLIT3"};
     for (const char *name : names) {
         const std::string env = std::string("RLLAMA_HIP_") + name;
         const char *val = getenv(env.c_str());
@@ -914,13 +919,15 @@ static int ensure_prefill_scratch(rlh_model *m, int n) {
     A((void **)&S.g, N * F * es);
     if (es == 4) A((void **)&S.u, N * F * es); // f16 mode: w3's epilogue consumes its product on the spot
     A((void **)&S.mm, N * F * es);
-    A((void **)&S.gemm_ws, PrefillScratch::kGemmWsBytes);
+    const size_t ws_bytes = es == 4 ? PrefillScratch::kGemmWsBytesF32 : PrefillScratch::kGemmWsBytes;
+    if (e == hipSuccess) e = hipMalloc(&S.gemm_ws, ws_bytes); // (written before it is read, always)
     if (e == hipSuccess) e = hipStreamSynchronize(m->ctx->stream);
     if (e != hipSuccess) {
         S.release();
         return fail(e == hipErrorOutOfMemory ? RLH_ERR_OOM : RLH_ERR_HIP, "prefill work buffers for %d tokens: %s", n, hipGetErrorString(e));
     }
     S.n_cap = n;
+    S.gemm_ws_bytes = ws_bytes;
     S.gemm_attention = gemm_attention;
     S.t_pad = (int)tp;
     return RLH_OK;
@@ -969,7 +976,7 @@ static int enqueue_prefill(rlh_model *m, rlh_caches *c, const int32_t *tokens, i
         g.ldc = ldc;
         g.batch = 1;
         g.workspace = S.gemm_ws;
-        g.workspace_bytes = PrefillScratch::kGemmWsBytes;
+        g.workspace_bytes = S.gemm_ws_bytes;
         HIP_TRY(launch_gemm_f16(g, epi, st));
         return RLH_OK;
     };
@@ -1012,7 +1019,7 @@ static int enqueue_prefill(rlh_model *m, rlh_caches *c, const int32_t *tokens, i
             g.ldc = 3 * d;
             g.batch = 1;
             g.workspace = S.gemm_ws;
-            g.workspace_bytes = PrefillScratch::kGemmWsBytes;
+            g.workspace_bytes = S.gemm_ws_bytes;
             g.rope = rp;
             if (gemm_f16_rope_supported(g)) {
                 HIP_TRY(launch_gemm_f16(g, kGemmEpiRopeQkv, st));
@@ -1109,7 +1116,7 @@ static int enqueue_prefill(rlh_model *m, rlh_caches *c, const int32_t *tokens, i
             g.ldc = F;
             g.batch = 1;
             g.workspace = S.gemm_ws; // the same policy as rlh_ffn_gate: whether the pass runs is decided with the work memory in place
-            g.workspace_bytes = PrefillScratch::kGemmWsBytes;
+            g.workspace_bytes = S.gemm_ws_bytes;
             if (gemm_f16_dual_gate_supported(g)) {
                 HIP_TRY(launch_gemm_f16(g, kGemmEpiSiluGateF16, st));
             } else {
@@ -1182,7 +1189,7 @@ static int enqueue_prefill_f32(rlh_model *m, rlh_caches *c, const int32_t *token
         g.accumulate = accumulate;
         g.f32_operands = 1;
         g.workspace = S.gemm_ws;
-        g.workspace_bytes = PrefillScratch::kGemmWsBytes;
+        g.workspace_bytes = S.gemm_ws_bytes;
         HIP_TRY(launch_gemm_f16(g, kGemmEpiF32, st));
         return RLH_OK;
     };

@@ -32,9 +32,9 @@ struct OpScratch {
     size_t attn_ws_floats = 0;
     unsigned *tickets = nullptr;   // [kOpMaxHeads]
     int32_t *token = nullptr;      // one id
-    void *gemm_ws = nullptr;       // partial sums of products cut along K (kOpGemmWsBytes), as the forward's prompt path has
+    void *gemm_ws = nullptr;       // partial sums of products cut along K and the parts of an fp32 operand (kOpGemmWsBytes)
 };
-constexpr size_t kOpGemmWsBytes = (size_t)64 << 20;
+constexpr size_t kOpGemmWsBytes = (size_t)192 << 20;
 constexpr int kOpMaxHeads = 1024;
 
 // The library's switches.  Read from the environment (RLLAMA_HIP_<NAME>) once, when the context is made, and changed

@@ -761,6 +761,13 @@ static hipError_t launch_split_finish(const GemmParams &p, int splits, hipStream
     return hipGetLastError();
 }
 
+hipError_t launch_gemm_split_finish_f32(const GemmParams &p, const float *partial, int pieces, hipStream_t s) {
+    const size_t work = (size_t)p.m * (p.n / 4);
+    const unsigned blocks = (unsigned)((work + 255) / 256 < 4096 ? (work + 255) / 256 : 4096);
+    hipLaunchKernelGGL(gemm_split_finish_kernel<kGemmEpiF32>, dim3(blocks), dim3(256), 0, s, p, partial, pieces);
+    return hipGetLastError();
+}
+
 // Two products in one pass pay off where their workgroups fill the compute units about as well as the best single-product
 // tile does.  Returns 0 (two launches), 1 (workgroups of 256 x 192 of both products, eight wavefronts, all of the LDS),
 // 2 (128 x 192 of both, four wavefronts: prompts of about 300 to 512 rows, where the 128 x 128 tile of a single product needs two

@@ -1,0 +1,65 @@
+"""fp32 products on the bf16 matrix cores (three parts per value): against float64, against the fp32 matrix instruction, and the
+values the parts cannot hold."""
+import numpy as np
+import pytest
+
+from common import options
+from rllama_amd import Tensor
+
+pytestmark = pytest.mark.gpu
+f32 = np.float32
+
+
+def _product(ctx, a, b):
+    return Tensor.from_numpy(ctx, a).matrix_mul_transposed(Tensor.from_numpy(ctx, b)).to_numpy()
+
+
+# rows: one to eight 32-row tiles of a workgroup (with both parities of their split between the row groups), remainders, more than
+# one row tile; columns: less than, exactly and just over a tile of 128; k: one K-tile, fewer than the stages, cut along K
+@pytest.mark.parametrize("m,n,k", [(2, 128, 32), (33, 129, 96), (65, 300, 64), (97, 2816, 160), (128, 4096, 4096), (160, 130, 1184), (192, 384, 352),
+                                   (200, 3072, 1024), (255, 64, 512), (257, 515, 2048), (300, 4096, 4096)])
+def test_split3_product_against_float64(ctx, m, n, k):
+    rng = np.random.default_rng(m * 131 + n)
+    a = rng.standard_normal((m, k)).astype(f32)
+    b = (rng.standard_normal((n, k)) * 0.02).astype(f32)
+    exact = a.astype(np.float64) @ b.astype(np.float64).T
+    got = _product(ctx, a, b)
+    # 6 products of every 16 values of k are added one after the other, each addition rounded to at most 2^-24 of a partial sum
+    # that sum |a| |b| bounds (2^-23: the matrix cores may truncate), plus the parts left out (2^-24) and the pieces' sums (18)
+    bound = (np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64).T) * ((6 * k / 16 + 1 + 18) * 2.0 ** -23)
+    assert np.all(np.abs(got - exact) <= bound)
+    with options(ctx, GEMM_SPLIT3="0"):
+        plain = _product(ctx, a, b)
+    err, err_plain = (np.linalg.norm(x - exact) / np.linalg.norm(exact) for x in (got, plain))
+    assert err <= max(err_plain, 2.0 ** -24), (err, err_plain)
+
+
+def test_split3_product_with_infinities_nan_and_the_largest_values(ctx):
+    rng = np.random.default_rng(5)
+    m, n, k = 40, 3072, 256
+    a = rng.standard_normal((m, k)).astype(f32)
+    b = rng.standard_normal((n, k)).astype(f32)
+    a[3, 5], a[7, 9], a[11, 1], a[21, 3] = np.inf, -np.inf, np.nan, np.finfo(f32).max   # the last rounds to a bf16 infinity
+    b[50, 200], b[51, 5], b[60], b[70, 3] = np.inf, 0.0, 0.0, 1e-30
+    b[:, 3] *= f32(0.125)                                                                 # FLT_MAX times this stays finite ...
+    b[2000:, 3] *= f32(1000.0)                                                            # ... or overflows
+    with np.errstate(all="ignore"):
+        want = (a.astype(np.float64) @ b.astype(np.float64).T).astype(f32)
+    got = _product(ctx, a, b)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(np.isposinf(got), np.isposinf(want)) and np.array_equal(np.isneginf(got), np.isneginf(want))
+    ok = np.isfinite(want)
+    with np.errstate(all="ignore"):
+        bound = (np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64).T)[ok] * ((k + 20) * 2.0 ** -23)
+    assert np.all(np.abs(got[ok].astype(np.float64) - want[ok]) <= bound)
+
+
+def test_split3_product_in_passes_over_the_rows(ctx):
+    # 6 bytes per element of a: 1500 rows of 32768 need more than the work memory holds, so the rows go in several passes
+    rng = np.random.default_rng(6)
+    m, n, k = 1500, 96, 32768
+    a = rng.standard_normal((m, k), dtype=f32)
+    b = rng.standard_normal((n, k), dtype=f32)
+    exact = a.astype(np.float64) @ b.astype(np.float64).T
+    got = _product(ctx, a, b)
+    assert np.linalg.norm(got - exact) <= 2e-6 * np.linalg.norm(exact)  # sqrt(6 k / 16) roundings of 2^-24 is 6.6e-6 / 3 when they are independent
