@@ -170,6 +170,7 @@ bool tunables_set(Tunables &t, const char *name, const char *value) {
     if (n == "GEMM_ROPE") return flag_off(t.gemm.no_rope_epilogue);
     if (n == "FINISH_NORM") return flag_off(t.gemm.no_finish_norm);
     if (n == "GEMM_KGROUP") return flag_off(t.gemm.no_kgroup);
+    if (n == "GEMM_SKINNY") return flag_off(t.gemm.no_skinny);
     if (n == "GEMM_SPLIT3") return flag_off(t.gemm.no_split3);
     return false;
 }
@@ -177,7 +178,7 @@ bool tunables_set(Tunables &t, const char *name, const char *value) {
 void tunables_from_env(Tunables &t) {
     static const char *const names[] = {"GEMV_BURST", "ATTN_CHUNK", "ATTN_SINGLE_MAX", "ATTN_MERGE", "ATTN_LDS", "PREFILL_ATTN", "PREFILL_ATTN_ORDER",
                                         "DECODE_GRAPH", "DECODE_FOLD", "GEMM_TILE", "GEMM_SPLIT_K", "GEMM_SPLIT_HALF", "GEMM_DUAL", "GEMM_DUAL_CUT",
-                                        "GEMM_ROPE", "FINISH_NORM", "GEMM_KGROUP", "GEMM_SPLIT3"};
+                                        "GEMM_ROPE", "FINISH_NORM", "GEMM_KGROUP", "GEMM_SKINNY", "GEMM_SPLIT3"};
     for (const char *name : names) {
         const std::string env = std::string("RLLAMA_HIP_") + name;
         const char *val = getenv(env.c_str());

@@ -831,6 +831,7 @@ static int choose_dual(const GemmParams &p, int *cut_cols = nullptr) {
 
 bool gemm_f16_dual_gate_supported(const GemmParams &p) {
     int n1 = 0;
+    if (gemm_f16_skinny_supported(p, kGemmEpiSiluGateF16)) return true;
     return choose_dual(p, &n1) != 0;
 }
 
@@ -845,13 +846,14 @@ bool gemm_f16_rope_supported(const GemmParams &p) {
     for (const void *q : {(const void *)R.q_hi, (const void *)R.q_lo, (const void *)R.cache_k, (const void *)R.cache_v, (const void *)R.v_t})
         if (q == nullptr || (reinterpret_cast<uintptr_t>(q) % 16) != 0) return false;
     if (R.freqs == nullptr || (reinterpret_cast<uintptr_t>(R.freqs) % 8) != 0) return false;
-    return choose_split_k(p, choose_tile(p)) == 1;
+    return gemm_f16_skinny_supported(p, kGemmEpiRopeQkv) || choose_split_k(p, choose_tile(p)) == 1;
 }
 
 hipError_t launch_gemm_f16_dma(const GemmParams &p_in, int epilogue, hipStream_t s) {
     if (!gemm_f16_dma_supported(p_in) || p_in.m <= 0 || p_in.n <= 0 || p_in.batch < 1) return hipErrorInvalidValue;
     if (epilogue == kGemmEpiResAddF32 && (p_in.residual == nullptr || p_in.batch != 1)) return hipErrorInvalidValue;
     if (epilogue == kGemmEpiRopeQkv && !gemm_f16_rope_supported(p_in)) return hipErrorInvalidValue;
+    if (gemm_f16_skinny_supported(p_in, epilogue)) return launch_gemm_f16_skinny(p_in, epilogue, s);
     if (p_in.b2 != nullptr) {
         int n1 = 0;
         const int dual = epilogue == kGemmEpiSiluGateF16 ? choose_dual(p_in, &n1) : 0;

@@ -1,0 +1,69 @@
+"""f16 products of prompts of at most 16 rows."""
+import numpy as np
+import pytest
+
+from common import Shape, make_gpu, make_oracle, max_rel_err, synth_weights
+from rllama_amd import Tensor
+
+pytestmark = pytest.mark.gpu
+TOL_F16 = 1e-2  # relative, as the other whole-model tests: f16 rounding decisions flip with the order of sums
+
+
+def _f16(rng, rows, cols, std):
+    return (rng.standard_normal((rows, cols)) * std).astype(np.float16)
+
+
+def _exact(a, b):
+    """The float64 product and how far an f16-rounded fp32 sum may lie from it: half a unit in the last place of f16, and k / 16 + 16
+    additions that round (or truncate) to 2^-23 of a partial sum bounded by sum |a| |b|."""
+    a64, b64 = a.astype(np.float64), b.astype(np.float64)
+    exact = a64 @ b64.T
+    noise = (np.abs(a64) @ np.abs(b64).T) * ((a.shape[1] / 16 + 16) * 2.0 ** -23)
+    return exact, 0.5 * _ulp(np.abs(exact) + noise) + noise
+
+
+def _ulp(x):
+    return np.spacing(np.maximum(x, 2.0 ** -14).astype(np.float16)).astype(np.float64)
+
+
+def _check(got, a, b):
+    exact, tol = _exact(a, b)
+    assert np.all(np.abs(got.astype(np.float64) - exact) <= tol)
+
+
+def _check_gate(got, a, w1, w3):
+    """f16(silu(g) u) with g and u off by their tolerances: |silu'| <= 1.1, so |u| 1.1 dg + |silu(g)| du + 1.1 dg du, 1e-6 of the value for
+    the hardware exponential and reciprocal, and the last rounding."""
+    (g, dg), (u, du) = _exact(a, w1), _exact(a, w3)
+    silu = g / (1.0 + np.exp(-g))
+    tol = np.abs(u) * 1.1 * dg + np.abs(silu) * du + 1.1 * dg * du + 1e-6 * np.abs(silu * u)
+    assert np.all(np.abs(got.astype(np.float64) - silu * u) <= tol + 0.5 * _ulp(np.abs(silu * u) + tol))
+
+
+# k: one K-step for sixteen wavefronts, a burst and a remainder, several bursts; columns: less than a tile, a remainder, and more tiles than
+# the part has compute units once (8 wavefronts) and twice (4 wavefronts)
+@pytest.mark.parametrize("m,n,k", [(2, 8, 32), (16, 40, 1056), (7, 4099, 96), (15, 8216, 416), (16, 1024, 2080), (9, 2048, 2816)])
+def test_product_of_few_rows(ctx, m, n, k):
+    rng = np.random.default_rng(m + n + k)
+    a, b = _f16(rng, m, k, 1.0), _f16(rng, n, k, 0.05)
+    A, B = Tensor.from_numpy(ctx, a), Tensor.from_numpy(ctx, b)
+    _check(A.matrix_mul_transposed(B).to_numpy(), a, b)
+    if n % 8 == 0:
+        w3 = _f16(rng, n, k, 0.05)
+        _check_gate(A.ffn_gate(B, Tensor.from_numpy(ctx, w3)).to_numpy(), a, b, w3)
+
+
+@pytest.mark.parametrize("dim,heads,ffn", [(1024, 16, 2816), (256, 2, 704), (64, 4, 192)])
+@pytest.mark.parametrize("n", [2, 15, 16, 17])
+def test_prompt_of_few_rows(ctx, dim, heads, ffn, n):
+    """A whole prompt and the token behind it, head dimensions 64, 128 and 16: residual, SiLU-gate and RoPE / cache / V^T epilogues."""
+    shape = Shape(dim=dim, n_layers=2, n_heads=heads, ffn_hidden=ffn, vocab_size=64, max_seq_len=80)
+    W = synth_weights(shape, seed=91, std=0.05, norm_ones=False)
+    toks = np.random.default_rng(92).integers(0, shape.vocab_size, 71)
+    om, gm = make_oracle(shape, W, True), make_gpu(ctx, shape, W, True)
+    gc, oc = gm.make_caches(), om.make_caches()
+    gm.forward(toks[:70], 0, gc)  # leaves other rows' values in the work buffers
+    gc = gm.make_caches()
+    assert max_rel_err(gm.forward(toks[:n], 0, gc), om.forward(toks[:n], 0, oc)) < TOL_F16
+    assert max_rel_err(gm.forward(toks[n:n + 1], n, gc), om.forward(toks[n:n + 1], n, oc)) < TOL_F16
+    gm.free()
