@@ -579,7 +579,7 @@ static int device_compute_units() {
 // larger tiles are more efficient (less L2 -> LDS traffic per flop) but leave compute units idle on small outputs.
 static int choose_tile(const GemmParams &p, double *model_time = nullptr) {
     const int forced = p.tune.tile_plus1 - 1; // -1: by the model below
-    if (forced >= 1 && forced <= 3) return forced;
+    if ((forced >= 1 && forced <= 3) || (forced >= 5 && forced <= 7 && p.k * (p.f32_operands ? 2 : 1) % 64 == 0)) return forced;
     const int k_halves = p.k * (p.f32_operands ? 2 : 1);
     if (forced == 0 && k_halves % 64 == 0) return 0;
     const int n_cu = device_compute_units();
@@ -721,12 +721,34 @@ __global__ __launch_bounds__(256) void gemm_split_finish_norm_kernel(GemmParams 
     }
 }
 
+// Products whose K is short: the lowest of the 32 / 64 / 128-row x 64-column tiles with which all workgroups run in one round, or -1.
+// A workgroup then takes about 3 us + K x 4.1 / 4.7 / 5.4 ns whatever the number of workgroups, which beats a cut along K (two
+// launches) and half-empty 128 x 128 tiles until K x 4.1 ns outgrows them; with few workgroups the cut wins earlier.  Former choice ->
+// this, us: 3072 x 1024 weights, 40 / 131 / 300 / 600 rows: 11.8 / 13.8 / 15.5 / 20.4 -> 7.4 / 7.8 / 9.4 / 11.0; 6144 x 2048, 20 / 40 / 80 / 200:
+// 17.2 / 22.0 / 26.0 / 18.4 -> 11.8 / 12.0 / 13.8 / 16.8; 3072 x 3072, 20 / 131 / 300: 19.5 / 25.8 / 20.3 -> 15.5 / 16.5 / 19.9; 1024 x 2816, 131 / 300:
+// 15.4 / 26.2 -> 14.6 / 15.0, but 20 / 40 rows (16 / 32 workgroups): 11.3 / 13.5 against 14.5 / 14.6; 4096 x 4096, 80 rows: 18.7 against 20.2.
+static int choose_narrow(const GemmParams &p) {
+    if (p.f32_operands || p.batch != 1 || p.split_k > 1 || p.k_seg != 0 || p.causal != 0 || p.b2 != nullptr || p.k % 64 != 0 || p.k > 3072) return -1;
+    if (p.tune.tile_plus1 != 0 || p.tune.split_k > 1) return -1;
+    const int heights[3] = {32, 64, 128}, tiles[3] = {6, 7, 5};
+    const long n_cu = device_compute_units(), least = p.k <= 1024 ? 1 : p.k <= 2048 ? n_cu / 8 : n_cu / 8 + 1;
+    for (int i = 0; i < 3; i++) {
+        const long blocks = (long)((p.n + 63) / 64) * ((p.m + heights[i] - 1) / heights[i]);
+        if (blocks > n_cu) continue;
+        // a cut product brings the RMSNorm behind it along (gemm_split_finish_norm_kernel), which this leaves to a launch of its own: worth it
+        // only where the cut is one for lack of workgroups (2048 x 2048 at 600 rows and 3072 x 3072 at 300 rows lose 2 % of the prompt)
+        if (i > 0 && p.norm_w != nullptr && (long)((p.n + 127) / 128) * ((p.m + 127) / 128) > n_cu / 4) return -1;
+        return blocks >= least ? tiles[i] : -1;
+    }
+    return -1;
+}
+
 // Products with few output tiles (few prompt rows) leave most compute units without a workgroup, and what bounds them is
 // streaming the weights once: the K range is then cut into split_k pieces that run as separate workgroups (more weight bytes
 // in flight, every compute unit busy), their fp32 partial sums go to the caller's workspace and a second small kernel adds
 // them and applies the epilogue.  Returns 1 for "run as one product".
 static int choose_split_k(const GemmParams &p, int tile) {
-    if (p.workspace == nullptr || p.batch != 1 || p.k_seg != 0 || p.causal != 0) return 1;
+    if (p.workspace == nullptr || p.batch != 1 || p.k_seg != 0 || p.causal != 0 || choose_narrow(p) >= 0) return 1;
     const int k_halves = p.k * (p.f32_operands ? 2 : 1);
     if (tile != 0 || (p.n % 4) != 0 || (p.ldc % 4) != 0 || k_halves % 64 != 0) return 1;
     const int forced = p.tune.split_k;
@@ -771,7 +793,8 @@ hipError_t launch_gemm_split_finish_f32(const GemmParams &p, const float *partia
 // Two products in one pass pay off where their workgroups fill the compute units about as well as the best single-product
 // tile does.  Returns 0 (two launches), 1 (workgroups of 256 x 192 of both products, eight wavefronts, all of the LDS),
 // 2 (128 x 192 of both, four wavefronts: prompts of about 300 to 512 rows, where the 128 x 128 tile of a single product needs two
-// rounds of workgroups and this form one) or 3 / 4 / 5 (32 / 64 / 128 rows x 64 columns of both: short prompts).  The model is choose_tile's: rounds of workgroups x outputs per workgroup / relative
+// rounds of workgroups and this form one) or 3 / 4 / 5 / 6 / 7 (32 / 64 / 128 / 192 / 256 rows x 64 columns of both: prompts of up to
+// 256 rows).  The model is choose_tile's: rounds of workgroups x outputs per workgroup / relative
 // throughput of a busy compute unit, with 1.23 x 1.18 measured for the 256-row form (7B and 13B shapes, 256 to 2048 prompt
 // rows: faster from 768 rows on except where the last round is nearly empty) and 0.87 for the 128-row form (7B shape: 3 - 4 % of
 // the time to the first token at 384 and 512 rows, slower at 256 and 640).
@@ -780,19 +803,24 @@ hipError_t launch_gemm_split_finish_f32(const GemmParams &p, const float *partia
 // rows: 576 = 2.25 rounds of 256), the bit costs a whole round, and as two small products it costs a fraction of one.
 static int choose_dual(const GemmParams &p, int *cut_cols = nullptr) {
     if (cut_cols != nullptr) *cut_cols = 0;
-    const int mode = p.tune.dual_plus1 - 1; // 0: never, 1 ... 5: that form wherever the kernel can run (tests), -1: by shape
+    const int mode = p.tune.dual_plus1 - 1; // 0: never, 1 ... 7: that form wherever the kernel can run (tests), -1: by shape
     if (mode == 0 || p.f32_operands || !gemm_f16_dma_supported(p) || p.batch != 1 || p.k_seg != 0 || p.causal != 0 || p.k % 64 != 0) return 0;
     if ((p.ldc % 8) != 0 || (p.n % 8) != 0 || (reinterpret_cast<uintptr_t>(p.c) % 16) != 0) return 0;
-    if (mode >= 1 && mode <= 5) return mode;
+    if (mode >= 1 && mode <= 7) return mode;
     // Up to 128 rows both products are bound by streaming their weights once, and one launch whose workgroups each take 64
     // rows of w1 and the same 64 of w3 streams them at the rate of the single-row kernel (7B shape: 29.8 / 34.3 / 40.0 us at
     // 16 / 48 / 128 rows against 41.7 / 49.1 / 60.3 us for two launches on 64 rows per workgroup; the single-row pair: 29.9).
     // Beyond one round of such workgroups (65B shape: 344) only the 32-row form still gains (168 against 184 us).
-    if (p.m <= 128) {
-        const bool one_round = (p.n + 63) / 64 <= device_compute_units();
-        if (p.m <= 32) return 3;
-        if (one_round) return p.m <= 64 ? 4 : 5;
-    }
+    if (p.m <= 32) return 3;
+    // More rows: the lowest row tile with which all workgroups run in one round (a taller one only leaves compute units idle, and
+    // two launches of 128 x 128 tiles cover 129 to 256 rows with two row tiles, the second mostly padding).  Former choice -> this, us:
+    // 2816 x 1024 weights, 40 / 80 / 131 / 200 / 300 / 600 rows: 11.3 / 12.1 / 27.0 / 30.1 / 30.7 / 37.7 -> 10.4 / 10.3 / 10.4 / 12.1 / 12.5 / 14.1;
+    // 5632 x 2048, 131 / 200 / 400 rows: 36.7 / 38.7 / 48.1 -> 22.4 / 22.6 / 36.7; 7B shape, 131 / 160 / 192 / 256: 96 / 95 / 95 / 97 -> 62 / 60 /
+    // 65 / 80; 13B shape: 124 / 123 / 129 / 132 -> 91 / 91 / 96 / 115.  Beyond one round (65B shape, 344 workgroups) it gains 4 % up to
+    // 192 rows and loses 16 % at 256.
+    const int heights[5] = {32, 64, 128, 192, 256};
+    for (int i = 0; i < 5; i++)
+        if ((long)((p.n + 63) / 64) * ((p.m + heights[i] - 1) / heights[i]) <= device_compute_units()) return 3 + i;
     double single = 0.0;
     const int tile = choose_tile(p, &single);
     if (tile < 0 || tile > 3 || choose_split_k(p, tile) != 1) return 0;
@@ -879,6 +907,8 @@ hipError_t launch_gemm_f16_dma(const GemmParams &p_in, int epilogue, hipStream_t
         if (dual == 3) return launch_dma<kGemmEpiSiluGateF16, 1, 1, 64, 7, false, 1, true>(p_in, s); // 32 x 64 of both, two wavefronts
         if (dual == 4) return launch_dma<kGemmEpiSiluGateF16, 1, 1, 64, 6, false, 2, true>(p_in, s); // 64 x 64 of both, two wavefronts
         if (dual == 5) return launch_dma<kGemmEpiSiluGateF16, 2, 1, 64, 4, false, 2, true>(p_in, s); // 128 x 64 of both, four wavefronts
+        if (dual == 6) return launch_dma<kGemmEpiSiluGateF16, 2, 1, 64, 4, false, 3, true>(p_in, s); // 192 x 64 of both, four wavefronts
+        if (dual == 7) return launch_dma<kGemmEpiSiluGateF16, 2, 1, 64, 3, false, 4, true>(p_in, s); // 256 x 64 of both, four wavefronts
         return hipErrorInvalidValue;
     }
     if (epilogue == kGemmEpiSiluGateF16 && (p_in.gate == nullptr || p_in.batch != 1 || p_in.f32_operands)) return hipErrorInvalidValue;
@@ -911,7 +941,8 @@ hipError_t launch_gemm_f16_dma(const GemmParams &p_in, int epilogue, hipStream_t
         }
     }
     const GemmParams &p = p_in;
-    int tile = choose_tile(p);
+    const int narrow = choose_narrow(p);
+    int tile = narrow >= 0 ? narrow : choose_tile(p);
     if (tile == 0) {
         // With at most one workgroup per compute unit anyway, the LDS that a second one would need buys a deeper load
         // pipeline instead (measured on the wo / w2 products of a 1024-token 7B prefill: 108 -> 85 us per launch).

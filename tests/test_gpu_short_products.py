@@ -1,8 +1,9 @@
-"""f16 products of prompts of at most 16 rows."""
+"""f16 products of short prompts: the kernel for at most 16 rows, and the row heights of the 64-column tiles that keep a product
+(or w1 and w3 in one pass) in one round of workgroups."""
 import numpy as np
 import pytest
 
-from common import Shape, make_gpu, make_oracle, max_rel_err, synth_weights
+from common import Shape, make_gpu, make_oracle, max_rel_err, options, synth_weights
 from rllama_amd import Tensor
 
 pytestmark = pytest.mark.gpu
@@ -67,3 +68,16 @@ def test_prompt_of_few_rows(ctx, dim, heads, ffn, n):
     assert max_rel_err(gm.forward(toks[:n], 0, gc), om.forward(toks[:n], 0, oc)) < TOL_F16
     assert max_rel_err(gm.forward(toks[n:n + 1], n, gc), om.forward(toks[n:n + 1], n, oc)) < TOL_F16
     gm.free()
+
+
+# 44 column tiles: row tiles of 32 up to 160 rows, of 64 to 320, of 128 to 640, of 192 to 960, of 256 to 1280; 16 and 48 column tiles
+@pytest.mark.parametrize("m,n,k", [(33, 2816, 1024), (160, 2816, 128), (161, 2816, 1024), (321, 2816, 64), (641, 2816, 64), (961, 2816, 64), (600, 1024, 2816),
+                                   (40, 1024, 2816), (130, 3072, 3072), (300, 3000, 1024)])
+def test_lowest_row_tile_in_one_round(ctx, m, n, k):
+    rng = np.random.default_rng(m + n + k)
+    a, b, w3 = _f16(rng, m, k, 1.0), _f16(rng, n, k, 0.05), _f16(rng, n, k, 0.05)
+    A, B, W3 = (Tensor.from_numpy(ctx, t) for t in (a, b, w3))
+    _check(A.matrix_mul_transposed(B).to_numpy(), a, b)
+    got = A.ffn_gate(B, W3).to_numpy()
+    with options(ctx, GEMM_DUAL="1"):  # another tile, the same order of additions
+        assert np.array_equal(got, A.ffn_gate(B, W3).to_numpy())
