@@ -7,6 +7,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <map>
 #include <mutex>
 
 namespace rlh {
@@ -37,6 +38,35 @@ struct OpScratch {
 constexpr size_t kOpGemmWsBytes = (size_t)192 << 20;
 constexpr int kOpMaxHeads = 1024;
 
+// Device buffers of freed op-level tensors, kept for the next tensor of the same size: an operation's result is a new tensor, and
+// hipMalloc + hipFree (which waits for the device) cost more than the operation.  Everything that touches a tensor's buffer is
+// ordered on the context's one stream, so a buffer may be handed out while work of its former owner is still queued.  Bounded in the
+// size of a buffer and in total, guarded by the context's lock, given back when memory runs out and by rlh_shutdown.
+struct TensorPool {
+    static constexpr size_t kMaxBuffer = (size_t)8 << 20, kMaxTotal = (size_t)64 << 20;
+    std::multimap<size_t, void *> free_buffers; // by size in bytes
+    size_t total = 0;
+    void *take(size_t bytes) {
+        auto it = free_buffers.find(bytes);
+        if (it == free_buffers.end()) return nullptr;
+        void *p = it->second;
+        free_buffers.erase(it);
+        total -= bytes;
+        return p;
+    }
+    bool give(void *p, size_t bytes) {
+        if (bytes > kMaxBuffer || total + bytes > kMaxTotal) return false;
+        free_buffers.emplace(bytes, p);
+        total += bytes;
+        return true;
+    }
+    void release() { // the caller has waited for the stream
+        for (auto &kv : free_buffers) (void)hipFree(kv.second);
+        free_buffers.clear();
+        total = 0;
+    }
+};
+
 // The library's switches.  Read from the environment (RLLAMA_HIP_<NAME>) once, when the context is made, and changed
 // afterwards only through rlh_set_option under the context lock: no launch path reads the environment.
 struct Tunables {
@@ -65,6 +95,7 @@ struct rlh_ctx {
     hipDeviceProp_t prop;
     std::recursive_mutex mu;
     OpScratch ops;
+    TensorPool pool;
     Tunables tun;
     unsigned tun_version = 0;        // bumped by rlh_set_option: captured decode steps of an older version are dropped
     void *noalloc_scratch = nullptr; // this device's address of the library's static work memory (api_ops.hip)
