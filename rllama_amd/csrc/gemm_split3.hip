@@ -327,7 +327,8 @@ struct Split3Plan {
 // What a pass over `m` rows needs: row tiles of equal height, pieces along K by a model of the time in microseconds --
 // rounds of workgroups x (K-tiles of a piece x its cycles + 4 us to start and drain), and for a cut product the partial sums written
 // and read back at 4 TB/s and the launch that adds them.  Cycles of a K-tile: 384 MFMA cycles per SIMD and 32-row tile + 400 for
-// the barrier and the decomposition of B's first fragments.
+// the barrier and the decomposition of B's first fragments.  (A lone product measures 0.75 / 1.5 / 2.5 us per K-tile with one / four /
+// eight 32-row tiles; with those in the model it cuts finer, which loses: 11008 x 4096, 8 / 200 rows 53 / 154 -> 63 / 157 us.)
 static Split3Plan plan_split3(const GemmParams &p, int n_cu) {
     Split3Plan best;
     const size_t row_bytes = (size_t)p.k * 6;
