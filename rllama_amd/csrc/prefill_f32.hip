@@ -8,7 +8,7 @@ namespace rlh {
 
 // RMSNorm::forward per row (transformer.rs:476-480).  One workgroup per row; rows of up to 256 x 4 x kNormF32Vecs floats are read once, in
 // 16-byte pieces that stay in registers, with the weights requested in front of the row sum.  Bound by its memory latencies: 200 rows of
-// 4096, one element per load and two passes 11.1 us, this way 5.4.
+// 4096, one element per load and two passes 11.1 us, this way 5.1.
 constexpr int kNormF32Vecs = 8;
 __global__ __launch_bounds__(256) void rmsnorm_rows_f32_kernel(float *y, const float *x, const float *w, int d, float eps) {
     __shared__ float red[16];
