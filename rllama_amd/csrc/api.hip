@@ -162,10 +162,10 @@ bool tunables_set(Tunables &t, const char *name, const char *value) {
     if (n == "PREFILL_ATTN_ORDER") { t.prefill_attn_order = reset ? dflt.prefill_attn_order : v; return reset || (v >= 0 && v <= 2); }
     if (n == "DECODE_GRAPH") { t.decode_graph = reset ? 0 : (v != 0); return true; }
     if (n == "DECODE_FOLD") { t.decode_fold = reset ? 1 : (v != 0); return true; }
-    if (n == "GEMM_TILE") { t.gemm.tile_plus1 = reset ? 0 : v + 1; return reset || (v >= 0 && v <= 7 && v != 4); }
+    if (n == "GEMM_TILE") { t.gemm.tile_plus1 = reset ? 0 : v + 1; return reset || (v >= 0 && v <= 3); }
     if (n == "GEMM_SPLIT_K") { t.gemm.split_k = reset ? 0 : v; return reset || v >= 0; }
     if (n == "GEMM_SPLIT_HALF") return flag_off(t.gemm.no_split_half);
-    if (n == "GEMM_DUAL") { t.gemm.dual_plus1 = reset ? 0 : v + 1; return reset || (v >= 0 && v <= 7); }
+    if (n == "GEMM_DUAL") { t.gemm.dual_plus1 = reset ? 0 : v + 1; return reset || (v >= 0 && v <= 5); }
     if (n == "GEMM_DUAL_CUT") return flag_off(t.gemm.no_dual_cut);
     if (n == "GEMM_ROPE") return flag_off(t.gemm.no_rope_epilogue);
     if (n == "FINISH_NORM") return flag_off(t.gemm.no_finish_norm);

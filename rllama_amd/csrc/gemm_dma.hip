@@ -579,7 +579,7 @@ static int device_compute_units() {
 // larger tiles are more efficient (less L2 -> LDS traffic per flop) but leave compute units idle on small outputs.
 static int choose_tile(const GemmParams &p, double *model_time = nullptr) {
     const int forced = p.tune.tile_plus1 - 1; // -1: by the model below
-    if ((forced >= 1 && forced <= 3) || (forced >= 5 && forced <= 7 && p.k * (p.f32_operands ? 2 : 1) % 64 == 0)) return forced;
+    if (forced >= 1 && forced <= 3) return forced;
     const int k_halves = p.k * (p.f32_operands ? 2 : 1);
     if (forced == 0 && k_halves % 64 == 0) return 0;
     const int n_cu = device_compute_units();
@@ -721,14 +721,14 @@ __global__ __launch_bounds__(256) void gemm_split_finish_norm_kernel(GemmParams 
     }
 }
 
-// Products whose K is short: the lowest of the 32 / 64 / 128-row x 64-column tiles with which all workgroups run in one round, or -1.
+// Products with 1024 to 3072 values of k: the lowest of the 32 / 64 / 128-row x 64-column tiles with which all workgroups run in one round, or -1.
 // A workgroup then takes about 3 us + K x 4.1 / 4.7 / 5.4 ns whatever the number of workgroups, which beats a cut along K (two
 // launches) and half-empty 128 x 128 tiles until K x 4.1 ns outgrows them; with few workgroups the cut wins earlier.  Former choice ->
 // this, us: 3072 x 1024 weights, 40 / 131 / 300 / 600 rows: 11.8 / 13.8 / 15.5 / 20.4 -> 7.4 / 7.8 / 9.4 / 11.0; 6144 x 2048, 20 / 40 / 80 / 200:
 // 17.2 / 22.0 / 26.0 / 18.4 -> 11.8 / 12.0 / 13.8 / 16.8; 3072 x 3072, 20 / 131 / 300: 19.5 / 25.8 / 20.3 -> 15.5 / 16.5 / 19.9; 1024 x 2816, 131 / 300:
 // 15.4 / 26.2 -> 14.6 / 15.0, but 20 / 40 rows (16 / 32 workgroups): 11.3 / 13.5 against 14.5 / 14.6; 4096 x 4096, 80 rows: 18.7 against 20.2.
 static int choose_narrow(const GemmParams &p) {
-    if (p.f32_operands || p.batch != 1 || p.split_k > 1 || p.k_seg != 0 || p.causal != 0 || p.b2 != nullptr || p.k % 64 != 0 || p.k > 3072) return -1;
+    if (p.f32_operands || p.batch != 1 || p.split_k > 1 || p.k_seg != 0 || p.causal != 0 || p.b2 != nullptr || p.k % 64 != 0 || p.k < 1024 || p.k > 3072) return -1; // (measured from 1024 on)
     if (p.tune.tile_plus1 != 0 || p.tune.split_k > 1) return -1;
     const int heights[3] = {32, 64, 128}, tiles[3] = {6, 7, 5};
     const long n_cu = device_compute_units(), least = p.k <= 1024 ? 1 : p.k <= 2048 ? n_cu / 8 : n_cu / 8 + 1;
@@ -803,10 +803,10 @@ hipError_t launch_gemm_split_finish_f32(const GemmParams &p, const float *partia
 // rows: 576 = 2.25 rounds of 256), the bit costs a whole round, and as two small products it costs a fraction of one.
 static int choose_dual(const GemmParams &p, int *cut_cols = nullptr) {
     if (cut_cols != nullptr) *cut_cols = 0;
-    const int mode = p.tune.dual_plus1 - 1; // 0: never, 1 ... 7: that form wherever the kernel can run (tests), -1: by shape
+    const int mode = p.tune.dual_plus1 - 1; // 0: never, 1 ... 5: that form wherever the kernel can run (tests), -1: by shape
     if (mode == 0 || p.f32_operands || !gemm_f16_dma_supported(p) || p.batch != 1 || p.k_seg != 0 || p.causal != 0 || p.k % 64 != 0) return 0;
     if ((p.ldc % 8) != 0 || (p.n % 8) != 0 || (reinterpret_cast<uintptr_t>(p.c) % 16) != 0) return 0;
-    if (mode >= 1 && mode <= 7) return mode;
+    if (mode >= 1 && mode <= 5) return mode;
     // Up to 128 rows both products are bound by streaming their weights once, and one launch whose workgroups each take 64
     // rows of w1 and the same 64 of w3 streams them at the rate of the single-row kernel (7B shape: 29.8 / 34.3 / 40.0 us at
     // 16 / 48 / 128 rows against 41.7 / 49.1 / 60.3 us for two launches on 64 rows per workgroup; the single-row pair: 29.9).
@@ -819,7 +819,7 @@ static int choose_dual(const GemmParams &p, int *cut_cols = nullptr) {
     // 65 / 80; 13B shape: 124 / 123 / 129 / 132 -> 91 / 91 / 96 / 115.  Beyond one round (65B shape, 344 workgroups) it gains 4 % up to
     // 192 rows and loses 16 % at 256.
     const int heights[5] = {32, 64, 128, 192, 256};
-    for (int i = 0; i < 5; i++)
+    for (int i = 0; i < 5 && (p.m <= 128 || p.k >= 512); i++) // (measured from k = 512 on beyond 128 rows)
         if ((long)((p.n + 63) / 64) * ((p.m + heights[i] - 1) / heights[i]) <= device_compute_units()) return 3 + i;
     double single = 0.0;
     const int tile = choose_tile(p, &single);

@@ -131,7 +131,8 @@ static int compute_units() {
 
 bool gemm_f16_skinny_supported(const GemmParams &p, int epilogue) {
     if (p.tune.no_skinny || p.tune.dual_plus1 != 0 || p.tune.tile_plus1 != 0 || p.tune.split_k != 0 || p.f32_operands || p.batch != 1 || p.split_k > 1 || p.k_seg != 0 || p.causal != 0) return false;
-    if (p.m < 1 || p.m > 16 || p.n < 1 || p.k < 32 || p.k % 32 != 0 || p.lda % 8 != 0 || p.ldb % 8 != 0) return false;
+    if (p.m < 1 || p.m > 16 || p.n < 1 || p.k < 1024 || p.k % 32 != 0 || p.lda % 8 != 0 || p.ldb % 8 != 0) return false;
+    // (shorter rows than 1024 leave sixteen wavefronts less than two K-steps each and stay on the tiled kernels)
     // Fragments of 16 rows are 64 bytes per row and load instruction, which the memory path takes at about 4.7 TB/s; large products
     // are faster through LDS in whole lines in spite of their second kernel (7B shape, 8 rows: w1|w3 42 us here, 36 there)
     if ((size_t)p.n * p.k * (p.b2 != nullptr ? 4 : 2) > ((size_t)48 << 20)) return false;

@@ -127,10 +127,10 @@ enum GemmEpilogue {
 // Switches of the prompt-path products; all zero = the launchers' own choices.  They come from the context (parsed from the
 // environment once, when the context is made; rlh_set_option changes them), never from the environment at launch time.
 struct GemmTune {
-    int tile_plus1;       // GEMM_TILE=0..3, 5..7 forces the tile (128x128, 256x128, 256x192, 256x256; 128x64, 32x64, 64x64): stored as tile + 1
+    int tile_plus1;       // GEMM_TILE=0..3 forces the tile (128x128, 256x128, 256x192, 256x256): stored as tile + 1
     int split_k;          // GEMM_SPLIT_K=N forces N K-pieces for the products that qualify for a cut along K
     int no_split_half;    // GEMM_SPLIT_HALF=0: cut along K only when the tiles cover at most a quarter of the compute units
-    int dual_plus1;       // GEMM_DUAL=0..7: w1 and w3 in one pass never (0) / in that form wherever the kernel can run: stored as mode + 1
+    int dual_plus1;       // GEMM_DUAL=0..5: w1 and w3 in one pass never (0) / in that form wherever the kernel can run: stored as mode + 1
     int no_dual_cut;      // GEMM_DUAL_CUT=0: the one-pass w1|w3 product always covers all columns
     int no_rope_epilogue; // GEMM_ROPE=0: RoPE, q hi/lo, cache rows and V^T as a kernel of their own on the stored wq|wk|wv product
     int no_finish_norm;   // FINISH_NORM=0: the RMSNorm after a split wo / w2 product as a kernel of its own
