@@ -34,6 +34,7 @@
 // pieces by gemm_split_finish_kernel).
 #include "kernels.h"
 #include "device_utils.h"
+#include "split3_plan.h"
 
 #include <type_traits>
 
@@ -43,8 +44,6 @@ typedef __attribute__((ext_vector_type(16))) float float16_t;
 typedef __attribute__((ext_vector_type(8))) float float8_t;
 typedef __attribute__((ext_vector_type(8))) __bf16 bf8_t;
 
-constexpr int kS3K = 32;        // k values per K-tile
-constexpr int kS3Cols = 128;    // columns of a workgroup's tile
 constexpr int kS3Waves = 8;
 constexpr int kS3BStage = kS3Cols * kS3K * 4;
 constexpr int s3_a_stage(int t) { return 3 * t * 32 * kS3K * 2; }
@@ -316,49 +315,6 @@ static hipError_t launch_split3(const Split3Params &p, hipStream_t s) {
     return hipGetLastError();
 }
 
-struct Split3Plan {
-    int rows = 0;      // rows of A per pass over B (what the planes have room for)
-    int tiles = 0;     // 32-row tiles per workgroup
-    int m_pad = 0;     // of a full pass
-    int pieces = 1;
-    size_t planes_bytes = 0;
-};
-
-// What a pass over `m` rows needs: row tiles of equal height, pieces along K by a model of the time in microseconds --
-// rounds of workgroups x (K-tiles of a piece x its cycles + 4 us to start and drain), and for a cut product the partial sums written
-// and read back at 4 TB/s and the launch that adds them.  Cycles of a K-tile: 384 MFMA cycles per SIMD and 32-row tile + 400 for
-// the barrier and the decomposition of B's first fragments.  (A lone product measures 0.75 / 1.5 / 2.5 us per K-tile with one / four /
-// eight 32-row tiles; with those in the model it cuts finer, which loses: 11008 x 4096, 8 / 200 rows 53 / 154 -> 63 / 157 us.)
-static Split3Plan plan_split3(const GemmParams &p, int n_cu) {
-    Split3Plan best;
-    const size_t row_bytes = (size_t)p.k * 6;
-    const int cap = (int)((p.workspace_bytes / row_bytes) & ~(size_t)31);
-    int rows = p.m;
-    if (((rows + 31) & ~31) > cap) rows = cap / 256 * 256;
-    if (rows <= 0) return best;
-    const int row_tiles = (rows + 255) / 256;
-    best.rows = rows;
-    best.tiles = ((rows + row_tiles - 1) / row_tiles + 31) / 32;
-    best.m_pad = row_tiles * best.tiles * 32;
-    best.planes_bytes = row_bytes * best.m_pad;
-    if (best.planes_bytes > p.workspace_bytes) return Split3Plan();
-    const int kt = p.k / kS3K;
-    const long tiles = (long)((p.n + kS3Cols - 1) / kS3Cols) * row_tiles;
-    const double us_kt = (384.0 * best.tiles + 400.0) / 2200.0;
-    const size_t room = p.workspace_bytes - best.planes_bytes, per = (size_t)rows * p.n * 4;
-    double best_t = 0.0;
-    for (int s = 1; s <= 16 && (s == 1 || kt / s >= 4); s++) {
-        if (s > 1 && ((size_t)s * per > room || p.n % 4 != 0 || p.ldc % 4 != 0)) break;
-        const long rounds = (tiles * s + n_cu - 1) / n_cu;
-        const double t = rounds * (((kt + s - 1) / s) * us_kt + 4.0) + (s > 1 ? 5.0 + s * (double)per * 2.0 / 4e6 : 0.0);
-        if (s == 1 || t < best_t) {
-            best.pieces = s;
-            best_t = t;
-        }
-    }
-    return best;
-}
-
 static int compute_units() {
     static const int n_cu = [] {
         int dev = 0, cu = 256;
@@ -379,7 +335,7 @@ bool gemm_split3_supported(const GemmParams &p, int epilogue) {
     // 16 / 26 against 19 / 29; but 1536 x 1536 20 / 31 against 17 / 28, 2048 x 4096 at 200 rows 56 against 50)
     const int tiles64 = (p.n + 63) / 64;
     if (((p.n <= 1024 && p.m <= 256) || (p.n <= 2048 && p.m <= 128)) && compute_units() % tiles64 == 0) return false;
-    return plan_split3(p, compute_units()).rows > 0;
+    return plan_split3(p.m, p.n, p.k, p.ldc, p.workspace_bytes, compute_units()).rows > 0; // the first pass, and with it every one
 }
 
 hipError_t launch_gemm_split3(const GemmParams &p, int epilogue, hipStream_t s) {
@@ -389,7 +345,7 @@ hipError_t launch_gemm_split3(const GemmParams &p, int epilogue, hipStream_t s) 
         part.m = p.m - r0;
         part.a = reinterpret_cast<const half_t *>(reinterpret_cast<const float *>(p.a) + (size_t)r0 * p.lda);
         part.c = reinterpret_cast<float *>(p.c) + (size_t)r0 * p.ldc;
-        const Split3Plan plan = plan_split3(part, compute_units());
+        const Split3Plan plan = plan_split3(part.m, p.n, p.k, p.ldc, p.workspace_bytes, compute_units());
         if (plan.rows <= 0) return hipErrorInvalidValue;
         part.m = plan.rows;
         unsigned char *planes = reinterpret_cast<unsigned char *>(p.workspace);

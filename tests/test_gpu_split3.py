@@ -54,10 +54,10 @@ def test_split3_product_with_infinities_nan_and_the_largest_values(ctx):
     assert np.all(np.abs(got[ok].astype(np.float64) - want[ok]) <= bound)
 
 
-def test_split3_product_in_passes_over_the_rows(ctx):
-    # 6 bytes per element of a: 1500 rows of 32768 need more than the work memory holds, so the rows go in several passes
+@pytest.mark.parametrize("m,n,k", [(1500, 96, 32768), (1537, 96, 40960)])  # the second: rows left after a pass pad to more than the capacity
+def test_split3_product_in_passes_over_the_rows(ctx, m, n, k):
+    # 6 bytes per element of a: the rows need more than the work memory holds, so they go in several passes
     rng = np.random.default_rng(6)
-    m, n, k = 1500, 96, 32768
     a = rng.standard_normal((m, k), dtype=f32)
     b = rng.standard_normal((n, k), dtype=f32)
     exact = a.astype(np.float64) @ b.astype(np.float64).T
