@@ -401,7 +401,7 @@ __global__ __launch_bounds__(128 * kWavesM) void gemm_f16_dma_kernel(GemmParams 
             for (int j = 0; j < kNT; j++)
 #pragma unroll
                 for (int v = 0; v < 16; v++) tile[(i * 32 + (v >> 2) * 8 + row_in + (v & 3)) * kTS + j * 32 + col_in] = (half_t)acc[i][j][v];
-        rope_qkv_from_tile<kWR, kTW, kTS>(tile, lane, bm0 + wm * kWR, bn0 + wn * kTW, M, N, R);
+        rope_qkv_from_tile<kWR, kTW, kTS>(tile, lane, bm0 + wm * kWR, bn0 + wn * kTW, M, N, (int)gridDim.y * kBM, R);
         return;
     }
     if constexpr (kEpi == kGemmEpiF16 || kEpi == kGemmEpiSiluGateF16) {

@@ -10,9 +10,9 @@ namespace rlh {
 // LDS at `tile` (first row = position wr0, first column wc0 of the [m x 3 dim] product): handled in 16-byte pieces of 8
 // consecutive columns, each of which lies within q, k or v of one head -- RoPE on q and k in fp32 (transformer.rs:823-856), q
 // as hi + lo f16 halves for the attention kernel, k and v rounded into the cache (tensor.rs:373-376), and v once more
-// transposed, 8 positions per piece.
+// transposed, 8 positions per piece.  rows_end: the end of the rows that all tiles of the launch cover together.
 template <int kRows, int kTW, int kTS>
-__device__ __forceinline__ void rope_qkv_from_tile(const half_t *tile, int lane, int wr0, int wc0, int M, int N, const PrefillRopeParams &R) {
+__device__ __forceinline__ void rope_qkv_from_tile(const half_t *tile, int lane, int wr0, int wc0, int M, int N, int rows_end, const PrefillRopeParams &R) {
     constexpr int kChunks = kTW / 8;
     const int d = R.dim, hd = R.head_dim, half_hd = hd / 2;
     half_t *qhi = reinterpret_cast<half_t *>(R.q_hi), *qlo = reinterpret_cast<half_t *>(R.q_lo);
@@ -71,6 +71,16 @@ __device__ __forceinline__ void rope_qkv_from_tile(const half_t *tile, int lane,
                     o[e] = tile[src * kTS + cc];
                 }
                 *reinterpret_cast<half8_t *>(vt + (size_t)(c - 2 * d) * R.t_pad + pos0) = o;
+            }
+        }
+        // The two-product form of attention multiplies V^T up to t_pad with probabilities that are 0 there: what an earlier prompt
+        // left behind the last row tile must not be infinite or NaN (tiles of 32 and 64 rows end before t_pad, a multiple of 128)
+        if (wr0 + kRows == rows_end) {
+            const int pieces = (R.t_pad - rows_end) / 8; // negative: nothing to do
+            for (int idx = lane; idx < kTW * pieces; idx += 64) {
+                const int cc = idx / pieces, c = wc0 + cc;
+                if (c >= 2 * d && c < N)
+                    *reinterpret_cast<half8_t *>(vt + (size_t)(c - 2 * d) * R.t_pad + rows_end + (idx - cc * pieces) * 8) = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
             }
         }
     }

@@ -116,7 +116,7 @@ __global__ __launch_bounds__(64 * kSkWaves, 4) void gemm_f16_skinny_kernel(GemmP
         // the tile of 64 rows covers a whole key tile of the attention kernel: rows past m are zeros, finite padding of V^T
         for (int i = tid + 16 * kTS; i < 64 * kTS; i += 64 * kSkWaves) tile[i] = (half_t)0.0f;
         __syncthreads();
-        if (wave == 0) rope_qkv_from_tile<64, kSkCols, kTS>(tile, lane, 0, n0, p.m, p.n, p.rope);
+        if (wave == 0) rope_qkv_from_tile<64, kSkCols, kTS>(tile, lane, 0, n0, p.m, p.n, 64, p.rope);
     }
 }
 

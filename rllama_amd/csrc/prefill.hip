@@ -188,6 +188,14 @@ __global__ __launch_bounds__(256) void rope_kv_prefill_tiled_kernel(PrefillRopeP
         const int jrow = c / (kRopeTileRows / 8), ch = c - jrow * (kRopeTileRows / 8);
         *reinterpret_cast<h8 *>(vt + (size_t)jrow * p.t_pad + ch * 8) = *reinterpret_cast<const h8 *>(&vt_tile[jrow * kPad + ch * 8]);
     }
+    // zeros from the last tile to t_pad as well: the two-product form of attention multiplies them with probabilities of 0
+    if (blockIdx.x == gridDim.x - 1) {
+        const int pieces = (p.t_pad - r0 - kRopeTileRows) / 8;
+        for (int c = threadIdx.x; c < hd * pieces; c += blockDim.x) {
+            const int jrow = c / pieces, ch = c - jrow * pieces;
+            *reinterpret_cast<h8 *>(vt + (size_t)jrow * p.t_pad + kRopeTileRows + ch * 8) = h8{0, 0, 0, 0, 0, 0, 0, 0};
+        }
+    }
 }
 
 hipError_t launch_rope_kv_prefill(const PrefillRopeParams &p, hipStream_t s) {
