@@ -1,5 +1,7 @@
 """fp32 products on the bf16 matrix cores (three parts per value): against float64, against the fp32 matrix instruction, and the
 values the parts cannot hold."""
+import time
+
 import numpy as np
 import pytest
 
@@ -52,6 +54,29 @@ def test_split3_product_with_infinities_nan_and_the_largest_values(ctx):
     with np.errstate(all="ignore"):
         bound = (np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64).T)[ok] * ((k + 20) * 2.0 ** -23)
     assert np.all(np.abs(got[ok].astype(np.float64) - want[ok]) <= bound)
+
+
+def test_split3_product_of_nan_is_not_slow(ctx):
+    """Elements that are not finite are computed again: that is at most the product on the fp32 instruction (1.5 times this one) with
+    loads that are not staged, about 3 times the product in all; a plain loop per element takes 100 times."""
+    rng = np.random.default_rng(7)
+    m, n, k = 200, 11008, 4096
+    b = Tensor.from_numpy(ctx, (rng.standard_normal((n, k), dtype=f32) * f32(0.02)))
+
+    def seconds(a):
+        A, times = Tensor.from_numpy(ctx, a), []
+        for _ in range(4):
+            ctx.sync()
+            t = time.perf_counter()
+            A.matrix_mul_transposed(b)
+            ctx.sync()
+            times.append(time.perf_counter() - t)
+        return min(times)
+
+    a = rng.standard_normal((m, k), dtype=f32)
+    plain = seconds(a)
+    a[:, 5] = np.nan
+    assert seconds(a) < 20 * plain
 
 
 @pytest.mark.parametrize("m,n,k", [(1500, 96, 32768), (1537, 96, 40960)])  # the second: rows left after a pass pad to more than the capacity
