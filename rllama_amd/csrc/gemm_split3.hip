@@ -9,15 +9,20 @@
 // addition to the accumulator per 16 values of k and product instead of one per 2.  Six bf16 products cost 6/16 of the fp32
 // instruction's cycles.
 //
-// Values that the decomposition cannot hold (infinities, and finite values that round to a bf16 infinity: x - hi is then not a
-// remainder) make every product they enter NaN or infinite.  An element of C that comes out non-finite is therefore computed
-// again, with the fp32 matrix instruction on the operands themselves, so infinities and NaN are those of the plain sum.
+// Both operands are multiplied by 2^16 first and the sums by 2^-32 at the end, all exact: the last bit of the smallest fp32 number,
+// 2^-149, becomes 2^-133, the last bit of a bf16 number, so the parts hold every value however small.  (Without it values below 2^-109
+// lose bits: 2-norm error 2.2e-3 at 2^-126.  Two more vector instructions per pair: 11008 x 4096 weights, 8 / 64 / 200 / 1024 rows 51 / 75
+// / 178 / 555 -> 53 / 80 / 174 / 560 us per call, 7B prompt of 200 rows unchanged.)
+//
+// Values that the decomposition cannot hold (infinities, and finite values from 2^112 on, whose bf16 part is infinite: x - hi is then not
+// a remainder), and sums from 2^96 on, make every product they enter NaN or infinite.  An element of C that comes out non-finite is
+// therefore computed again, with the fp32 matrix instruction on the operands themselves, so infinities and NaN are those of the plain sum.
 // (A wavefront repeats every 32 x 32 tile that holds such an element.  Call of 200 x 11008 x 4096, 225 us without one: one NaN in A
 // 290 us, one infinity in B 450, NaN in every row 640; the fp32 instruction throughout 340.)
 //
 // A (the activations, few rows) is decomposed once by a kernel of its own into three bf16 planes laid out as the LDS image of a
 // K-tile, so that staging it is a linear copy.  B (the weights, read once) is staged as fp32 and decomposed by the wavefront
-// that feeds it to the matrix cores: 11 vector instructions per pair of values against 12 MFMAs per fragment and row tile.
+// that feeds it to the matrix cores: 13 vector instructions per pair of values against 12 MFMAs per fragment and row tile.
 //
 // Blocking.  A workgroup owns 32 kT rows x 128 columns and has eight wavefronts: 2 row groups x 2 column groups x 2 K-groups
 // (K-group g takes the g-th 16 of the 32 values of k in a K-tile).  A wavefront's tile is up to 128 x 64, which needs 16 KB of
@@ -30,8 +35,7 @@
 // compute units that have a tile.  Against the fp32 instruction, decomposition of A and sum of the pieces included, us:
 // 11008 x 4096 weights, 16 / 64 / 128 / 200 / 300 / 1024 rows: 84 / 142 / 157 / 271 / 443 / 746 -> 53 / 83 / 110 / 154 / 211 / 515;
 // 4096 x 11008: 64 / 107 / 123 / 206 / 395 / 707 -> 51 / 77 / 99 / 140 / 186 / 472.  7B shape, 200 prompt rows: 38.0 -> 21.6 ms.
-// Error against float64 (2-norm, 200 x 12288 x 4096): 5.0e-7 where the fp32 instruction has 1.15e-6 (fewer additions).  Values
-// below 2^-109 lose bits where their parts become bf16 subnormals: an absolute error of at most 2^-134 each.
+// Error against float64 (2-norm, 200 x 12288 x 4096): 5.0e-7 where the fp32 instruction has 1.15e-6 (fewer additions).
 // Products whose tiles do not fill the compute units are cut along K (partial sums in the workspace, added in order of the
 // pieces by gemm_split_finish_kernel).
 #include "kernels.h"
@@ -47,6 +51,8 @@ typedef __attribute__((ext_vector_type(8))) float float8_t;
 typedef __attribute__((ext_vector_type(8))) __bf16 bf8_t;
 
 constexpr int kS3Waves = 8;
+constexpr float kS3Scale = 65536.0f; // of every operand, exact: keeps the parts of the smallest values
+constexpr float kS3Unscale = 1.0f / (kS3Scale * kS3Scale);
 constexpr int kS3BStage = kS3Cols * kS3K * 4;
 constexpr int s3_a_stage(int t) { return 3 * t * 32 * kS3K * 2; }
 constexpr int s3_a_stages(int t) { return t >= 6 ? 2 : t >= 4 ? 3 : 4; }
@@ -66,7 +72,8 @@ struct Split3Params {
     size_t stride_c;             // elements between the pieces' partial sums
 };
 
-__device__ __forceinline__ void split3(const float8_t x, bf8_t &hi, bf8_t &mid, bf8_t &lo) {
+__device__ __forceinline__ void split3(const float8_t x_in, bf8_t &hi, bf8_t &mid, bf8_t &lo) {
+    const float8_t x = x_in * kS3Scale;
     hi = __builtin_convertvector(x, bf8_t);
     const float8_t r = x - __builtin_convertvector(hi, float8_t); // exact
     mid = __builtin_convertvector(r, bf8_t);
@@ -237,7 +244,7 @@ __global__ __launch_bounds__(64 * kS3Waves) void gemm_split3_kernel(Split3Params
                     for (int q = 0; q < 6; q++)
 #pragma unroll
                         for (int j = 0; j < 2; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[cur][kPa[q]], bs[kBCur][j][kPb[q]], acc[i][j], 0, 0, 0);
-                    if (i + 1 < kA) { // LDS reads first, then B's decomposition (about 44 vector instructions) between the MFMAs
+                    if (i + 1 < kA) { // LDS reads first, then B's decomposition (about 52 vector instructions) between the MFMAs
                         if (i < 2) __builtin_amdgcn_sched_group_barrier(0x100, 5, 0);
                         else __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
 #pragma unroll
@@ -279,7 +286,7 @@ __global__ __launch_bounds__(64 * kS3Waves) void gemm_split3_kernel(Split3Params
                 bool bad = false;
 #pragma unroll
                 for (int v = 0; v < 16; v++) {
-                    o[v] = (kg ? acc[i][1][v] : acc[i][0][v]) + theirs[(i * 16 + v) * 64];
+                    o[v] = ((kg ? acc[i][1][v] : acc[i][0][v]) + theirs[(i * 16 + v) * 64]) * kS3Unscale;
                     bad |= !__builtin_isfinite(o[v]);
                     const int r = r0 + (v >> 2) * 8 + (v & 3);
                     prev[v] = p.accumulate && r < p.m && c < p.n ? out[(size_t)r * p.ldc + c] : 0.0f;

@@ -41,7 +41,7 @@ def test_split3_product_with_infinities_nan_and_the_largest_values(ctx):
     m, n, k = 40, 3072, 256
     a = rng.standard_normal((m, k)).astype(f32)
     b = rng.standard_normal((n, k)).astype(f32)
-    a[3, 5], a[7, 9], a[11, 1], a[21, 3] = np.inf, -np.inf, np.nan, np.finfo(f32).max   # the last rounds to a bf16 infinity
+    a[3, 5], a[7, 9], a[11, 1], a[21, 3] = np.inf, -np.inf, np.nan, np.finfo(f32).max   # the parts cannot hold the last
     b[50, 200], b[51, 5], b[60], b[70, 3] = np.inf, 0.0, 0.0, 1e-30
     b[:, 3] *= f32(0.125)                                                                 # FLT_MAX times this stays finite ...
     b[2000:, 3] *= f32(1000.0)                                                            # ... or overflows
@@ -54,6 +54,25 @@ def test_split3_product_with_infinities_nan_and_the_largest_values(ctx):
     with np.errstate(all="ignore"):
         bound = (np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64).T)[ok] * ((k + 20) * 2.0 ** -23)
     assert np.all(np.abs(got[ok].astype(np.float64) - want[ok]) <= bound)
+
+
+# operands down to the smallest fp32 numbers (beside large ones, so that the product is not tiny), and products that are subnormal
+@pytest.mark.parametrize("ea,eb", [(-109, 60), (-120, 60), (60, -126), (-140, 60), (60, -145), (-70, -70), (-20, -115)])
+def test_split3_product_of_tiny_values(ctx, ea, eb):
+    rng = np.random.default_rng(8)
+    m, n, k = 33, 3072, 288
+    a = (rng.standard_normal((m, k)) * 2.0 ** ea).astype(f32)
+    b = (rng.standard_normal((n, k)) * 2.0 ** eb).astype(f32)
+    exact = a.astype(np.float64) @ b.astype(np.float64).T
+    got = _product(ctx, a, b)
+    # the bound of the ordinary values, and half a unit of the smallest fp32 number where the result is one
+    bound = (np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64).T) * ((6 * k / 16 + 1 + 18) * 2.0 ** -23) + 2.0 ** -150
+    assert np.all(np.abs(got - exact) <= bound)
+    if ea + eb > -100 and min(ea, eb) >= -126:  # (operands of few bits: the additions of both ways are nearly exact, neither is ahead)
+        with options(ctx, GEMM_SPLIT3="0"):
+            plain = _product(ctx, a, b)
+        err, err_plain = (np.linalg.norm((x - exact) / np.abs(exact).max()) for x in (got, plain))
+        assert err <= err_plain, (err, err_plain)
 
 
 def test_split3_product_of_nan_is_not_slow(ctx):
