@@ -7,6 +7,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
+#include <initializer_list>
 #include <map>
 #include <mutex>
 
@@ -40,7 +42,8 @@ constexpr int kOpMaxHeads = 1024;
 
 // Device buffers of freed op-level tensors, kept for the next tensor of the same size: an operation's result is a new tensor, and
 // hipMalloc + hipFree (which waits for the device) cost more than the operation.  Everything that touches a tensor's buffer is
-// ordered on the context's one stream, so a buffer may be handed out while work of its former owner is still queued.  Bounded in the
+// ordered on the context's one stream (tensors that another context's operation used are not kept: rlh_tensor::lent), so a buffer may be
+// handed out while work of its former owner is still queued.  Bounded in the
 // size of a buffer and in total, guarded by the context's lock, given back when memory runs out and by rlh_shutdown.
 struct TensorPool {
     static constexpr size_t kMaxBuffer = (size_t)8 << 20, kMaxTotal = (size_t)64 << 20;
@@ -105,6 +108,9 @@ struct rlh_tensor {
     rlh_ctx *ctx = nullptr;
     void *p = nullptr;
     int rows = 0, cols = 0, dtype = RLH_F16;
+    // an operation of another context has read or written the buffer: work on that context's stream may still be queued when the tensor
+    // is freed, so the buffer is not handed out again but freed, which waits for the device
+    mutable std::atomic<bool> lent{false};
     size_t esize() const { return dtype == RLH_F16 ? 2 : 4; }
     size_t count() const { return (size_t)rows * cols; }
 };
@@ -118,6 +124,12 @@ struct CtxLock {
     std::lock_guard<std::recursive_mutex> g;
     explicit CtxLock(rlh_ctx *c) : g(c->mu) { (void)hipSetDevice(c->device); }
 };
+
+// Notes that an operation of `user` is about to use the tensors.
+inline void lend(const rlh_ctx *user, std::initializer_list<const rlh_tensor *> tensors) {
+    for (const rlh_tensor *t : tensors)
+        if (t->ctx != user) t->lent.store(true, std::memory_order_relaxed);
+}
 
 namespace rlh {
 void ops_release(rlh_ctx *ctx); // frees the op-level work memory (rlh_shutdown)

@@ -84,7 +84,7 @@ extern "C" int rlh_tensor_download(rlh_tensor *t, void *host, int cols_capacity,
 extern "C" void rlh_tensor_free(rlh_tensor *t) {
     if (!t) return;
     CtxLock lock(t->ctx);
-    if (t->p && !t->ctx->pool.give(t->p, t->count() * t->esize())) {
+    if (t->p && (t->lent.load(std::memory_order_relaxed) || !t->ctx->pool.give(t->p, t->count() * t->esize()))) {
         (void)hipStreamSynchronize(t->ctx->stream);
         (void)hipFree(t->p);
     }
@@ -142,6 +142,7 @@ static int same_shape(const rlh_tensor *a, const rlh_tensor *b) { return a->rows
 extern "C" int rlh_copy_inplace(rlh_tensor *dst, const rlh_tensor *src) {
     if (!dst || !src || !same_shape(dst, src)) return fail(RLH_ERR_INVALID, "rlh_copy_inplace: shape/dtype mismatch");
     CtxLock lock(dst->ctx);
+    lend(dst->ctx, {src});
     // a plain copy kernel (the reference's copy_inplace is a kernel too); also the calibration point for HBM counters
     HIP_TRY(launch_convert(dst->p, dst->dtype == RLH_F16, src->p, src->dtype == RLH_F16, dst->count(), dst->ctx->stream));
     return RLH_OK;
@@ -152,6 +153,7 @@ extern "C" int rlh_transpose_from(rlh_tensor *dst, const rlh_tensor *src) {
         return fail(RLH_ERR_INVALID, "rlh_transpose_from: shape/dtype mismatch");
     }
     CtxLock lock(dst->ctx);
+    lend(dst->ctx, {src});
     HIP_TRY(launch_transpose(dst->p, src->p, src->rows, src->cols, src->dtype == RLH_F16, dst->ctx->stream));
     return RLH_OK;
 }
@@ -159,6 +161,7 @@ extern "C" int rlh_transpose_from(rlh_tensor *dst, const rlh_tensor *src) {
 extern "C" int rlh_hadamard_product_inplace(rlh_tensor *dst, const rlh_tensor *src) {
     if (!dst || !src || !same_shape(dst, src)) return fail(RLH_ERR_INVALID, "rlh_hadamard_product_inplace: shape/dtype mismatch");
     CtxLock lock(dst->ctx);
+    lend(dst->ctx, {src});
     HIP_TRY(launch_hadamard(dst->p, src->p, dst->count(), dst->dtype == RLH_F16, dst->ctx->stream));
     return RLH_OK;
 }
@@ -177,6 +180,7 @@ extern "C" int rlh_gemv(rlh_tensor *y, const rlh_tensor *w, const rlh_tensor *x,
     const int vec = w->dtype == RLH_F16 ? 8 : 4;
     if (w->cols % vec != 0) return fail(RLH_ERR_UNSUPPORTED, "rlh_gemv: k must be a multiple of %d", vec);
     CtxLock lock(y->ctx);
+    lend(y->ctx, {w, x});
     GemvParams p{};
     p.w = w->p;
     p.w_is_f16 = w->dtype == RLH_F16;
@@ -201,6 +205,7 @@ extern "C" int rlh_matrix_mul_inplace_transposed(rlh_tensor *dst, const rlh_tens
     const int f16 = src->dtype == RLH_F16;
     if (src->cols % (f16 ? 8 : 4) != 0) return fail(RLH_ERR_UNSUPPORTED, "rlh_matrix_mul_inplace_transposed: k must be a multiple of %d", f16 ? 8 : 4);
     CtxLock lock(dst->ctx);
+    lend(dst->ctx, {src, other});
     hipStream_t st = dst->ctx->stream;
     const int n = src->rows, k = src->cols, mrows = other->rows;
     if (n > 1 && (f16 || k % 32 == 0)) {
@@ -255,6 +260,7 @@ extern "C" int rlh_rmsnorm(rlh_tensor *y, const rlh_tensor *x, const rlh_tensor 
     if (x->dtype != RLH_F32 || y->dtype != RLH_F32 || w->dtype != RLH_F32) return fail(RLH_ERR_INVALID, "rlh_rmsnorm: f32 tensors only");
     if (!same_shape(x, y) || w->rows != 1 || w->cols != x->cols) return fail(RLH_ERR_INVALID, "rlh_rmsnorm: shape mismatch");
     CtxLock lock(y->ctx);
+    lend(y->ctx, {x, w});
     HIP_TRY(launch_rmsnorm_rows((float *)y->p, (const float *)x->p, (const float *)w->p, x->rows, x->cols, (float)eps, round_y, y->ctx->stream));
     return RLH_OK;
 }
@@ -286,6 +292,7 @@ extern "C" int rlh_add(rlh_tensor *dst, const rlh_tensor *a, const rlh_tensor *b
     if (!dst || !a || !b || !same_shape(dst, a) || !same_shape(dst, b)) return fail(RLH_ERR_INVALID, "rlh_add: shape/dtype mismatch");
     if (dst->dtype != RLH_F32) return fail(RLH_ERR_UNSUPPORTED, "rlh_add: f32 tensors only (the residual stream is f32, transformer.rs:442)");
     CtxLock lock(dst->ctx);
+    lend(dst->ctx, {a, b});
     HIP_TRY(launch_add_f32((float *)dst->p, (const float *)a->p, (const float *)b->p, dst->count(), dst->ctx->stream));
     return RLH_OK;
 }
@@ -293,6 +300,7 @@ extern "C" int rlh_add(rlh_tensor *dst, const rlh_tensor *a, const rlh_tensor *b
 extern "C" int rlh_silu_mul(rlh_tensor *dst, const rlh_tensor *gate, const rlh_tensor *up) {
     if (!dst || !gate || !up || !same_shape(dst, gate) || !same_shape(dst, up)) return fail(RLH_ERR_INVALID, "rlh_silu_mul: shape/dtype mismatch");
     CtxLock lock(dst->ctx);
+    lend(dst->ctx, {gate, up});
     if (dst->dtype == RLH_F16) HIP_TRY(launch_silu_mul_f16(gate->p, up->p, dst->p, dst->count(), dst->ctx->stream));
     else HIP_TRY(launch_silu_mul_f32((const float *)gate->p, (const float *)up->p, (float *)dst->p, dst->count(), dst->ctx->stream));
     return RLH_OK;
@@ -307,6 +315,7 @@ extern "C" int rlh_ffn_gate(rlh_tensor *dst, const rlh_tensor *x, const rlh_tens
     }
     if (x->cols % 8 != 0) return fail(RLH_ERR_UNSUPPORTED, "rlh_ffn_gate: k must be a multiple of 8");
     CtxLock lock(dst->ctx);
+    lend(dst->ctx, {x, w1, w3});
     hipStream_t st = dst->ctx->stream;
     GemmParams g{};
     g.tune = dst->ctx->tun.gemm;
@@ -366,6 +375,7 @@ extern "C" int rlh_rope_kvwrite(rlh_tensor *q, const rlh_tensor *k, const rlh_te
     }
     if (pos < 0 || pos >= max_seq_len) return fail(RLH_ERR_STATE, "rlh_rope_kvwrite: position %d outside the cache (max_seq_len %d)", pos, max_seq_len);
     CtxLock lock(q->ctx);
+    lend(q->ctx, {k, v, cache_k, cache_v});
     hipStream_t st = q->ctx->stream;
     const std::vector<float2> tab = rope_table(hd, pos, 1);
     float2 *dev = nullptr;
@@ -495,6 +505,7 @@ extern "C" int rlh_attn_decode(rlh_tensor *out, const rlh_tensor *q, const rlh_t
     if (rc != RLH_OK) return rc;
     rlh_ctx *ctx = out->ctx;
     CtxLock lock(ctx);
+    lend(ctx, {q, cache_k, cache_v});
     rc = ensure_op_scratch(ctx, attn_decode_workspace_floats(n_heads, hd, n_splits));
     if (rc != RLH_OK) return rc;
     HIP_TRY(enqueue_attn_decode(ctx, out, q, cache_k, cache_v, n_heads, hd, max_seq_len, T, n_splits, round_out, ctx->ops.state, ctx->ops.attn_ws,
@@ -514,6 +525,7 @@ extern "C" int rlh_attn_prefill(rlh_tensor *out, const rlh_tensor *qkv, rlh_tens
     if (n > max_seq_len) return fail(RLH_ERR_STATE, "rlh_attn_prefill: %d rows exceed max_seq_len %d", n, max_seq_len);
     rlh_ctx *ctx = out->ctx;
     CtxLock lock(ctx);
+    lend(ctx, {qkv, cache_k, cache_v});
     hipStream_t st = ctx->stream;
     const int tp = (n + 127) & ~127;
     const std::vector<float2> tab = rope_table(hd, 0, n);
@@ -624,6 +636,7 @@ extern "C" int rlh_attn_decode_noalloc(rlh_tensor *out, const rlh_tensor *q, con
     }
     rlh_ctx *ctx = out->ctx;
     CtxLock lock(ctx);
+    lend(ctx, {q, cache_k, cache_v});
     unsigned char *base = static_cast<unsigned char *>(ctx->noalloc_scratch); // this device's address of `scratch`, from rlh_init
     if (!base) return fail(RLH_ERR_STATE, "rlh_attn_decode_noalloc: the context holds no address of the static work memory");
     HIP_TRY(enqueue_attn_decode(ctx, out, q, cache_k, cache_v, n_heads, hd, max_seq_len, T, n_splits, round_out,

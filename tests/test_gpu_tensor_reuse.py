@@ -2,7 +2,7 @@
 import numpy as np
 import pytest
 
-from rllama_amd import Tensor, TensorDType
+from rllama_amd import Context, Tensor, TensorDType
 
 pytestmark = pytest.mark.gpu
 
@@ -28,3 +28,24 @@ def test_upload_and_download_of_reused_buffers(ctx, rows, cols):
         t = Tensor.from_numpy(ctx, x)
         assert np.array_equal(t.to_numpy(), x)
         t.free()
+
+
+def test_buffers_that_another_context_uses_are_not_handed_out(ctx):
+    """A tensor freed while an operation of another context (another stream) reads it: a new tensor of its size must not get the buffer."""
+    rng = np.random.default_rng(4)
+    other = Context(0)
+    try:
+        x = Tensor.from_numpy(other, rng.standard_normal((512, 1024)).astype(np.float32))
+        w = rng.standard_normal((2048, 1024)).astype(np.float32)
+        junk = np.full_like(w, 7.0)
+        want = x.matrix_mul_transposed(Tensor.from_numpy(other, w)).to_numpy()
+        for _ in range(20):
+            W = Tensor.from_numpy(ctx, w)
+            for _ in range(4):  # work of the other context that is still queued when the tensor is freed
+                got = x.matrix_mul_transposed(W)
+            W.free()
+            J = Tensor.from_numpy(ctx, junk)
+            assert np.array_equal(got.to_numpy(), want)
+            assert np.array_equal(J.to_numpy(), junk)
+    finally:
+        other.close()
