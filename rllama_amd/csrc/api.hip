@@ -253,6 +253,7 @@ extern "C" void rlh_shutdown(rlh_ctx *ctx) {
     if (ctx->stream) {
         (void)hipStreamSynchronize(ctx->stream);
         (void)hipStreamDestroy(ctx->stream);
+        ctx->stream = nullptr;
     }
     ops_release(ctx);
     delete ctx;

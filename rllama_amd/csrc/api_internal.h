@@ -4,12 +4,12 @@
 
 #include "../../include/rllama_hip.h"
 #include "kernels.h"
+#include "tensor_pool.h"
 
 #include <hip/hip_runtime.h>
 
 #include <atomic>
 #include <initializer_list>
-#include <map>
 #include <mutex>
 
 namespace rlh {
@@ -40,36 +40,6 @@ struct OpScratch {
 constexpr size_t kOpGemmWsBytes = (size_t)192 << 20;
 constexpr int kOpMaxHeads = 1024;
 
-// Device buffers of freed op-level tensors, kept for the next tensor of the same size: an operation's result is a new tensor, and
-// hipMalloc + hipFree (which waits for the device) cost more than the operation.  Everything that touches a tensor's buffer is
-// ordered on the context's one stream (tensors that another context's operation used are not kept: rlh_tensor::lent), so a buffer may be
-// handed out while work of its former owner is still queued.  Bounded in the
-// size of a buffer and in total, guarded by the context's lock, given back when memory runs out and by rlh_shutdown.
-struct TensorPool {
-    static constexpr size_t kMaxBuffer = (size_t)8 << 20, kMaxTotal = (size_t)64 << 20;
-    std::multimap<size_t, void *> free_buffers; // by size in bytes
-    size_t total = 0;
-    void *take(size_t bytes) {
-        auto it = free_buffers.find(bytes);
-        if (it == free_buffers.end()) return nullptr;
-        void *p = it->second;
-        free_buffers.erase(it);
-        total -= bytes;
-        return p;
-    }
-    bool give(void *p, size_t bytes) {
-        if (bytes > kMaxBuffer || total + bytes > kMaxTotal) return false;
-        free_buffers.emplace(bytes, p);
-        total += bytes;
-        return true;
-    }
-    void release() { // the caller has waited for the stream
-        for (auto &kv : free_buffers) (void)hipFree(kv.second);
-        free_buffers.clear();
-        total = 0;
-    }
-};
-
 // The library's switches.  Read from the environment (RLLAMA_HIP_<NAME>) once, when the context is made, and changed
 // afterwards only through rlh_set_option under the context lock: no launch path reads the environment.
 struct Tunables {
@@ -98,7 +68,10 @@ struct rlh_ctx {
     hipDeviceProp_t prop;
     std::recursive_mutex mu;
     OpScratch ops;
-    TensorPool pool;
+    // Buffers of freed tensors, guarded by mu.  Everything that touches a tensor's buffer is ordered on the context's one stream (tensors
+    // that another context's operation used are not kept: rlh_tensor::lent), so a buffer may be handed out while work of its former owner
+    // is still queued.  Given back by rlh_shutdown.
+    rlh::TensorPool pool;
     Tunables tun;
     unsigned tun_version = 0;        // bumped by rlh_set_option: captured decode steps of an older version are dropped
     void *noalloc_scratch = nullptr; // this device's address of the library's static work memory (api_ops.hip)
@@ -108,6 +81,7 @@ struct rlh_tensor {
     rlh_ctx *ctx = nullptr;
     void *p = nullptr;
     int rows = 0, cols = 0, dtype = RLH_F16;
+    size_t capacity = 0; // bytes allocated at p
     // an operation of another context has read or written the buffer: work on that context's stream may still be queued when the tensor
     // is freed, so the buffer is not handed out again but freed, which waits for the device
     mutable std::atomic<bool> lent{false};
@@ -124,6 +98,10 @@ struct CtxLock {
     std::lock_guard<std::recursive_mutex> g;
     explicit CtxLock(rlh_ctx *c) : g(c->mu) { (void)hipSetDevice(c->device); }
 };
+
+namespace rlh {
+void pool_release(rlh_ctx *ctx); // waits for the stream and frees the kept buffers
+} // namespace rlh
 
 // Notes that an operation of `user` is about to use the tensors.
 inline void lend(const rlh_ctx *user, std::initializer_list<const rlh_tensor *> tensors) {

@@ -23,14 +23,14 @@ extern "C" int rlh_tensor_alloc(rlh_ctx *ctx, int rows, int cols, int dtype, rlh
     t->cols = cols;
     t->dtype = dtype;
     const size_t bytes = t->count() * t->esize();
-    t->p = ctx->pool.take(bytes);
+    t->p = ctx->pool.take(bytes, &t->capacity);
     hipError_t e = hipSuccess;
     if (!t->p) {
+        t->capacity = bytes;
         e = hipMalloc(&t->p, bytes);
-        if (e == hipErrorOutOfMemory && ctx->pool.total > 0) {
+        if (e == hipErrorOutOfMemory && ctx->pool.count() > 0) {
             (void)hipGetLastError();
-            (void)hipStreamSynchronize(ctx->stream);
-            ctx->pool.release();
+            pool_release(ctx);
             e = hipMalloc(&t->p, bytes);
         }
     }
@@ -84,7 +84,14 @@ extern "C" int rlh_tensor_download(rlh_tensor *t, void *host, int cols_capacity,
 extern "C" void rlh_tensor_free(rlh_tensor *t) {
     if (!t) return;
     CtxLock lock(t->ctx);
-    if (t->p && (t->lent.load(std::memory_order_relaxed) || !t->ctx->pool.give(t->p, t->count() * t->esize()))) {
+    TensorPool &pool = t->ctx->pool;
+    if (t->p && TensorPool::keeps(t->capacity) && !t->lent.load(std::memory_order_relaxed)) {
+        if (!pool.room(t->capacity)) {
+            (void)hipStreamSynchronize(t->ctx->stream);
+            while (!pool.room(t->capacity)) (void)hipFree(pool.drop());
+        }
+        pool.put(t->p, t->capacity);
+    } else if (t->p) {
         (void)hipStreamSynchronize(t->ctx->stream);
         (void)hipFree(t->p);
     }
@@ -441,8 +448,14 @@ static int ensure_op_scratch(rlh_ctx *ctx, size_t attn_ws_floats) {
 }
 
 namespace rlh {
+void pool_release(rlh_ctx *ctx) {
+    if (ctx->pool.count() == 0) return;
+    if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
+    while (void *p = ctx->pool.drop()) (void)hipFree(p);
+}
+
 void ops_release(rlh_ctx *ctx) {
-    ctx->pool.release();
+    pool_release(ctx);
     OpScratch &o = ctx->ops;
     void *all[] = {o.state, o.attn_ws, o.tickets, o.token, o.gemm_ws};
     for (void *b : all)

@@ -20,7 +20,7 @@ def test_freed_buffers_come_back_zeroed_and_in_order(ctx):
         assert np.array_equal(got.to_numpy(), first)
 
 
-@pytest.mark.parametrize("rows,cols", [(1, 1), (3, 7), (2048, 1024), (2049, 1024)])  # the last is over the size that is kept
+@pytest.mark.parametrize("rows,cols", [(1, 1), (3, 7), (2048, 1024), (2049, 1024), (8193, 1024)])  # the last is over the size that is kept
 def test_upload_and_download_of_reused_buffers(ctx, rows, cols):
     rng = np.random.default_rng(rows)
     for _ in range(4):
@@ -28,6 +28,22 @@ def test_upload_and_download_of_reused_buffers(ctx, rows, cols):
         t = Tensor.from_numpy(ctx, x)
         assert np.array_equal(t.to_numpy(), x)
         t.free()
+
+
+def test_tensors_of_changing_sizes(ctx):
+    """More sizes than the pool holds, in buffers of larger ones: new tensors are zero to their end, contents are their own."""
+    rng = np.random.default_rng(5)
+    kept = []
+    for i in range(400):
+        rows = int(rng.integers(1, 700))
+        z = Tensor.zeros(ctx, rows, 4100, TensorDType.Float32)
+        x = rng.standard_normal((rows, 11)).astype(np.float32)
+        kept.append((x, Tensor.from_numpy(ctx, x)))
+        if i % 10 == 0:
+            assert not z.to_numpy().any()
+            for want, t in kept:
+                assert np.array_equal(t.to_numpy(), want)
+            kept = kept[-3:]
 
 
 def test_buffers_that_another_context_uses_are_not_handed_out(ctx):

@@ -1,0 +1,94 @@
+"""The bookkeeping of kept device buffers (rllama_amd/csrc/tensor_pool.h), on the CPU: its bounds, which buffer a tensor gets, which one goes
+first, and that a host whose sizes change keeps finding buffers."""
+import os
+import subprocess
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "rllama_amd", "csrc")
+
+PROGRAM = r"""
+#include "tensor_pool.h"
+#include <cstdint>
+#include <cstdio>
+#include <cstdlib>
+#include <map>
+using namespace rlh;
+#define CHECK(x) do { if (!(x)) { printf("line %d: %s\n", __LINE__, #x); return 1; } } while (0)
+
+static TensorPool pool;
+static std::map<void *, size_t> live; // buffers in existence, kept ones among them
+static long allocations = 0;
+
+static void *get(size_t bytes, size_t *cap) {
+    void *p = pool.take(bytes, cap);
+    if (!p) {
+        p = reinterpret_cast<void *>((uintptr_t)++allocations * 64);
+        live[p] = *cap = bytes;
+    }
+    return p;
+}
+static void give(void *p, size_t cap) {
+    if (!TensorPool::keeps(cap)) { live.erase(p); return; }
+    while (!pool.room(cap)) live.erase(pool.drop());
+    pool.put(p, cap);
+}
+
+int main() {
+    const size_t MB = (size_t)1 << 20;
+    size_t cap = 0;
+    // the smallest that holds it, at most twice as large, the latest of equals; whole and once
+    pool.put((void *)64, 1000); pool.put((void *)128, 1100); pool.put((void *)192, 1000);
+    CHECK(pool.take(1101, &cap) == nullptr && pool.take(499, &cap) == nullptr);
+    CHECK(pool.take(900, &cap) == (void *)192 && cap == 1000);
+    CHECK(pool.take(1000, &cap) == (void *)64 && cap == 1000);
+    CHECK(pool.take(1000, &cap) == (void *)128 && cap == 1100);
+    CHECK(pool.take(1000, &cap) == nullptr && pool.total() == 0 && pool.count() == 0 && pool.drop() == nullptr);
+    // bounds: number, total, size; the longest waiting goes first
+    for (int i = 0; i < 200; i++) give(get(64 + 1000 * (size_t)i, &cap), 64 + 1000 * (size_t)i);
+    CHECK(pool.count() <= TensorPool::kMaxCount && pool.take(64, &cap) == nullptr && pool.take(199064, &cap) != nullptr);
+    while (pool.drop()) {}
+    for (int i = 0; i < 40; i++) {
+        give(get((20 + i % 12) * MB + 64 * i, &cap), cap);
+        CHECK(pool.total() <= TensorPool::kMaxTotal);
+    }
+    CHECK(!TensorPool::keeps(TensorPool::kMaxBuffer + 1) && TensorPool::keeps(27 * MB) && pool.count() >= 3);
+    while (pool.drop()) {}
+    // feed-forward blocks through the ops, one after the other at changing row counts: the results of a block are alive together.
+    // Hardly any needs a new buffer once the pool has seen a few.
+    srand(1);
+    for (size_t es : {2, 4})
+        for (int pass = 0; pass < 2; pass++) {
+            const long before = allocations;
+            long wanted = 0;
+            for (int i = 0; i < 2000; i++) {
+                const size_t n = 1 + rand() % 512, d = 5120, f = 13824;
+                const size_t sizes[4] = {n * f * es, n * f * es, n * f * es, n * d * es};
+                void *p[4];
+                size_t c[4];
+                for (int j = 0; j < 4; j++, wanted++) p[j] = get(sizes[j], &c[j]);
+                for (int j = 0; j < 4; j++) {
+                    CHECK(c[j] >= sizes[j] && live.count(p[j]) == 1 && live[p[j]] == c[j]);
+                    for (int k = 0; k < j; k++) CHECK(p[j] != p[k]);
+                }
+                for (int j = 0; j < 4; j++) give(p[j], c[j]);
+                CHECK(pool.total() <= TensorPool::kMaxTotal && pool.count() <= TensorPool::kMaxCount);
+            }
+            printf("element size %zu: %ld of %ld tensors allocated\n", es, allocations - before, wanted);
+            if (pass == 1) CHECK((allocations - before) * 10 < wanted);
+        }
+    // all sizes of one host that settles down again
+    for (int i = 0; i < 100; i++) give(get(77 * 11008 * 2, &cap), cap);
+    const long before = allocations;
+    for (int i = 0; i < 100; i++) give(get(77 * 11008 * 2, &cap), cap);
+    CHECK(allocations == before);
+    return 0;
+}
+"""
+
+
+def test_kept_buffers_stay_within_bounds_and_follow_their_user(tmp_path):
+    src, exe = tmp_path / "pool.cpp", tmp_path / "pool"
+    src.write_text(PROGRAM.replace("#include <cstdint>", "#include <cstdint>\n#include <initializer_list>"))
+    subprocess.check_call(["g++", "-O1", "-std=c++17", "-Wall", "-I", CSRC, str(src), "-o", str(exe)])
+    r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=300)
+    print(r.stdout)
+    assert r.returncode == 0, r.stdout
