@@ -282,11 +282,11 @@ static void free_weight(Weight &w) {
     w.p = nullptr;
 }
 
-static int alloc_weight(Weight &w, int rows, int cols, int f16) {
+static int alloc_weight(rlh_ctx *ctx, Weight &w, int rows, int cols, int f16) {
     w.rows = rows;
     w.cols = cols;
     w.f16 = f16;
-    HIP_TRY(hipMalloc(&w.p, w.bytes()));
+    HIP_TRY(device_alloc(ctx, &w.p, w.bytes()));
     return RLH_OK;
 }
 
@@ -333,7 +333,7 @@ extern "C" int rlh_model_create(rlh_ctx *ctx, const rlh_model_params *prm, rlh_m
     const int d = prm->dim, F = prm->ffn_hidden, V = prm->vocab_size;
     int rc = RLH_OK;
     auto A = [&](Weight &w, int r, int c, int f16) {
-        if (rc == RLH_OK) rc = alloc_weight(w, r, c, f16);
+        if (rc == RLH_OK) rc = alloc_weight(ctx, w, r, c, f16);
     };
     for (int l = 0; l < m->n_resident; l++) {
         Layer &L = m->layers[(size_t)l];
@@ -363,13 +363,13 @@ extern "C" int rlh_model_create(rlh_ctx *ctx, const rlh_model_params *prm, rlh_m
                 tab[(size_t)pos * (hd / 2) + j] = make_float2((float)std::cos(ang), (float)std::sin(ang));
             }
         }
-        hipError_t e = hipMalloc((void **)&m->freqs, tab.size() * sizeof(float2));
+        hipError_t e = device_alloc(ctx, (void **)&m->freqs, tab.size() * sizeof(float2));
         if (e == hipSuccess) e = hipMemcpy(m->freqs, tab.data(), tab.size() * sizeof(float2), hipMemcpyHostToDevice);
         if (e != hipSuccess) rc = fail(RLH_ERR_HIP, "rlh_model_create: RoPE table: %s", hipGetErrorString(e));
     }
     auto B = [&](void **p, size_t bytes) {
         if (rc != RLH_OK) return;
-        hipError_t e = hipMalloc(p, bytes);
+        hipError_t e = device_alloc(ctx, p, bytes);
         if (e == hipSuccess) e = hipMemset(*p, 0, bytes);
         if (e != hipSuccess) rc = fail(e == hipErrorOutOfMemory ? RLH_ERR_OOM : RLH_ERR_HIP, "rlh_model_create: %s", hipGetErrorString(e));
     };
@@ -472,7 +472,7 @@ extern "C" int rlh_model_set_tensor(rlh_model *m, int kind, int layer, const voi
         // stored in the source's dtype: lossless either way
         if (s.w->p && s.w->f16 != (src_dtype == RLH_F16)) free_weight(*s.w);
         if (!s.w->p) {
-            rc = alloc_weight(*s.w, rows, cols, src_dtype == RLH_F16);
+            rc = alloc_weight(m->ctx, *s.w, rows, cols, src_dtype == RLH_F16);
             if (rc != RLH_OK) return rc;
         }
     }
@@ -486,7 +486,7 @@ extern "C" int rlh_model_set_tensor(rlh_model *m, int kind, int layer, const voi
         // widen (f16 file -> f32 tensor, tensor.rs:2467) or narrow (Tensor::to_f16 under --f16, tensor.rs:2281-2314) on the device
         void *tmp = nullptr;
         const size_t sb = n * (src_dtype == RLH_F16 ? 2 : 4);
-        HIP_TRY(hipMalloc(&tmp, sb));
+        HIP_TRY(device_alloc(m->ctx, &tmp, sb));
         hipError_t e = hipMemcpyAsync(tmp, host, sb, hipMemcpyHostToDevice, st);
         if (e == hipSuccess) e = launch_convert(dst, dst_f16, tmp, src_dtype == RLH_F16, n, st);
         hipError_t e2 = hipStreamSynchronize(st);
@@ -518,7 +518,7 @@ extern "C" int rlh_model_get_tensor(rlh_model *m, int kind, int layer, void *hos
         return RLH_OK;
     }
     void *tmp = nullptr;
-    HIP_TRY(hipMalloc(&tmp, db));
+    HIP_TRY(device_alloc(m->ctx, &tmp, db));
     hipError_t e = launch_convert(tmp, want_f16, src, s.w->f16, n, st);
     if (e == hipSuccess) e = hipMemcpyAsync(host_out, tmp, db, hipMemcpyDeviceToHost, st);
     hipError_t e2 = hipStreamSynchronize(st);
@@ -536,7 +536,7 @@ extern "C" int rlh_model_fill_synthetic(rlh_model *m, uint64_t seed, double std)
     const bool whole = m->n_resident == m->prm.n_layers; // a split model leaves embedding, final norm and head to the host (transformer.rs:296-308)
     for (Weight *w : {&m->tok_emb, &m->output}) {
         if (whole && !w->p) {
-            int rc = alloc_weight(*w, w->rows, w->cols, 1);
+            int rc = alloc_weight(m->ctx, *w, w->rows, w->cols, 1);
             if (rc != RLH_OK) return rc;
         }
     }
@@ -626,8 +626,8 @@ extern "C" int rlh_caches_create(rlh_model *m, rlh_caches **out) {
     c->max_seq_len = m->prm.max_seq_len;
     c->f16 = m->prm.force_f16 ? 1 : 0; // transformer.rs:138-142
     c->bytes_each = (size_t)c->n_layers * c->n_heads * c->max_seq_len * c->head_dim * (c->f16 ? 2 : 4);
-    hipError_t e = hipMalloc(&c->k, c->bytes_each);
-    if (e == hipSuccess) e = hipMalloc(&c->v, c->bytes_each);
+    hipError_t e = device_alloc(c->ctx, &c->k, c->bytes_each);
+    if (e == hipSuccess) e = device_alloc(c->ctx, &c->v, c->bytes_each);
     if (e == hipSuccess) e = hipMemsetAsync(c->k, 0, c->bytes_each, c->ctx->stream); // Tensor::zeros
     if (e == hipSuccess) e = hipMemsetAsync(c->v, 0, c->bytes_each, c->ctx->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(c->ctx->stream);
@@ -649,8 +649,8 @@ extern "C" int rlh_caches_true_clone(const rlh_caches *src, rlh_caches **out) {
     rlh_caches *c = new rlh_caches(*src);
     c->k = c->v = nullptr;
     c->step_graphs.clear(); // captured steps hold the source's cache addresses: the clone captures its own
-    hipError_t e = hipMalloc(&c->k, c->bytes_each);
-    if (e == hipSuccess) e = hipMalloc(&c->v, c->bytes_each);
+    hipError_t e = device_alloc(c->ctx, &c->k, c->bytes_each);
+    if (e == hipSuccess) e = device_alloc(c->ctx, &c->v, c->bytes_each);
     if (e == hipSuccess) e = hipMemcpyAsync(c->k, src->k, c->bytes_each, hipMemcpyDeviceToDevice, ctx->stream);
     if (e == hipSuccess) e = hipMemcpyAsync(c->v, src->v, c->bytes_each, hipMemcpyDeviceToDevice, ctx->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
@@ -669,8 +669,14 @@ extern "C" int rlh_caches_shift_left(rlh_caches *c, int shifts) {
     if (shifts == 0) return RLH_OK;
     CtxLock lock(c->ctx);
     const size_t planes = (size_t)c->n_layers * c->n_heads;
-    HIP_TRY(launch_cache_shift_left(c->k, c->f16, planes, c->max_seq_len, c->head_dim, shifts, c->ctx->stream));
-    HIP_TRY(launch_cache_shift_left(c->v, c->f16, planes, c->max_seq_len, c->head_dim, shifts, c->ctx->stream));
+    void *tmp = nullptr;
+    HIP_TRY(device_alloc(c->ctx, &tmp, c->bytes_each));
+    hipError_t e = launch_cache_shift_left(c->k, tmp, c->f16, planes, c->max_seq_len, c->head_dim, shifts, c->ctx->stream);
+    if (e == hipSuccess) e = launch_cache_shift_left(c->v, tmp, c->f16, planes, c->max_seq_len, c->head_dim, shifts, c->ctx->stream);
+    hipError_t e2 = hipStreamSynchronize(c->ctx->stream);
+    (void)hipFree(tmp);
+    HIP_TRY(e);
+    HIP_TRY(e2);
     return RLH_OK;
 }
 
@@ -693,7 +699,7 @@ extern "C" int rlh_caches_read(const rlh_caches *c, int layer, int head, int whi
     const size_t off = ((size_t)layer * c->n_heads + head) * per_plane * (c->f16 ? 2 : 4);
     const char *plane = (const char *)(which ? c->v : c->k) + off;
     float *tmp = nullptr;
-    HIP_TRY(hipMalloc((void **)&tmp, per_plane * 4));
+    HIP_TRY(device_alloc(c->ctx, (void **)&tmp, per_plane * 4));
     hipError_t e = launch_cache_read(tmp, plane, c->f16, c->max_seq_len, c->head_dim, st);
     if (e == hipSuccess) e = hipMemcpyAsync(host_out, tmp, per_plane * 4, hipMemcpyDeviceToHost, st);
     hipError_t e2 = hipStreamSynchronize(st);
@@ -906,7 +912,7 @@ static int ensure_prefill_scratch(rlh_model *m, int n) {
     hipError_t e = hipSuccess;
     auto A = [&](void **p, size_t bytes) {
         if (e != hipSuccess) return;
-        e = hipMalloc(p, bytes);
+        e = device_alloc(m->ctx, p, bytes);
         if (e == hipSuccess) e = hipMemsetAsync(*p, 0, bytes, m->ctx->stream); // padding must hold finite values
     };
     A((void **)&S.x, N * d * 4);
@@ -922,7 +928,7 @@ static int ensure_prefill_scratch(rlh_model *m, int n) {
     if (es == 4) A((void **)&S.u, N * F * es); // f16 mode: w3's epilogue consumes its product on the spot
     A((void **)&S.mm, N * F * es);
     const size_t ws_bytes = es == 4 ? PrefillScratch::kGemmWsBytesF32 : PrefillScratch::kGemmWsBytes;
-    if (e == hipSuccess) e = hipMalloc(&S.gemm_ws, ws_bytes); // (written before it is read, always)
+    if (e == hipSuccess) e = device_alloc(m->ctx, &S.gemm_ws, ws_bytes); // (written before it is read, always)
     if (e == hipSuccess) e = hipStreamSynchronize(m->ctx->stream);
     if (e != hipSuccess) {
         S.release();
@@ -1612,11 +1618,11 @@ extern "C" int rlh_time_gemv(rlh_ctx *ctx, int rows, int k, int w_dtype, int rou
     hipEvent_t e0 = nullptr, e1 = nullptr;
     hipError_t e = hipSuccess;
     for (int i = 0; e == hipSuccess && i < n_buffers; i++) {
-        e = hipMalloc(&bufs[(size_t)i], wbytes);
+        e = device_alloc(ctx, &bufs[(size_t)i], wbytes);
         if (e == hipSuccess) e = launch_synth_fill(bufs[(size_t)i], f16, (uint64_t)rows * k, synth_key(99, (uint64_t)i), 0.02, st);
     }
-    if (e == hipSuccess) e = hipMalloc((void **)&x, sizeof(float) * (size_t)k);
-    if (e == hipSuccess) e = hipMalloc((void **)&y, sizeof(float) * (size_t)rows);
+    if (e == hipSuccess) e = device_alloc(ctx, (void **)&x, sizeof(float) * (size_t)k);
+    if (e == hipSuccess) e = device_alloc(ctx, (void **)&y, sizeof(float) * (size_t)rows);
     if (e == hipSuccess) e = launch_fill_f32(x, (uint64_t)k, 0.5f, st);
     if (e == hipSuccess) e = hipEventCreate(&e0);
     if (e == hipSuccess) e = hipEventCreate(&e1);
@@ -1667,12 +1673,12 @@ extern "C" int rlh_probe_gemv_phases(rlh_ctx *ctx, int rows, int k, int n_buffer
     const size_t max_waves = 2048 + 64;
     hipError_t e = hipSuccess;
     for (int i = 0; e == hipSuccess && i < n_buffers; i++) {
-        e = hipMalloc(&bufs[(size_t)i], wbytes);
+        e = device_alloc(ctx, &bufs[(size_t)i], wbytes);
         if (e == hipSuccess) e = launch_synth_fill(bufs[(size_t)i], 1, (uint64_t)rows * k, synth_key(98, (uint64_t)i), 0.02, st);
     }
-    if (e == hipSuccess) e = hipMalloc((void **)&x, sizeof(float) * (size_t)k);
-    if (e == hipSuccess) e = hipMalloc((void **)&y, sizeof(float) * (size_t)rows);
-    if (e == hipSuccess) e = hipMalloc((void **)&stamps, sizeof(unsigned long long) * (size_t)launches * max_waves * kS);
+    if (e == hipSuccess) e = device_alloc(ctx, (void **)&x, sizeof(float) * (size_t)k);
+    if (e == hipSuccess) e = device_alloc(ctx, (void **)&y, sizeof(float) * (size_t)rows);
+    if (e == hipSuccess) e = device_alloc(ctx, (void **)&stamps, sizeof(unsigned long long) * (size_t)launches * max_waves * kS);
     if (e == hipSuccess) e = hipMemsetAsync(stamps, 0, sizeof(unsigned long long) * (size_t)launches * max_waves * kS, st);
     if (e == hipSuccess) e = launch_fill_f32(x, (uint64_t)k, 0.5f, st);
     GemvParams p{};

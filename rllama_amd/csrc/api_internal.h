@@ -70,7 +70,7 @@ struct rlh_ctx {
     OpScratch ops;
     // Buffers of freed tensors, guarded by mu.  Everything that touches a tensor's buffer is ordered on the context's one stream (tensors
     // that another context's operation used are not kept: rlh_tensor::lent), so a buffer may be handed out while work of its former owner
-    // is still queued.  Given back by rlh_shutdown.
+    // is still queued.  Given back when memory runs out (device_alloc) and by rlh_shutdown.
     rlh::TensorPool pool;
     Tunables tun;
     unsigned tun_version = 0;        // bumped by rlh_set_option: captured decode steps of an older version are dropped
@@ -101,6 +101,8 @@ struct CtxLock {
 
 namespace rlh {
 void pool_release(rlh_ctx *ctx); // waits for the stream and frees the kept buffers
+// hipMalloc for everything the library holds on the device: when memory runs out, the context's kept buffers are freed first
+hipError_t device_alloc(rlh_ctx *ctx, void **p, size_t bytes);
 } // namespace rlh
 
 // Notes that an operation of `user` is about to use the tensors.

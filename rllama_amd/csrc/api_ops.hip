@@ -27,12 +27,7 @@ extern "C" int rlh_tensor_alloc(rlh_ctx *ctx, int rows, int cols, int dtype, rlh
     hipError_t e = hipSuccess;
     if (!t->p) {
         t->capacity = bytes;
-        e = hipMalloc(&t->p, bytes);
-        if (e == hipErrorOutOfMemory && ctx->pool.count() > 0) {
-            (void)hipGetLastError();
-            pool_release(ctx);
-            e = hipMalloc(&t->p, bytes);
-        }
+        e = device_alloc(ctx, &t->p, bytes);
     }
     if (e == hipSuccess) e = hipMemsetAsync(t->p, 0, bytes, ctx->stream);
     if (e != hipSuccess) {
@@ -230,15 +225,15 @@ extern "C" int rlh_matrix_mul_inplace_transposed(rlh_tensor *dst, const rlh_tens
         g.ldc = mrows;
         g.batch = 1;
         g.f32_operands = f16 ? 0 : 1;
-        if (!dst->ctx->ops.gemm_ws) HIP_TRY(hipMalloc(&dst->ctx->ops.gemm_ws, kOpGemmWsBytes));
+        if (!dst->ctx->ops.gemm_ws) HIP_TRY(device_alloc(dst->ctx, &dst->ctx->ops.gemm_ws, kOpGemmWsBytes));
         g.workspace = dst->ctx->ops.gemm_ws;
         g.workspace_bytes = kOpGemmWsBytes;
         HIP_TRY(launch_gemm_f16(g, f16 ? kGemmEpiF16 : kGemmEpiF32, st));
         return RLH_OK;
     }
     float *xf = nullptr, *yf = nullptr;
-    HIP_TRY(hipMalloc((void **)&xf, sizeof(float) * (size_t)n * k));
-    hipError_t e = hipMalloc((void **)&yf, sizeof(float) * (size_t)n * mrows);
+    HIP_TRY(device_alloc(dst->ctx, (void **)&xf, sizeof(float) * (size_t)n * k));
+    hipError_t e = device_alloc(dst->ctx, (void **)&yf, sizeof(float) * (size_t)n * mrows);
     if (e == hipSuccess) e = launch_convert(xf, 0, src->p, f16, (uint64_t)n * k, st);
     for (int r = 0; e == hipSuccess && r < n; r++) {
         GemvParams p{};
@@ -284,7 +279,7 @@ extern "C" int rlh_rope_inplace(rlh_tensor *x, int n_heads, int head_dim, int po
         tab[(size_t)j] = make_float2((float)std::cos(ang), (float)std::sin(ang));
     }
     float2 *dev = nullptr;
-    HIP_TRY(hipMalloc((void **)&dev, tab.size() * sizeof(float2)));
+    HIP_TRY(device_alloc(x->ctx, (void **)&dev, tab.size() * sizeof(float2)));
     hipError_t e = hipMemcpyAsync(dev, tab.data(), tab.size() * sizeof(float2), hipMemcpyHostToDevice, x->ctx->stream);
     if (e == hipSuccess) e = launch_rope_row((float *)x->p, n_heads, head_dim, dev, x->ctx->stream);
     hipError_t e2 = hipStreamSynchronize(x->ctx->stream);
@@ -335,7 +330,7 @@ extern "C" int rlh_ffn_gate(rlh_tensor *dst, const rlh_tensor *x, const rlh_tens
     g.lda = g.ldb = x->cols;
     g.ldc = w1->rows;
     g.batch = 1;
-    if (!dst->ctx->ops.gemm_ws) HIP_TRY(hipMalloc(&dst->ctx->ops.gemm_ws, kOpGemmWsBytes));
+    if (!dst->ctx->ops.gemm_ws) HIP_TRY(device_alloc(dst->ctx, &dst->ctx->ops.gemm_ws, kOpGemmWsBytes));
     g.workspace = dst->ctx->ops.gemm_ws;
     g.workspace_bytes = kOpGemmWsBytes;
     GemmParams both = g;
@@ -386,7 +381,7 @@ extern "C" int rlh_rope_kvwrite(rlh_tensor *q, const rlh_tensor *k, const rlh_te
     hipStream_t st = q->ctx->stream;
     const std::vector<float2> tab = rope_table(hd, pos, 1);
     float2 *dev = nullptr;
-    HIP_TRY(hipMalloc((void **)&dev, tab.size() * sizeof(float2)));
+    HIP_TRY(device_alloc(q->ctx, (void **)&dev, tab.size() * sizeof(float2)));
     hipError_t e = hipMemcpyAsync(dev, tab.data(), tab.size() * sizeof(float2), hipMemcpyHostToDevice, st);
     if (e == hipSuccess)
         e = launch_rope_kvwrite((float *)q->p, (const float *)k->p, (const float *)v->p, cache_k->p, cache_v->p, cache_k->dtype == RLH_F16, n_heads, hd,
@@ -426,12 +421,12 @@ int attn_splits_rule(int T, int n_heads, int compute_units, int single_max, int 
 static int ensure_op_scratch(rlh_ctx *ctx, size_t attn_ws_floats) {
     OpScratch &o = ctx->ops;
     if (!o.state) {
-        HIP_TRY(hipMalloc((void **)&o.state, sizeof(DecodeState)));
+        HIP_TRY(device_alloc(ctx, (void **)&o.state, sizeof(DecodeState)));
         HIP_TRY(hipMemset(o.state, 0, sizeof(DecodeState)));
     }
-    if (!o.token) HIP_TRY(hipMalloc((void **)&o.token, sizeof(int32_t)));
+    if (!o.token) HIP_TRY(device_alloc(ctx, (void **)&o.token, sizeof(int32_t)));
     if (!o.tickets) {
-        HIP_TRY(hipMalloc((void **)&o.tickets, sizeof(unsigned) * kOpMaxHeads));
+        HIP_TRY(device_alloc(ctx, (void **)&o.tickets, sizeof(unsigned) * kOpMaxHeads));
         HIP_TRY(hipMemset(o.tickets, 0, sizeof(unsigned) * kOpMaxHeads));
     }
     if (attn_ws_floats > o.attn_ws_floats) {
@@ -441,7 +436,7 @@ static int ensure_op_scratch(rlh_ctx *ctx, size_t attn_ws_floats) {
             o.attn_ws = nullptr;
             o.attn_ws_floats = 0;
         }
-        HIP_TRY(hipMalloc((void **)&o.attn_ws, attn_ws_floats * sizeof(float)));
+        HIP_TRY(device_alloc(ctx, (void **)&o.attn_ws, attn_ws_floats * sizeof(float)));
         o.attn_ws_floats = attn_ws_floats;
     }
     return RLH_OK;
@@ -452,6 +447,17 @@ void pool_release(rlh_ctx *ctx) {
     if (ctx->pool.count() == 0) return;
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
     while (void *p = ctx->pool.drop()) (void)hipFree(p);
+}
+
+hipError_t device_alloc(rlh_ctx *ctx, void **p, size_t bytes) {
+    std::lock_guard<std::recursive_mutex> g(ctx->mu);
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory && ctx->pool.count() > 0) {
+        (void)hipGetLastError();
+        pool_release(ctx);
+        e = hipMalloc(p, bytes);
+    }
+    return e;
 }
 
 void ops_release(rlh_ctx *ctx) {
@@ -545,9 +551,9 @@ extern "C" int rlh_attn_prefill(rlh_tensor *out, const rlh_tensor *qkv, rlh_tens
     float2 *freqs = nullptr;
     void *q2 = nullptr, *v_t = nullptr;
     const size_t q2_bytes = (size_t)n * d * 2 * 2, vt_bytes = (size_t)n_heads * hd * tp * 2;
-    hipError_t e = hipMalloc((void **)&freqs, tab.size() * sizeof(float2));
-    if (e == hipSuccess) e = hipMalloc(&q2, q2_bytes);
-    if (e == hipSuccess) e = hipMalloc(&v_t, vt_bytes);
+    hipError_t e = device_alloc(ctx, (void **)&freqs, tab.size() * sizeof(float2));
+    if (e == hipSuccess) e = device_alloc(ctx, &q2, q2_bytes);
+    if (e == hipSuccess) e = device_alloc(ctx, &v_t, vt_bytes);
     if (e == hipSuccess) e = hipMemsetAsync(v_t, 0, vt_bytes, st); // the padding past n must hold finite values
     if (e == hipSuccess) e = hipMemcpyAsync(freqs, tab.data(), tab.size() * sizeof(float2), hipMemcpyHostToDevice, st);
     if (e == hipSuccess) {

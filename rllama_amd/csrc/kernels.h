@@ -257,8 +257,8 @@ hipError_t launch_silu_mul_f16(const void *g, const void *u, void *m, size_t tot
 // RoPE on q (in place) and k at `pos`, k and v into the cache planes [head][position][head_dim] at `pos`
 hipError_t launch_rope_kvwrite(float *q, const float *k, const float *v, void *cache_k, void *cache_v, int cache_f16, int n_heads, int head_dim,
                                int max_seq_len, int pos, const float2 *freqs_at_pos, hipStream_t s);
-// KV-cache services (transformer.rs:180-197): shift positions left by `shifts` within each (head) plane
-hipError_t launch_cache_shift_left(void *cache, int is_f16, size_t planes, int max_seq_len, int head_dim, int shifts, hipStream_t s);
+// KV-cache services (transformer.rs:180-197): shift positions left by `shifts` within each (head) plane; tmp: work memory of the size of the cache
+hipError_t launch_cache_shift_left(void *cache, void *tmp, int is_f16, size_t planes, int max_seq_len, int head_dim, int shifts, hipStream_t s);
 // test hook: [head_dim x max_seq_len] f32 view of one head's plane
 hipError_t launch_cache_read(float *dst, const void *plane, int is_f16, int max_seq_len, int head_dim, hipStream_t s);
 

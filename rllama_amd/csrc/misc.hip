@@ -422,20 +422,15 @@ __global__ void cache_shift_kernel(T *dst, const T *src, size_t planes, int max_
     }
 }
 
-hipError_t launch_cache_shift_left(void *cache, int is_f16, size_t planes, int max_seq_len, int head_dim, int shifts, hipStream_t s) {
+hipError_t launch_cache_shift_left(void *cache, void *tmp, int is_f16, size_t planes, int max_seq_len, int head_dim, int shifts, hipStream_t s) {
     const size_t total = planes * (size_t)max_seq_len * head_dim;
     const size_t bytes = total * (is_f16 ? 2 : 4);
-    void *tmp = nullptr;
-    hipError_t e = hipMalloc(&tmp, bytes);
-    if (e != hipSuccess) return e;
     dim3 g(fill_blocks(total)), b(256);
     if (is_f16) hipLaunchKernelGGL(cache_shift_kernel<half_t>, g, b, 0, s, (half_t *)tmp, (const half_t *)cache, planes, max_seq_len, head_dim, shifts);
     else hipLaunchKernelGGL(cache_shift_kernel<float>, g, b, 0, s, (float *)tmp, (const float *)cache, planes, max_seq_len, head_dim, shifts);
-    e = hipGetLastError();
+    hipError_t e = hipGetLastError();
     if (e == hipSuccess) e = hipMemcpyAsync(cache, tmp, bytes, hipMemcpyDeviceToDevice, s);
-    hipError_t e2 = hipStreamSynchronize(s);
-    (void)hipFree(tmp);
-    return e != hipSuccess ? e : e2;
+    return e;
 }
 
 template <typename T>

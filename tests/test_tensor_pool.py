@@ -1,6 +1,8 @@
 """The bookkeeping of kept device buffers (rllama_amd/csrc/tensor_pool.h), on the CPU: its bounds, which buffer a tensor gets, which one goes
 first, and that a host whose sizes change keeps finding buffers."""
+import glob
 import os
+import re
 import subprocess
 
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "rllama_amd", "csrc")
@@ -92,3 +94,15 @@ def test_kept_buffers_stay_within_bounds_and_follow_their_user(tmp_path):
     r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=300)
     print(r.stdout)
     assert r.returncode == 0, r.stdout
+
+
+def test_every_device_allocation_can_take_the_kept_buffers_back():
+    """When device memory runs out the kept buffers are freed before a call fails: device_alloc does it, so nothing else calls hipMalloc."""
+    for path in sorted(glob.glob(os.path.join(CSRC, "*.hip"))):
+        with open(path) as f:
+            text = re.sub(r"//[^\n]*", "", f.read())
+        if os.path.basename(path) == "api_ops.hip":
+            body = re.search(r"hipError_t device_alloc\(.*?\n}\n", text, re.S).group(0)
+            assert body.index("hipMalloc") < body.index("pool_release") < body.rindex("hipMalloc")
+            text = text.replace(body, "")
+        assert not re.search(r"\bhip(Ext)?Malloc(Async|Managed|WithFlags)?\b", text), path
