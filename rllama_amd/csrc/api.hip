@@ -6,6 +6,7 @@
 // -> rlh_caches; OpenCLTensor (tensor_opencl_support.rs:23-38) -> rlh_tensor.
 #include "../../include/rllama_hip.h"
 #include "api_internal.h"
+#include "split3_plan.h"
 #include "synth.h"
 
 #include <hip/hip_runtime.h>
@@ -74,10 +75,6 @@ struct PrefillScratch {
     void *gemm_ws = nullptr; // fp32 partial sums of split-K products (short prompts); f32 mode: also the parts of one operand
     size_t gemm_ws_bytes = 0;
     bool gemm_attention = false; // the buffers of the two-GEMM form of attention (scores, p2) exist
-    static constexpr size_t kGemmWsBytes = (size_t)64 << 20;
-    // f32 mode: three bf16 parts of an activation matrix (6 bytes per element: 85 MB for 1024 rows of 13824) beside the partial
-    // sums; a product whose rows need more runs in several passes over the weights
-    static constexpr size_t kGemmWsBytesF32 = (size_t)192 << 20;
     void release() {
         void *all[] = {x, h, scores, xn, qkv, q2, v_t, p2, a, g, u, mm, gemm_ws};
         for (void *b : all)
@@ -927,15 +924,19 @@ static int ensure_prefill_scratch(rlh_model *m, int n) {
     A((void **)&S.g, N * F * es);
     if (es == 4) A((void **)&S.u, N * F * es); // f16 mode: w3's epilogue consumes its product on the spot
     A((void **)&S.mm, N * F * es);
-    const size_t ws_bytes = es == 4 ? PrefillScratch::kGemmWsBytesF32 : PrefillScratch::kGemmWsBytes;
-    if (e == hipSuccess) e = device_alloc(m->ctx, &S.gemm_ws, ws_bytes); // (written before it is read, always)
+    // f32 mode: for the product that needs most; the parts of A take 6 bytes per element (85 MB for 1024 rows of 13824).  Written before
+    // it is read, always.
+    size_t need = 0;
+    if (es == 4)
+        for (size_t b : {split3_work_bytes(n, 3 * (int)d, (int)d), split3_work_bytes(n, (int)d, (int)d), split3_work_bytes(n, (int)F, (int)d), split3_work_bytes(n, (int)d, (int)F)})
+            if (b > need) need = b;
+    if (e == hipSuccess) e = gemm_work_reserve(m->ctx, &S.gemm_ws, &S.gemm_ws_bytes, need);
     if (e == hipSuccess) e = hipStreamSynchronize(m->ctx->stream);
     if (e != hipSuccess) {
         S.release();
         return fail(e == hipErrorOutOfMemory ? RLH_ERR_OOM : RLH_ERR_HIP, "prefill work buffers for %d tokens: %s", n, hipGetErrorString(e));
     }
     S.n_cap = n;
-    S.gemm_ws_bytes = ws_bytes;
     S.gemm_attention = gemm_attention;
     S.t_pad = (int)tp;
     return RLH_OK;

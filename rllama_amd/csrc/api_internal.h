@@ -35,9 +35,9 @@ struct OpScratch {
     size_t attn_ws_floats = 0;
     unsigned *tickets = nullptr;   // [kOpMaxHeads]
     int32_t *token = nullptr;      // one id
-    void *gemm_ws = nullptr;       // partial sums of products cut along K and the parts of an fp32 operand (kOpGemmWsBytes)
+    void *gemm_ws = nullptr;       // partial sums of products cut along K and the parts of an fp32 operand (gemm_work_reserve)
+    size_t gemm_ws_bytes = 0;
 };
-constexpr size_t kOpGemmWsBytes = (size_t)192 << 20;
 constexpr int kOpMaxHeads = 1024;
 
 // The library's switches.  Read from the environment (RLLAMA_HIP_<NAME>) once, when the context is made, and changed
@@ -103,6 +103,9 @@ namespace rlh {
 void pool_release(rlh_ctx *ctx); // waits for the stream and frees the kept buffers
 // hipMalloc for everything the library holds on the device: when memory runs out, the context's kept buffers are freed first
 hipError_t device_alloc(rlh_ctx *ctx, void **p, size_t bytes);
+// Work memory of products: kGemmPartialBytes, and where `need` (split3_work_bytes) is more, as much of that as kGemmWorkMax allows -- or
+// what there is already, if memory runs out on the way: products then go in more passes.  Growing waits for the context's stream.
+hipError_t gemm_work_reserve(rlh_ctx *ctx, void **p, size_t *bytes, size_t need);
 } // namespace rlh
 
 // Notes that an operation of `user` is about to use the tensors.

@@ -2,6 +2,7 @@
 // on them, mirroring OpenCLTensor (Noeda/rllama, src/tensor_opencl_support.rs:134-405) plus the steps of the forward the
 // reference runs on the host (attention, residual add, greedy pick) so that each kernel can be checked alone.
 #include "api_internal.h"
+#include "split3_plan.h"
 
 #include <cmath>
 #include <cstdio>
@@ -225,9 +226,10 @@ extern "C" int rlh_matrix_mul_inplace_transposed(rlh_tensor *dst, const rlh_tens
         g.ldc = mrows;
         g.batch = 1;
         g.f32_operands = f16 ? 0 : 1;
-        if (!dst->ctx->ops.gemm_ws) HIP_TRY(device_alloc(dst->ctx, &dst->ctx->ops.gemm_ws, kOpGemmWsBytes));
-        g.workspace = dst->ctx->ops.gemm_ws;
-        g.workspace_bytes = kOpGemmWsBytes;
+        OpScratch &o = dst->ctx->ops;
+        HIP_TRY(gemm_work_reserve(dst->ctx, &o.gemm_ws, &o.gemm_ws_bytes, f16 ? 0 : split3_work_bytes(n, mrows, k)));
+        g.workspace = o.gemm_ws;
+        g.workspace_bytes = o.gemm_ws_bytes;
         HIP_TRY(launch_gemm_f16(g, f16 ? kGemmEpiF16 : kGemmEpiF32, st));
         return RLH_OK;
     }
@@ -330,9 +332,10 @@ extern "C" int rlh_ffn_gate(rlh_tensor *dst, const rlh_tensor *x, const rlh_tens
     g.lda = g.ldb = x->cols;
     g.ldc = w1->rows;
     g.batch = 1;
-    if (!dst->ctx->ops.gemm_ws) HIP_TRY(device_alloc(dst->ctx, &dst->ctx->ops.gemm_ws, kOpGemmWsBytes));
-    g.workspace = dst->ctx->ops.gemm_ws;
-    g.workspace_bytes = kOpGemmWsBytes;
+    OpScratch &o = dst->ctx->ops;
+    HIP_TRY(gemm_work_reserve(dst->ctx, &o.gemm_ws, &o.gemm_ws_bytes, 0));
+    g.workspace = o.gemm_ws;
+    g.workspace_bytes = o.gemm_ws_bytes;
     GemmParams both = g;
     both.b2 = (const _Float16 *)w3->p;
     if (gemm_f16_dual_gate_supported(both)) { // both products in one pass over x
@@ -458,6 +461,27 @@ hipError_t device_alloc(rlh_ctx *ctx, void **p, size_t bytes) {
         e = hipMalloc(p, bytes);
     }
     return e;
+}
+
+hipError_t gemm_work_reserve(rlh_ctx *ctx, void **p, size_t *bytes, size_t need) {
+    size_t want = need <= kGemmPartialBytes ? kGemmPartialBytes : (need + kGemmPartialBytes - 1) / kGemmPartialBytes * kGemmPartialBytes;
+    if (want > kGemmWorkMax) want = kGemmWorkMax;
+    if (*bytes >= want) return hipSuccess;
+    void *grown = nullptr;
+    hipError_t e = device_alloc(ctx, &grown, want);
+    if (e == hipErrorOutOfMemory && want > kGemmPartialBytes) {
+        (void)hipGetLastError();
+        if (*bytes > 0) return hipSuccess;
+        e = device_alloc(ctx, &grown, want = kGemmPartialBytes);
+    }
+    if (e != hipSuccess) return e;
+    if (*p) {
+        (void)hipStreamSynchronize(ctx->stream);
+        (void)hipFree(*p);
+    }
+    *p = grown;
+    *bytes = want;
+    return hipSuccess;
 }
 
 void ops_release(rlh_ctx *ctx) {

@@ -771,7 +771,8 @@ static int choose_split_k(const GemmParams &p, int tile) {
     if (forced <= 1 && blocks > n_cu / 4) s = 2;
     if (s > k_tiles / 4) s = k_tiles / 4;                  // at least 4 K-tiles per piece
     const size_t per = (size_t)p.m * p.n * sizeof(float);
-    if (per > 0 && (size_t)s * per > p.workspace_bytes) s = (long)(p.workspace_bytes / per);
+    const size_t room = p.workspace_bytes < kGemmPartialBytes ? p.workspace_bytes : kGemmPartialBytes; // the same cut whoever's work memory it is
+    if (per > 0 && (size_t)s * per > room) s = (long)(room / per);
     return s < 2 ? 1 : (int)s;
 }
 

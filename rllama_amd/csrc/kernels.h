@@ -139,6 +139,10 @@ struct GemmTune {
     int no_split3;        // GEMM_SPLIT3=0: fp32 products stay on the fp32 matrix instruction
 };
 
+// Work memory of a product: what partial sums of a product cut along K may take, and the most that a fp32 product uses (partial sums and
+// the parts of A, split3_work_bytes)
+constexpr size_t kGemmPartialBytes = (size_t)64 << 20, kGemmWorkMax = (size_t)192 << 20;
+
 struct GemmParams {
     const _Float16 *a;      // [m x k], row stride lda
     const _Float16 *b;      // [n x k], row stride ldb

@@ -9,6 +9,7 @@ namespace rlh {
 constexpr int kS3K = 32;      // k values per K-tile
 constexpr int kS3Cols = 128;  // columns of a workgroup's tile
 constexpr int kS3RowMax = 256; // rows of the highest tile
+constexpr int kS3MaxPieces = 16;
 
 struct Split3Plan {
     int rows = 0;      // rows of A of the next pass over B (0: the work memory is too small)
@@ -50,7 +51,7 @@ inline Split3Plan plan_split3(int m, int n, int k, int ldc, size_t workspace_byt
     const double us_kt = (384.0 * best.tiles + 400.0) / 2200.0;
     const size_t room = workspace_bytes - best.planes_bytes, per = (size_t)best.rows * n * 4;
     double best_t = 0.0;
-    for (int s = 1; s <= 16 && (s == 1 || kt / s >= 4); s++) {
+    for (int s = 1; s <= kS3MaxPieces && (s == 1 || kt / s >= 4); s++) {
         if (s > 1 && ((size_t)s * per > room || n % 4 != 0 || ldc % 4 != 0)) break;
         const long rounds = (tiles * s + n_cu - 1) / n_cu;
         const double t = rounds * (((kt + s - 1) / s) * us_kt + 4.0) + (s > 1 ? 5.0 + s * (double)per * 2.0 / 4e6 : 0.0);
@@ -60,6 +61,12 @@ inline Split3Plan plan_split3(int m, int n, int k, int ldc, size_t workspace_byt
         }
     }
     return best;
+}
+
+// The most work memory that a product of up to `m` rows makes use of: with that much or more its plan is the same.
+inline size_t split3_work_bytes(int m, int n, int k) {
+    const size_t tile = m > kS3RowMax ? kS3RowMax : 32, padded = ((size_t)m + tile - 1) / tile * tile;
+    return padded * k * 6 + (size_t)kS3MaxPieces * m * n * 4;
 }
 
 } // namespace rlh

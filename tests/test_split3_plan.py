@@ -43,6 +43,18 @@ int main() {
                     if (r == 0 && (mb << 20) >= (size_t)256 * k * 6) return printf("m %d k %d refused\n", m, k), 1;
                     (r ? fine : refused)++;
                 }
+    // with what split3_work_bytes asks for, for any number of rows up to the one asked for, the plan is that of more work memory
+    const size_t most = (size_t)192 << 20;
+    for (int k : ks)
+        for (int n : {96, 4096, 12288})
+            for (int cap : {1, 8, 131, 256, 257, 300, 1345, 2048}) {
+                size_t ws = split3_work_bytes(cap, n, k);
+                if (ws > most) continue;
+                for (int m = 1; m <= cap; m++) {
+                    const Split3Plan a = plan_split3(m, n, k, n, ws, 256), b = plan_split3(m, n, k, n, most, 256);
+                    if (a.rows != b.rows || a.tiles != b.tiles || a.m_pad != b.m_pad || a.pieces != b.pieces) return printf("m %d of %d n %d k %d: work memory %zu\n", m, cap, n, k, ws), 1;
+                }
+            }
     printf("%ld fine, %ld refused\n", fine, refused);
     return fine > 0 && refused > 0 ? 0 : 1;
 }
