@@ -81,3 +81,20 @@ def test_lowest_row_tile_in_one_round(ctx, m, n, k):
     got = A.ffn_gate(B, W3).to_numpy()
     with options(ctx, GEMM_DUAL="1"):  # another tile, the same order of additions
         assert np.array_equal(got, A.ffn_gate(B, W3).to_numpy())
+
+
+# wq|wk|wv, wo and w2 of whole prompts on the narrow tiles: dim 1024 has 48, 16 and 16 column tiles (row tiles of 32 up to 160 and 512 rows, of
+# 64 up to 320 and 1024, of 128 up to 640), 2048 has 96 and 32, 3072 has 144 and 48.  RoPE, cache rows and V^T over several row tiles, the
+# residual, and the RMSNorm as a launch of its own; head dimensions 64, 128, 16 and 32
+@pytest.mark.parametrize("dim,heads,ffn,rows", [(1024, 16, 2816, (33, 100, 161, 330, 600)), (1024, 32, 1024, (70, 200)), (1024, 64, 1056, (97,)),
+                                                (2048, 16, 1024, (40, 81, 130)), (3072, 24, 1024, (33, 70))])
+def test_prompt_on_narrow_tiles(ctx, dim, heads, ffn, rows):
+    shape = Shape(dim=dim, n_layers=2, n_heads=heads, ffn_hidden=ffn, vocab_size=64, max_seq_len=640)
+    W = synth_weights(shape, seed=93, std=0.05, norm_ones=False)
+    toks = np.random.default_rng(94).integers(0, shape.vocab_size, 640)
+    om, gm = make_oracle(shape, W, True), make_gpu(ctx, shape, W, True)
+    for n in rows:
+        gc, oc = gm.make_caches(), om.make_caches()
+        assert max_rel_err(gm.forward(toks[:n], 0, gc), om.forward(toks[:n], 0, oc)) < TOL_F16, n
+        assert max_rel_err(gm.forward(toks[n:n + 1], n, gc), om.forward(toks[n:n + 1], n, oc)) < TOL_F16, n
+    gm.free()

@@ -17,8 +17,9 @@ def _product(ctx, a, b):
 
 
 # rows: one to eight 32-row tiles of a workgroup (with both parities of their split between the row groups), remainders, more than
-# one row tile; columns: less than, exactly and just over a tile of 128; k: one K-tile, fewer than the stages, cut along K
-@pytest.mark.parametrize("m,n,k", [(2, 128, 32), (33, 129, 96), (65, 300, 64), (97, 2816, 160), (128, 4096, 4096), (160, 130, 1184), (192, 384, 352),
+# one row tile; columns: less than, exactly and just over a tile of 128; k: one K-tile, fewer than the stages, cut along K.  Two cases, of
+# few columns whose 64-wide tiles divide the compute units, belong to the fp32 instruction.
+@pytest.mark.parametrize("m,n,k", [(2, 128, 32), (2, 129, 32), (32, 300, 32), (255, 130, 512), (224, 300, 96), (33, 129, 96), (65, 300, 64), (97, 2816, 160), (128, 4096, 4096), (160, 130, 1184), (192, 384, 352),
                                    (200, 3072, 1024), (255, 64, 512), (257, 515, 2048), (300, 4096, 4096)])
 def test_split3_product_against_float64(ctx, m, n, k):
     rng = np.random.default_rng(m * 131 + n)
@@ -32,6 +33,7 @@ def test_split3_product_against_float64(ctx, m, n, k):
     assert np.all(np.abs(got - exact) <= bound)
     with options(ctx, GEMM_SPLIT3="0"):
         plain = _product(ctx, a, b)
+    assert np.array_equal(got, plain) == ((m, n) in ((2, 128), (255, 64)))  # the sums of the two ways differ in their last bits
     err, err_plain = (np.linalg.norm(x - exact) / np.linalg.norm(exact) for x in (got, plain))
     assert err <= max(err_plain, 2.0 ** -24), (err, err_plain)
 
