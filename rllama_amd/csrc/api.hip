@@ -968,6 +968,7 @@ static int enqueue_prefill(rlh_model *m, rlh_caches *c, const int32_t *tokens, i
                     const void *gate = nullptr, const float *norm_w = nullptr, int *norm_done = nullptr) -> int {
         GemmParams g{};
         g.tune = m->ctx->tun.gemm;
+        g.compute_units = m->ctx->prop.multiProcessorCount;
         g.a = (const _Float16 *)a;
         g.b = (const _Float16 *)b;
         g.c = cc;
@@ -1017,7 +1018,7 @@ static int enqueue_prefill(rlh_model *m, rlh_caches *c, const int32_t *tokens, i
             // the shape allows, else the product is stored and a kernel of its own does the same
             GemmParams g{};
             g.tune = m->ctx->tun.gemm;
-        g.tune = m->ctx->tun.gemm;
+            g.compute_units = m->ctx->prop.multiProcessorCount;
             g.a = (const _Float16 *)S.xn;
             g.b = (const _Float16 *)L.wqkv.p;
             g.c = S.qkv;
@@ -1060,8 +1061,7 @@ static int enqueue_prefill(rlh_model *m, rlh_caches *c, const int32_t *tokens, i
             for (int part = 0; part < (one_pass ? 1 : 2); part++) {
                 GemmParams g{};
                 g.tune = m->ctx->tun.gemm;
-            g.tune = m->ctx->tun.gemm;
-        g.tune = m->ctx->tun.gemm;
+                g.compute_units = m->ctx->prop.multiProcessorCount;
                 g.a = (const _Float16 *)S.q2 + (size_t)part * hd;
                 g.b = (const _Float16 *)ck;
                 g.c = S.scores;
@@ -1085,8 +1085,7 @@ static int enqueue_prefill(rlh_model *m, rlh_caches *c, const int32_t *tokens, i
                 // h * hd .. of the [n x dim] input of wo (the concat of heads and the rounding point of transformer.rs:783-796)
                 GemmParams g{};
                 g.tune = m->ctx->tun.gemm;
-            g.tune = m->ctx->tun.gemm;
-        g.tune = m->ctx->tun.gemm;
+                g.compute_units = m->ctx->prop.multiProcessorCount;
                 g.a = (const _Float16 *)S.p2;
                 g.b = (const _Float16 *)S.v_t;
                 g.c = S.a;
@@ -1113,7 +1112,7 @@ static int enqueue_prefill(rlh_model *m, rlh_caches *c, const int32_t *tokens, i
             // in one pass over xn; otherwise w1's product goes to memory and w3's epilogue consumes it
             GemmParams g{};
             g.tune = m->ctx->tun.gemm;
-        g.tune = m->ctx->tun.gemm;
+            g.compute_units = m->ctx->prop.multiProcessorCount;
             g.a = (const _Float16 *)S.xn;
             g.b = (const _Float16 *)L.w1.p;
             g.b2 = (const _Float16 *)L.w3.p;
@@ -1185,6 +1184,7 @@ static int enqueue_prefill_f32(rlh_model *m, rlh_caches *c, const int32_t *token
     auto gemm = [&](const void *a, int lda, const void *b, int ldb, float *cc, int ldc, int mm, int nn, int kk, int accumulate) -> int {
         GemmParams g{};
         g.tune = m->ctx->tun.gemm;
+        g.compute_units = m->ctx->prop.multiProcessorCount;
         g.a = (const _Float16 *)a;
         g.b = (const _Float16 *)b;
         g.c = cc;
@@ -1226,7 +1226,7 @@ static int enqueue_prefill_f32(rlh_model *m, rlh_caches *c, const int32_t *token
         {   // scores[h] = q[h] . K[h]^T, tiles above the diagonal skipped (transformer.rs:762-770)
             GemmParams g{};
             g.tune = m->ctx->tun.gemm;
-        g.tune = m->ctx->tun.gemm;
+            g.compute_units = m->ctx->prop.multiProcessorCount;
             g.a = (const _Float16 *)q;
             g.b = (const _Float16 *)ck;
             g.c = S.scores;
@@ -1248,7 +1248,7 @@ static int enqueue_prefill_f32(rlh_model *m, rlh_caches *c, const int32_t *token
         {   // out[h] = P[h] . V[h], written as columns h * hd .. of the [n x dim] input of wo (transformer.rs:777-796)
             GemmParams g{};
             g.tune = m->ctx->tun.gemm;
-        g.tune = m->ctx->tun.gemm;
+            g.compute_units = m->ctx->prop.multiProcessorCount;
             g.a = (const _Float16 *)S.scores;
             g.b = (const _Float16 *)v_t;
             g.c = att;

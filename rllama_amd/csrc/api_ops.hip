@@ -215,6 +215,7 @@ extern "C" int rlh_matrix_mul_inplace_transposed(rlh_tensor *dst, const rlh_tens
         // more than one row: the matrix-core GEMM (fp32 operands need whole K-tiles of 32, else the per-row path below)
         GemmParams g{};
         g.tune = dst->ctx->tun.gemm;
+        g.compute_units = dst->ctx->prop.multiProcessorCount;
         g.a = (const _Float16 *)src->p;
         g.b = (const _Float16 *)other->p;
         g.c = dst->p;
@@ -323,6 +324,7 @@ extern "C" int rlh_ffn_gate(rlh_tensor *dst, const rlh_tensor *x, const rlh_tens
     hipStream_t st = dst->ctx->stream;
     GemmParams g{};
     g.tune = dst->ctx->tun.gemm;
+    g.compute_units = dst->ctx->prop.multiProcessorCount;
     g.a = (const _Float16 *)x->p;
     g.b = (const _Float16 *)w1->p;
     g.c = dst->p;

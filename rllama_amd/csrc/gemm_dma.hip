@@ -566,15 +566,6 @@ static hipError_t launch_dma_epi(const GemmParams &p, int tile, hipStream_t s) {
     }
 }
 
-static int device_compute_units() {
-    static const int n_cu = [] {
-        int dev = 0, cu = 256;
-        if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&cu, hipDeviceAttributeMultiprocessorCount, dev);
-        return cu > 0 ? cu : 256;
-    }();
-    return n_cu;
-}
-
 // Tile choice: time ~ (rounds of workgroups over the compute units) x (work per workgroup) / (efficiency of the tile);
 // larger tiles are more efficient (less L2 -> LDS traffic per flop) but leave compute units idle on small outputs.
 static int choose_tile(const GemmParams &p, double *model_time = nullptr) {
@@ -582,7 +573,7 @@ static int choose_tile(const GemmParams &p, double *model_time = nullptr) {
     if (forced >= 1 && forced <= 3) return forced;
     const int k_halves = p.k * (p.f32_operands ? 2 : 1);
     if (forced == 0 && k_halves % 64 == 0) return 0;
-    const int n_cu = device_compute_units();
+    const int n_cu = p.compute_units;
     const int bms[4] = {128, 256, 256, 256}, bns[4] = {128, 128, 192, 256};
     // relative throughput of a busy compute unit, measured on 7B shapes.  (The 128 x 128 tile of the kernel whose wavefronts
     // split the K-steps, gemm_kgroup.hip, is 1.15 in one round of workgroups, but rating it so here sends products to it in
@@ -731,7 +722,7 @@ static int choose_narrow(const GemmParams &p) {
     if (p.f32_operands || p.batch != 1 || p.split_k > 1 || p.k_seg != 0 || p.causal != 0 || p.b2 != nullptr || p.k % 64 != 0 || p.k < 1024 || p.k > 3072) return -1; // (measured from 1024 on)
     if (p.tune.tile_plus1 != 0 || p.tune.split_k > 1) return -1;
     const int heights[3] = {32, 64, 128}, tiles[3] = {6, 7, 5};
-    const long n_cu = device_compute_units(), least = p.k <= 1024 ? 1 : p.k <= 2048 ? n_cu / 8 : n_cu / 8 + 1;
+    const long n_cu = p.compute_units, least = p.k <= 1024 ? 1 : p.k <= 2048 ? n_cu / 8 : n_cu / 8 + 1;
     for (int i = 0; i < 3; i++) {
         const long blocks = (long)((p.n + 63) / 64) * ((p.m + heights[i] - 1) / heights[i]);
         if (blocks > n_cu) continue;
@@ -752,7 +743,7 @@ static int choose_split_k(const GemmParams &p, int tile) {
     const int k_halves = p.k * (p.f32_operands ? 2 : 1);
     if (tile != 0 || (p.n % 4) != 0 || (p.ldc % 4) != 0 || k_halves % 64 != 0) return 1;
     const int forced = p.tune.split_k;
-    const int n_cu = device_compute_units();
+    const int n_cu = p.compute_units;
     const long blocks = (long)((p.n + 127) / 128) * ((p.m + 127) / 128);
     const int k_tiles = k_halves / 64;
     // Worth it while the partial sums (pieces x m x n floats, written and read back) stay small beside the weights: products
@@ -821,11 +812,11 @@ static int choose_dual(const GemmParams &p, int *cut_cols = nullptr) {
     // 192 rows and loses 16 % at 256.
     const int heights[5] = {32, 64, 128, 192, 256};
     for (int i = 0; i < 5 && (p.m <= 128 || p.k >= 512); i++) // (measured from k = 512 on beyond 128 rows)
-        if ((long)((p.n + 63) / 64) * ((p.m + heights[i] - 1) / heights[i]) <= device_compute_units()) return 3 + i;
+        if ((long)((p.n + 63) / 64) * ((p.m + heights[i] - 1) / heights[i]) <= p.compute_units) return 3 + i;
     double single = 0.0;
     const int tile = choose_tile(p, &single);
     if (tile < 0 || tile > 3 || choose_split_k(p, tile) != 1) return 0;
-    const int n_cu = device_compute_units();
+    const int n_cu = p.compute_units;
     const long cols = (p.n + 191) / 192;
     const long blocks256 = cols * ((p.m + 255) / 256), blocks128 = cols * ((p.m + 127) / 128);
     const double unit256 = 2.0 * 256 * 192 / (1.23 * 1.18);
@@ -948,10 +939,10 @@ hipError_t launch_gemm_f16_dma(const GemmParams &p_in, int epilogue, hipStream_t
         // With at most one workgroup per compute unit anyway, the LDS that a second one would need buys a deeper load
         // pipeline instead (measured on the wo / w2 products of a 1024-token 7B prefill: 108 -> 85 us per launch).
         const long blocks = (long)((p.n + 127) / 128) * ((p.m + 127) / 128) * p.batch;
-        if (blocks <= device_compute_units()) tile = 4;
+        if (blocks <= p.compute_units) tile = 4;
         // one row tile and few column tiles (a short prompt): half the tile width, so that twice the workgroups stream the
         // weights; the pieces of a split product use it too
-        if (p.m <= 128 && (p.batch == 1 || p.split_k > 1) && (long)((p.n + 127) / 128) * 2 <= device_compute_units() && p.k_seg == 0 && p.causal == 0) tile = p.m <= 32 ? 6 : p.m <= 64 ? 7 : 5;
+        if (p.m <= 128 && (p.batch == 1 || p.split_k > 1) && (long)((p.n + 127) / 128) * 2 <= p.compute_units && p.k_seg == 0 && p.causal == 0) tile = p.m <= 32 ? 6 : p.m <= 64 ? 7 : 5;
     }
     // 128 x 128 or 256 x 192 per workgroup it stays: the kernel whose wavefronts split the K-steps instead of the tile
     if (gemm_f16_kgroup_supported(p, epilogue, tile)) return launch_gemm_f16_kgroup(p, epilogue, tile, s);

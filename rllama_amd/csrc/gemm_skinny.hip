@@ -120,15 +120,6 @@ __global__ __launch_bounds__(64 * kSkWaves, 4) void gemm_f16_skinny_kernel(GemmP
     }
 }
 
-static int compute_units() {
-    static const int n_cu = [] {
-        int dev = 0, cu = 256;
-        if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&cu, hipDeviceAttributeMultiprocessorCount, dev);
-        return cu > 0 ? cu : 256;
-    }();
-    return n_cu;
-}
-
 bool gemm_f16_skinny_supported(const GemmParams &p, int epilogue) {
     if (p.tune.no_skinny || p.tune.dual_plus1 != 0 || p.tune.tile_plus1 != 0 || p.tune.split_k != 0 || p.f32_operands || p.batch != 1 || p.split_k > 1 || p.k_seg != 0 || p.causal != 0) return false;
     if (p.m < 1 || p.m > 16 || p.n < 1 || p.k < 1024 || p.k % 32 != 0 || p.lda % 8 != 0 || p.ldb % 8 != 0) return false;
@@ -149,7 +140,7 @@ bool gemm_f16_skinny_supported(const GemmParams &p, int epilogue) {
 template <int kEpi, bool kDual>
 static hipError_t launch_skinny(const GemmParams &p, hipStream_t s) {
     // sixteen wavefronts fit a compute unit: as many per workgroup as let all workgroups run at once
-    const int tiles = (p.n + kSkCols - 1) / kSkCols, n_cu = compute_units();
+    const int tiles = (p.n + kSkCols - 1) / kSkCols, n_cu = p.compute_units;
     if (tiles <= n_cu) hipLaunchKernelGGL((gemm_f16_skinny_kernel<kEpi, kDual, 16>), dim3(tiles), dim3(1024), 0, s, p);
     else if (tiles <= 2 * n_cu) hipLaunchKernelGGL((gemm_f16_skinny_kernel<kEpi, kDual, 8>), dim3(tiles), dim3(512), 0, s, p);
     else hipLaunchKernelGGL((gemm_f16_skinny_kernel<kEpi, kDual, 4>), dim3(tiles), dim3(256), 0, s, p);

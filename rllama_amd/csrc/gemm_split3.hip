@@ -335,15 +335,6 @@ static hipError_t launch_split3(const Split3Params &p, hipStream_t s) {
     return hipGetLastError();
 }
 
-static int compute_units() {
-    static const int n_cu = [] {
-        int dev = 0, cu = 256;
-        if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&cu, hipDeviceAttributeMultiprocessorCount, dev);
-        return cu > 0 ? cu : 256;
-    }();
-    return n_cu;
-}
-
 bool gemm_split3_supported(const GemmParams &p, int epilogue) {
     if (p.tune.no_split3 || !p.f32_operands || epilogue != kGemmEpiF32 || p.batch != 1 || p.k_seg != 0 || p.causal != 0 || p.split_k > 1) return false;
     if (p.m < 1 || p.n < 1 || p.k < kS3K || p.k % kS3K != 0 || p.lda % 4 != 0 || p.ldb % 4 != 0) return false;
@@ -354,8 +345,8 @@ bool gemm_split3_supported(const GemmParams &p, int epilogue) {
     // decomposition first (us, fp32 instruction against this: 1024 x 2816 weights 17 / 25 against 19 / 30 at 32 / 128 rows, 2048 x 2048
     // 16 / 26 against 19 / 29; but 1536 x 1536 20 / 31 against 17 / 28, 2048 x 4096 at 200 rows 56 against 50)
     const int tiles64 = (p.n + 63) / 64;
-    if (((p.n <= 1024 && p.m <= 256) || (p.n <= 2048 && p.m <= 128)) && compute_units() % tiles64 == 0) return false;
-    return plan_split3(p.m, p.n, p.k, p.ldc, p.workspace_bytes, compute_units()).rows > 0; // the first pass, and with it every one
+    if (((p.n <= 1024 && p.m <= 256) || (p.n <= 2048 && p.m <= 128)) && p.compute_units % tiles64 == 0) return false;
+    return plan_split3(p.m, p.n, p.k, p.ldc, p.workspace_bytes, p.compute_units).rows > 0; // the first pass, and with it every one
 }
 
 hipError_t launch_gemm_split3(const GemmParams &p, int epilogue, hipStream_t s) {
@@ -365,7 +356,7 @@ hipError_t launch_gemm_split3(const GemmParams &p, int epilogue, hipStream_t s) 
         part.m = p.m - r0;
         part.a = reinterpret_cast<const half_t *>(reinterpret_cast<const float *>(p.a) + (size_t)r0 * p.lda);
         part.c = reinterpret_cast<float *>(p.c) + (size_t)r0 * p.ldc;
-        const Split3Plan plan = plan_split3(part.m, p.n, p.k, p.ldc, p.workspace_bytes, compute_units());
+        const Split3Plan plan = plan_split3(part.m, p.n, p.k, p.ldc, p.workspace_bytes, p.compute_units);
         if (plan.rows <= 0) return hipErrorInvalidValue;
         part.m = plan.rows;
         unsigned char *planes = reinterpret_cast<unsigned char *>(p.workspace);

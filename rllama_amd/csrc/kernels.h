@@ -135,7 +135,7 @@ struct GemmTune {
     int no_rope_epilogue; // GEMM_ROPE=0: RoPE, q hi/lo, cache rows and V^T as a kernel of their own on the stored wq|wk|wv product
     int no_finish_norm;   // FINISH_NORM=0: the RMSNorm after a split wo / w2 product as a kernel of its own
     int no_kgroup;        // GEMM_KGROUP=0: 128x128 products stay on the kernel whose wavefronts split the tile
-    int no_skinny;        // GEMM_SKINNY=0: f16 products of at most 32 rows stay on the tiled kernels
+    int no_skinny;        // GEMM_SKINNY=0: f16 products of at most 16 rows stay on the tiled kernels
     int no_split3;        // GEMM_SPLIT3=0: fp32 products stay on the fp32 matrix instruction
 };
 
@@ -144,6 +144,7 @@ struct GemmTune {
 constexpr size_t kGemmPartialBytes = (size_t)64 << 20, kGemmWorkMax = (size_t)192 << 20;
 
 struct GemmParams {
+    int compute_units;      // of the context's device: the dispatch rules count rounds of workgroups with it
     const _Float16 *a;      // [m x k], row stride lda
     const _Float16 *b;      // [n x k], row stride ldb
     void *c;                // [m x n], row stride ldc
@@ -189,7 +190,7 @@ bool gemm_f16_dual_gate_supported(const GemmParams &p);
 // hands such products over
 bool gemm_f16_kgroup_supported(const GemmParams &p, int epilogue, int tile);
 hipError_t launch_gemm_f16_kgroup(const GemmParams &p, int epilogue, int tile, hipStream_t s);
-// at most 32 rows (gemm_skinny.hip): one pass over the weights, wavefronts split K
+// at most 16 rows, one fragment (gemm_skinny.hip): one pass over the weights, wavefronts split K
 bool gemm_f16_skinny_supported(const GemmParams &p, int epilogue);
 hipError_t launch_gemm_f16_skinny(const GemmParams &p, int epilogue, hipStream_t s);
 // fp32 operands as three bf16 parts each (gemm_split3.hip): launch_gemm_f16 picks it for unbatched fp32 products with work memory
