@@ -11,8 +11,7 @@
 //
 // Both operands are multiplied by 2^16 first and the sums by 2^-32 at the end, all exact: the last bit of the smallest fp32 number,
 // 2^-149, becomes 2^-133, the last bit of a bf16 number, so the parts hold every value however small.  (Without it values below 2^-109
-// lose bits: 2-norm error 2.2e-3 at 2^-126.  Two more vector instructions per pair: 11008 x 4096 weights, 8 / 64 / 200 / 1024 rows 51 / 75
-// / 178 / 555 -> 53 / 80 / 174 / 560 us per call, 7B prompt of 200 rows unchanged.)
+// lose bits: 2-norm error 2.2e-3 at 2^-126.)
 //
 // Values that the decomposition cannot hold (infinities, and finite values from 2^112 on, whose bf16 part is infinite: x - hi is then not
 // a remainder), and sums from 2^96 on, make every product they enter NaN or infinite.  An element of C that comes out non-finite is
@@ -22,7 +21,7 @@
 //
 // A (the activations, few rows) is decomposed once by a kernel of its own into three bf16 planes laid out as the LDS image of a
 // K-tile, so that staging it is a linear copy.  B (the weights, read once) is staged as fp32 and decomposed by the wavefront
-// that feeds it to the matrix cores: 13 vector instructions per pair of values against 12 MFMAs per fragment and row tile.
+// that feeds it to the matrix cores: 9 vector instructions per pair of values against 12 MFMAs per fragment and row tile.
 //
 // Blocking.  A workgroup owns 32 kT rows x 128 columns and has eight wavefronts: 2 row groups x 2 column groups x 2 K-groups
 // (K-group g takes the g-th 16 of the 32 values of k in a K-tile).  A wavefront's tile is up to 128 x 64, which needs 16 KB of
@@ -72,12 +71,30 @@ struct Split3Params {
     size_t stride_c;             // elements between the pieces' partial sums
 };
 
+// x - hi and the next remainder as v_dot2_f32_bf16 of the converted pair with (-1, 0) or (0, -1): one instruction instead of taking a half
+// out of the pair and subtracting it, and exact for all finite values, subnormals and pairs of any two magnitudes among them (checked
+// against the subtraction).  The constants come out of registers on purpose: as literals they are not what the instruction reads.  11 vector
+// instructions per pair of values without, 9 with it and the scale; call of 11008 x 4096 weights, 8 / 64 / 200 / 1024 rows, no scale and no
+// dot product -> both: 49 / 75 / 171 / 538 -> 45 / 68 / 141 / 541 us (scale alone: 53 / 80 / 174 / 560, 3 % of a 7B prompt of 64 to 100 rows).
 __device__ __forceinline__ void split3(const float8_t x_in, bf8_t &hi, bf8_t &mid, bf8_t &lo) {
-    const float8_t x = x_in * kS3Scale;
+    typedef __attribute__((ext_vector_type(2))) __bf16 bf2_t;
+    unsigned c0 = 0x0000bf80u, c1 = 0xbf800000u; // (-1, 0) and (0, -1)
+    asm("" : "+s"(c0), "+s"(c1));
+    const bf2_t first = __builtin_bit_cast(bf2_t, c0), second = __builtin_bit_cast(bf2_t, c1);
+    float8_t x = x_in * kS3Scale;
+    auto rest = [&](const bf8_t part) {
+#pragma unroll
+        for (int e = 0; e < 8; e += 2) {
+            const bf2_t pair = {part[e], part[e + 1]};
+            x[e] = __builtin_amdgcn_fdot2_f32_bf16(pair, first, x[e], false);
+            x[e + 1] = __builtin_amdgcn_fdot2_f32_bf16(pair, second, x[e + 1], false);
+        }
+    };
     hi = __builtin_convertvector(x, bf8_t);
-    const float8_t r = x - __builtin_convertvector(hi, float8_t); // exact
-    mid = __builtin_convertvector(r, bf8_t);
-    lo = __builtin_convertvector(r - __builtin_convertvector(mid, float8_t), bf8_t);
+    rest(hi);
+    mid = __builtin_convertvector(x, bf8_t);
+    rest(mid);
+    lo = __builtin_convertvector(x, bf8_t);
 }
 
 // A [m x k] fp32 -> planes.  Four threads per row and K-tile: a wavefront reads 16 rows x 128 bytes and writes 1 KiB per plane.
@@ -244,7 +261,7 @@ __global__ __launch_bounds__(64 * kS3Waves) void gemm_split3_kernel(Split3Params
                     for (int q = 0; q < 6; q++)
 #pragma unroll
                         for (int j = 0; j < 2; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[cur][kPa[q]], bs[kBCur][j][kPb[q]], acc[i][j], 0, 0, 0);
-                    if (i + 1 < kA) { // LDS reads first, then B's decomposition (about 52 vector instructions) between the MFMAs
+                    if (i + 1 < kA) { // LDS reads first, then B's decomposition (about 36 vector instructions) between the MFMAs
                         if (i < 2) __builtin_amdgcn_sched_group_barrier(0x100, 5, 0);
                         else __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
 #pragma unroll

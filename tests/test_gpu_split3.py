@@ -58,6 +58,16 @@ def test_split3_product_with_infinities_nan_and_the_largest_values(ctx):
     assert np.all(np.abs(got[ok].astype(np.float64) - want[ok]) <= bound)
 
 
+def test_split3_parts_add_up_to_the_value(ctx):
+    """Rows of the unit matrix pick values out of B: the three parts of every fp32 number below 2^112 (larger ones are not taken apart),
+    whatever stands beside it, add up to it."""
+    rng = np.random.default_rng(9)
+    n, k = 3072, 64
+    sign, exponent, fraction = (rng.integers(0, top, (n, k), dtype=np.uint32) for top in (2, 127 + 112, 1 << 23))
+    b = (sign << 31 | exponent << 23 | fraction).view(f32)
+    assert np.array_equal(_product(ctx, np.eye(k, dtype=f32), b), b.T)
+
+
 # operands down to the smallest fp32 numbers (beside large ones, so that the product is not tiny), and products that are subnormal
 @pytest.mark.parametrize("ea,eb", [(-109, 60), (-120, 60), (60, -126), (-140, 60), (60, -145), (-70, -70), (-20, -115)])
 def test_split3_product_of_tiny_values(ctx, ea, eb):
