@@ -168,7 +168,7 @@ bool tunables_set(Tunables &t, const char *name, const char *value) {
     if (n == "FINISH_NORM") return flag_off(t.gemm.no_finish_norm);
     if (n == "GEMM_KGROUP") return flag_off(t.gemm.no_kgroup);
     if (n == "GEMM_SKINNY") return flag_off(t.gemm.no_skinny);
-    if (n == "GEMM_SPLIT3") return flag_off(t.gemm.no_split3);
+    if (n == "GEMM_SPLIT3") { t.gemm.split3_plus1 = reset ? 0 : (v != 0) + 1; return true; }
     return false;
 }
 

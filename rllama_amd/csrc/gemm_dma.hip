@@ -592,7 +592,8 @@ static int choose_tile(const GemmParams &p, double *model_time = nullptr) {
     // fp32 operands run at a sixteenth of the f16 matrix rate, so what counts there is how evenly the tiles fill the compute
     // units, not the staging: the 128 x 64 tile (tile 5) is a candidate too (7B shape in f32 mode, 384 / 512 prompt rows:
     // 86 -> 65 / 87 -> 67 ms to the first token; its busy-unit throughput measured 0.93 of the 128 x 128 tile's)
-    // (products with so few tiles that they are cut along K instead keep the 128 x 128 tile that the cut expects)
+    // (products with so few tiles that they are cut along K instead keep the 128 x 128 tile that the cut expects; where the bf16 parts of
+    // gemm_split3.hip are faster, products come here only to be timed by gemm_f32_instruction_us)
     const long tiles128 = (long)((p.n + 127) / 128) * ((p.m + 127) / 128);
     if (p.f32_operands && p.batch == 1 && p.k_seg == 0 && p.causal == 0 && p.m > 128 && k_halves % 64 == 0 && tiles128 > n_cu / 4) {
         const long blocks = (long)((p.n + 63) / 64) * ((p.m + 127) / 128);
@@ -773,6 +774,20 @@ static hipError_t launch_split_finish(const GemmParams &p, int splits, hipStream
     const unsigned blocks = (unsigned)((work + 255) / 256 < 4096 ? (work + 255) / 256 : 4096);
     hipLaunchKernelGGL(gemm_split_finish_kernel<kEpi>, dim3(blocks), dim3(256), 0, s, p, (const float *)p.workspace, splits);
     return hipGetLastError();
+}
+
+// Rounds of workgroups x (K-tiles of a piece + 5 us to start and drain), and for a cut product its partial sums and their launch.  Fitted to
+// calls of 2 to 1024 rows, 64 to 12288 columns, K = 64 to 11008 (5 to 7 % standard deviation).
+double gemm_f32_instruction_us(const GemmParams &p) {
+    int tile = choose_tile(p);
+    const int pieces = choose_split_k(p, tile);
+    if (tile == 0 && p.m <= 128 && (long)((p.n + 127) / 128) * 2 <= p.compute_units) tile = p.m <= 32 ? 6 : p.m <= 64 ? 7 : 5;
+    const int rows[8] = {128, 256, 256, 256, 128, 128, 32, 64}, cols[8] = {128, 128, 192, 256, 128, 64, 64, 64};
+    const double us_kt[8] = {2.5, 4.3, 5.5, 7.6, 2.5, 1.3, 0.46, 0.97}; // per K-tile of 32 (the fourth by its area)
+    const long blocks = (long)((p.n + cols[tile] - 1) / cols[tile]) * ((p.m + rows[tile] - 1) / rows[tile]) * pieces;
+    const long rounds = (blocks + p.compute_units - 1) / p.compute_units;
+    const int kt = p.k / 32;
+    return rounds * (5.0 + (kt + pieces - 1) / pieces * us_kt[tile]) + (pieces > 1 ? 2.9 + 0.61e-6 * pieces * 4.0 * p.m * p.n : 0.0);
 }
 
 hipError_t launch_gemm_split_finish_f32(const GemmParams &p, const float *partial, int pieces, hipStream_t s) {

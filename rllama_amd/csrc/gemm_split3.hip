@@ -353,21 +353,22 @@ static hipError_t launch_split3(const Split3Params &p, hipStream_t s) {
 }
 
 bool gemm_split3_supported(const GemmParams &p, int epilogue) {
-    if (p.tune.no_split3 || !p.f32_operands || epilogue != kGemmEpiF32 || p.batch != 1 || p.k_seg != 0 || p.causal != 0 || p.split_k > 1) return false;
+    if (p.tune.split3_plus1 == 1 || !p.f32_operands || epilogue != kGemmEpiF32 || p.batch != 1 || p.k_seg != 0 || p.causal != 0 || p.split_k > 1) return false;
     if (p.m < 1 || p.n < 1 || p.k < kS3K || p.k % kS3K != 0 || p.lda % 4 != 0 || p.ldb % 4 != 0) return false;
     if ((reinterpret_cast<uintptr_t>(p.a) | reinterpret_cast<uintptr_t>(p.b)) % 16 != 0) return false;
     if (p.workspace == nullptr || reinterpret_cast<uintptr_t>(p.workspace) % 16 != 0) return false;
     if ((size_t)kS3Cols * p.ldb * 4 >= ((size_t)1 << 31)) return false; // 32-bit byte offsets within a column tile
-    // Few columns whose 64-wide tiles divide the compute units: the fp32 kernel's pieces make exactly one round there and need no
-    // decomposition first (us, fp32 instruction against this: 1024 x 2816 weights 17 / 25 against 19 / 30 at 32 / 128 rows, 2048 x 2048
-    // 16 / 26 against 19 / 29; but 1536 x 1536 20 / 31 against 17 / 28, 2048 x 4096 at 200 rows 56 against 50)
-    const int tiles64 = (p.n + 63) / 64;
-    if (((p.n <= 1024 && p.m <= 256) || (p.n <= 2048 && p.m <= 128)) && p.compute_units % tiles64 == 0) return false;
-    return plan_split3(p.m, p.n, p.k, p.ldc, p.workspace_bytes, p.compute_units).rows > 0; // the first pass, and with it every one
+    if (p.tune.split3_plus1 == 2) return plan_split3(p.m, p.n, p.k, p.ldc, p.workspace_bytes, p.compute_units).rows > 0; // the first pass, and with it every one
+    // Short rows, and columns whose tiles and pieces on the fp32 instruction make whole rounds, are faster there: one or two launches
+    // instead of two or three, and no decomposition.  No single size separates the two, so their times are estimated and compared: over
+    // 2688 sizes that loses more than 4 % against the better kernel at 28 (at most 12 %).  us, fp32 instruction against this: 704 x 256
+    // weights, 2 / 128 / 512 rows 10 / 17 / 26 against 13 / 22 / 34; 1408 x 1408, 24 / 128 / 512 rows 17 / 24 / 55 against 20 / 28 / 41;
+    // 64 x 2048, 1024 rows 30 against 39; 3072 x 1024, 2 / 200 rows 20 / 49 against 18 / 37.
+    const double us = split3_us(p.m, p.n, p.k, p.ldc, p.workspace_bytes, p.compute_units);
+    return us >= 0.0 && us < gemm_f32_instruction_us(p);
 }
 
-hipError_t launch_gemm_split3(const GemmParams &p, int epilogue, hipStream_t s) {
-    if (!gemm_split3_supported(p, epilogue)) return hipErrorInvalidValue;
+hipError_t launch_gemm_split3(const GemmParams &p, hipStream_t s) {
     for (int r0 = 0; r0 < p.m;) {
         GemmParams part = p;
         part.m = p.m - r0;

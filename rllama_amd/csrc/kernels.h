@@ -136,7 +136,7 @@ struct GemmTune {
     int no_finish_norm;   // FINISH_NORM=0: the RMSNorm after a split wo / w2 product as a kernel of its own
     int no_kgroup;        // GEMM_KGROUP=0: 128x128 products stay on the kernel whose wavefronts split the tile
     int no_skinny;        // GEMM_SKINNY=0: f16 products of at most 16 rows stay on the tiled kernels
-    int no_split3;        // GEMM_SPLIT3=0: fp32 products stay on the fp32 matrix instruction
+    int split3_plus1;     // GEMM_SPLIT3=0 / 1: fp32 products never / wherever the kernel can run as three bf16 parts per value: stored as value + 1
 };
 
 // Work memory of a product: what partial sums of a product cut along K may take, and the most that a fp32 product uses (partial sums and
@@ -193,9 +193,11 @@ hipError_t launch_gemm_f16_kgroup(const GemmParams &p, int epilogue, int tile, h
 // at most 16 rows, one fragment (gemm_skinny.hip): one pass over the weights, wavefronts split K
 bool gemm_f16_skinny_supported(const GemmParams &p, int epilogue);
 hipError_t launch_gemm_f16_skinny(const GemmParams &p, int epilogue, hipStream_t s);
-// fp32 operands as three bf16 parts each (gemm_split3.hip): launch_gemm_f16 picks it for unbatched fp32 products with work memory
+// fp32 operands as three bf16 parts each (gemm_split3.hip): launch_gemm_f16 picks it for unbatched fp32 products with work memory where it is faster than the fp32 instruction
 bool gemm_split3_supported(const GemmParams &p, int epilogue);
-hipError_t launch_gemm_split3(const GemmParams &p, int epilogue, hipStream_t s);
+hipError_t launch_gemm_split3(const GemmParams &p, hipStream_t s); // p: one that gemm_split3_supported takes
+// microseconds of a fp32 product on the fp32 matrix instruction, estimated (gemm_dma.hip)
+double gemm_f32_instruction_us(const GemmParams &p);
 // C (+)= the sum of `pieces` partial sums [m][n] (n and ldc multiples of 4), in their order (gemm_dma.hip)
 hipError_t launch_gemm_split_finish_f32(const GemmParams &p, const float *partial, int pieces, hipStream_t s);
 // whether the fast path applies RoPE and writes q / the cache / V^T straight from the wq|wk|wv product for this shape

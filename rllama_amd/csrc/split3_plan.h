@@ -33,9 +33,10 @@ inline void split3_row_tiles(int rows, Split3Plan &q) {
 //
 // Pieces along K by a model of the time in microseconds -- rounds of workgroups x (K-tiles of a piece x its cycles + 4 us to start and
 // drain), and for a cut product the partial sums written and read back at 4 TB/s and the launch that adds them.  Cycles of a K-tile:
-// 384 MFMA cycles per SIMD and 32-row tile + 400 for the barrier and the decomposition of B's first fragments.  (A lone product
-// measures 0.75 / 1.5 / 2.5 us per K-tile with one / four / eight 32-row tiles; with those in the model it cuts finer, which loses:
-// 11008 x 4096, 8 / 200 rows 53 / 154 -> 63 / 157 us.)
+// 384 MFMA cycles per SIMD and 32-row tile + 400 for the barrier and the decomposition of B's first fragments.  That is what a K-tile
+// costs its compute unit.  It takes longer (0.5 / 1.2 / 2.2 us with one / four / eight 32-row tiles, where this counts 0.36 / 0.88 / 1.6)
+// because all workgroups share the bandwidth that feeds them, and that part does not shrink when more of them run, so it is left out:
+// with it the model cuts finer, which loses (11008 x 4096, 8 / 200 rows 53 / 154 -> 63 / 157 us).
 inline Split3Plan plan_split3(int m, int n, int k, int ldc, size_t workspace_bytes, int n_cu) {
     Split3Plan best;
     const size_t row_bytes = (size_t)k * 6;
@@ -61,6 +62,21 @@ inline Split3Plan plan_split3(int m, int n, int k, int ldc, size_t workspace_byt
         }
     }
     return best;
+}
+
+// Microseconds of all passes, to compare with another kernel: rounds of workgroups, partial sums with their launch, and the kernel that takes
+// A apart.  Negative: no plan.  Fitted to lone calls (10 % standard deviation), so a K-tile counts in full here; see plan_split3.
+inline double split3_us(int m, int n, int k, int ldc, size_t workspace_bytes, int n_cu) {
+    double us = 0.0;
+    for (int left = m; left > 0;) {
+        const Split3Plan q = plan_split3(left, n, k, ldc, workspace_bytes, n_cu);
+        if (q.rows <= 0) return -1.0;
+        const long blocks = (long)((n + kS3Cols - 1) / kS3Cols) * (q.m_pad / (q.tiles * 32)) * q.pieces, rounds = (blocks + n_cu - 1) / n_cu;
+        us += rounds * (5.7 + (k / kS3K + q.pieces - 1) / q.pieces * 0.25 * (q.tiles + 1)) + 2.5 + 3.3e-6 * q.m_pad * (double)k;
+        if (q.pieces > 1) us += 2.9 + 0.62e-6 * q.pieces * 4.0 * q.rows * n;
+        left -= q.rows;
+    }
+    return us;
 }
 
 // The most work memory that a product of up to `m` rows makes use of: with that much or more its plan is the same.
