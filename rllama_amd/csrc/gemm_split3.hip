@@ -359,6 +359,7 @@ bool gemm_split3_supported(const GemmParams &p, int epilogue) {
     if (p.workspace == nullptr || reinterpret_cast<uintptr_t>(p.workspace) % 16 != 0) return false;
     if ((size_t)kS3Cols * p.ldb * 4 >= ((size_t)1 << 31)) return false; // 32-bit byte offsets within a column tile
     if (p.tune.split3_plus1 == 2) return plan_split3(p.m, p.n, p.k, p.ldc, p.workspace_bytes, p.compute_units).rows > 0; // the first pass, and with it every one
+    if (p.tune.tile_plus1 != 0 || p.tune.split_k != 0) return false; // those name tiles and pieces of the fp32 instruction's kernel
     // Short rows, and columns whose tiles and pieces on the fp32 instruction make whole rounds, are faster there: one or two launches
     // instead of two or three, and no decomposition.  No single size separates the two, so their times are estimated and compared: over
     // 2688 sizes that loses more than 4 % against the better kernel at 28 (at most 12 %).  us, fp32 instruction against this: 704 x 256

@@ -50,6 +50,14 @@ def test_the_faster_of_the_two_ways_is_taken(ctx, m, n, k, parts):
     assert np.array_equal(_product(ctx, a, b, None), by_parts if parts else plain)
 
 
+@pytest.mark.parametrize("switch", [{"GEMM_SPLIT_K": "3"}, {"GEMM_TILE": "1"}])
+def test_switches_of_the_fp32_instruction_take_effect(ctx, switch):
+    rng = np.random.default_rng(12)
+    a, b = rng.standard_normal((100, 4096), dtype=f32), rng.standard_normal((3000, 4096), dtype=f32)
+    with options(ctx, **switch):
+        assert np.array_equal(_product(ctx, a, b, None), _product(ctx, a, b, "0"))
+
+
 def test_split3_product_with_infinities_nan_and_the_largest_values(ctx):
     rng = np.random.default_rng(5)
     m, n, k = 40, 3072, 256
