@@ -1,12 +1,13 @@
-// gemm_skinny.hip -- C = A * B^T (f16 operands, fp32 accumulate) for prompts of at most 32 rows, where the product is one pass over
-// the weights B and everything else should stay out of its way.
+// gemm_skinny.hip -- C = A * B^T (f16 operands, fp32 accumulate) for prompts of at most 16 rows (one fragment; more would not be
+// stored), where the product is one pass over the weights B and everything else should stay out of its way.
 //
 // The tiled kernels (gemm_dma.hip) stage B through LDS on 64 columns per workgroup: 172 workgroups for 11008 columns, 64 for
 // 4096, so wo and w2 are cut along K and a second kernel adds the pieces.  Here a workgroup owns 16 columns (of one product, or
-// of w1 and w3 alike) and its eight wavefronts split K among them; B goes from memory straight into the registers that feed
-// v_mfma_f32_16x16x32_f16 (lane l: row l % 16, 8 values of k, 16 bytes), a burst of three or four K-steps in flight
-// while the previous one is consumed, sixteen wavefronts per compute unit, and A -- a few rows, resident in L2 -- comes the same way.  The eight partial sums are added through LDS in
-// the order of the wavefronts, so the result does not depend on timing, and the epilogue has whole sums: no second kernel.
+// of w1 and w3 alike) and its 16, 8 or 4 wavefronts split K among them; B goes from memory straight into the registers that feed
+// v_mfma_f32_16x16x32_f16 (lane l: row l % 16, 8 values of k, 16 bytes), a burst of four K-steps in flight while the previous one
+// is consumed, sixteen wavefronts per compute unit, and A -- a few rows, resident in L2 -- comes the same way.  The wavefronts'
+// partial sums are added through LDS in the order of the wavefronts, so the result does not depend on timing, and the epilogue has
+// whole sums: no second kernel.
 //
 // What bounds it: small products by the latency of their launches, larger ones by what the memory path takes in 64-byte pieces.
 // Time to the first token at 2 / 8 / 16 rows, ms, tiled kernels -> this: dim 1024, 8 layers 0.50 / 0.52 / 0.53 -> 0.41 / 0.43 / 0.44; dim 2048,
@@ -123,10 +124,25 @@ __global__ __launch_bounds__(64 * kSkWaves, 4) void gemm_f16_skinny_kernel(GemmP
 bool gemm_f16_skinny_supported(const GemmParams &p, int epilogue) {
     if (p.tune.no_skinny || p.tune.dual_plus1 != 0 || p.tune.tile_plus1 != 0 || p.tune.split_k != 0 || p.f32_operands || p.batch != 1 || p.split_k > 1 || p.k_seg != 0 || p.causal != 0) return false;
     if (p.m < 1 || p.m > 16 || p.n < 1 || p.k < 1024 || p.k % 32 != 0 || p.lda % 8 != 0 || p.ldb % 8 != 0) return false;
-    // (shorter rows than 1024 leave sixteen wavefronts less than two K-steps each and stay on the tiled kernels)
+    // (rows shorter than 1024 are not measured: they leave sixteen wavefronts less than two K-steps each)
     // Fragments of 16 rows are 64 bytes per row and load instruction, which the memory path takes at about 4.7 TB/s; large products
     // are faster through LDS in whole lines in spite of their second kernel (7B shape, 8 rows: w1|w3 42 us here, 36 there)
     if ((size_t)p.n * p.k * (p.b2 != nullptr ? 4 : 2) > ((size_t)48 << 20)) return false;
+    // What the tiled kernels do better (while K is whole K-tiles of theirs), us, tiled -> this:
+    const int tiles = (p.n + kSkCols - 1) / kSkCols, n_cu = p.compute_units;
+    if (p.k % 64 == 0 && tiles > n_cu) {
+        // Two products on more workgroups than compute units (w1|w3 of 5632 x 2048, 8 / 16 rows: 18.6 -> 19.1 / 20.6; 5120 x 1408: 15.5 -> 17.4 / 19.2).
+        if (p.b2 != nullptr) return false;
+        // One product: eight or four wavefronts share K, and a burst that is not whole requests its last K-step again (8192 columns, 8 / 16 rows:
+        // K = 2048 14.5 -> 12.9 / 13.6, 1536 13 -> 12.5 / 13.9, 1280 12.2 -> 12.9 / -, 2560 17 -> 16.7 / 18.5; 11008 x 2048 15.7 -> 14.8 / 17.1, x 1792
+        // 14.2 -> 15.3 / -).  Beyond K = 3072 the tiled kernels need two launches.
+        const bool whole = p.k % 1024 == 0;
+        if (tiles > 2 * n_cu ? !whole || p.m > 8 : !whole && p.k <= 3072 && p.m > (p.k < 1408 ? 4 : 10)) return false;
+    }
+    // Long rows, where each wavefront's chain of bursts is long and the tiled kernels cut K further: sooner where their 64-wide tiles and pieces
+    // make exactly one round (2048 columns, 7 / 12 / 16 rows: K = 4096 14.5 -> 12 / 12 / 12.5, 5632 15.8 -> 15.2 / 16.1 / 17.2, 8192 18 -> 18 / 19.4 / 20.8;
+    // 7 rows, K = 6912 15.7 -> 17.9; but 2816 columns 26 -> 18.7 / 19.8 / 21 at K = 8192).
+    if (p.b2 == nullptr && (p.k > 8192 || (n_cu % ((p.n + 63) / 64) == 0 && p.k > 4096 && (p.m * p.k > 40000 || (p.k > 6144 && p.k % 2048 != 0))))) return false;
     if ((reinterpret_cast<uintptr_t>(p.a) | reinterpret_cast<uintptr_t>(p.b) | reinterpret_cast<uintptr_t>(p.b2)) % 16 != 0) return false;
     switch (epilogue) {
     case kGemmEpiF16: return p.b2 == nullptr;
@@ -140,8 +156,10 @@ bool gemm_f16_skinny_supported(const GemmParams &p, int epilogue) {
 template <int kEpi, bool kDual>
 static hipError_t launch_skinny(const GemmParams &p, hipStream_t s) {
     // sixteen wavefronts fit a compute unit: as many per workgroup as let all workgroups run at once
-    const int tiles = (p.n + kSkCols - 1) / kSkCols, n_cu = p.compute_units;
-    if (tiles <= n_cu) hipLaunchKernelGGL((gemm_f16_skinny_kernel<kEpi, kDual, 16>), dim3(tiles), dim3(1024), 0, s, p);
+    const int tiles = (p.n + kSkCols - 1) / kSkCols;
+    [[maybe_unused]] const int n_cu = p.compute_units;
+    if constexpr (kDual) hipLaunchKernelGGL((gemm_f16_skinny_kernel<kEpi, kDual, 16>), dim3(tiles), dim3(1024), 0, s, p);
+    else if (tiles <= n_cu) hipLaunchKernelGGL((gemm_f16_skinny_kernel<kEpi, kDual, 16>), dim3(tiles), dim3(1024), 0, s, p);
     else if (tiles <= 2 * n_cu) hipLaunchKernelGGL((gemm_f16_skinny_kernel<kEpi, kDual, 8>), dim3(tiles), dim3(512), 0, s, p);
     else hipLaunchKernelGGL((gemm_f16_skinny_kernel<kEpi, kDual, 4>), dim3(tiles), dim3(256), 0, s, p);
     return hipGetLastError();

@@ -42,8 +42,8 @@ def _check_gate(got, a, w1, w3):
 
 
 # k: two K-steps for each of sixteen wavefronts, a remainder, bursts and a remainder, just below the kernel's range; columns: less than a tile, a remainder, and more tiles than
-# the part has compute units once (8 wavefronts) and twice (4 wavefronts)
-@pytest.mark.parametrize("m,n,k", [(2, 8, 1024), (16, 40, 1056), (7, 4099, 1120), (15, 8216, 1088), (16, 1024, 2080), (9, 2048, 2816), (5, 200, 992)])
+# the part has compute units once (8 wavefronts) and twice (4 wavefronts, at most 8 rows)
+@pytest.mark.parametrize("m,n,k", [(2, 8, 1024), (16, 40, 1056), (7, 4099, 1120), (15, 8216, 1088), (8, 8216, 1088), (16, 1024, 2080), (9, 2048, 2816), (5, 200, 992)])
 def test_product_of_few_rows(ctx, m, n, k):
     rng = np.random.default_rng(m + n + k)
     a, b = _f16(rng, m, k, 1.0), _f16(rng, n, k, 0.05)
@@ -52,6 +52,24 @@ def test_product_of_few_rows(ctx, m, n, k):
     if n % 8 == 0:
         w3 = _f16(rng, n, k, 0.05)
         _check_gate(A.ffn_gate(B, Tensor.from_numpy(ctx, w3)).to_numpy(), a, b, w3)
+
+
+# long rows, tiles that make one round and a half with bursts that are not whole, columns for more than three rounds
+@pytest.mark.parametrize("m,n,k", [(16, 2048, 5632), (2, 1024, 11008), (12, 6144, 2560), (8, 16384, 1408), (8, 5120, 1280), (3, 2048, 6912)])
+def test_few_rows_that_the_tiled_kernels_do_better(ctx, m, n, k):
+    rng = np.random.default_rng(m + n + k)
+    A, B = (Tensor.from_numpy(ctx, _f16(rng, r, k, std)) for r, std in ((m, 1.0), (n, 0.05)))
+    got = A.matrix_mul_transposed(B).to_numpy()
+    with options(ctx, GEMM_SKINNY="0"):
+        assert np.array_equal(got, A.matrix_mul_transposed(B).to_numpy())
+
+
+def test_two_products_of_few_rows_on_more_workgroups_than_compute_units(ctx):
+    rng = np.random.default_rng(95)
+    A, W1, W3 = (Tensor.from_numpy(ctx, _f16(rng, r, 2048, std)) for r, std in ((16, 1.0), (5632, 0.05), (5632, 0.05)))
+    got = A.ffn_gate(W1, W3).to_numpy()
+    with options(ctx, GEMM_SKINNY="0"):
+        assert np.array_equal(got, A.ffn_gate(W1, W3).to_numpy())
 
 
 @pytest.mark.parametrize("dim,heads,ffn", [(1024, 16, 2816), (1024, 8, 1024), (1024, 64, 1056)])
