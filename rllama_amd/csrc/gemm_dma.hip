@@ -800,8 +800,8 @@ hipError_t launch_gemm_split_finish_f32(const GemmParams &p, const float *partia
 // Two products in one pass pay off where their workgroups fill the compute units about as well as the best single-product
 // tile does.  Returns 0 (two launches), 1 (workgroups of 256 x 192 of both products, eight wavefronts, all of the LDS),
 // 2 (128 x 192 of both, four wavefronts: prompts of about 300 to 512 rows, where the 128 x 128 tile of a single product needs two
-// rounds of workgroups and this form one) or 3 / 4 / 5 / 6 / 7 (32 / 64 / 128 / 192 / 256 rows x 64 columns of both: prompts of up to
-// 256 rows).  The model is choose_tile's: rounds of workgroups x outputs per workgroup / relative
+// rounds of workgroups and this form one) or 3 / 4 / 5 / 6 / 7 (32 / 64 / 128 / 192 / 256 rows x 64 columns of both: any number of
+// rows whose tiles make one round).  The model is choose_tile's: rounds of workgroups x outputs per workgroup / relative
 // throughput of a busy compute unit, with 1.23 x 1.18 measured for the 256-row form (7B and 13B shapes, 256 to 2048 prompt
 // rows: faster from 768 rows on except where the last round is nearly empty) and 0.87 for the 128-row form (7B shape: 3 - 4 % of
 // the time to the first token at 384 and 512 rows, slower at 256 and 640).
@@ -825,13 +825,18 @@ static int choose_dual(const GemmParams &p, int *cut_cols = nullptr) {
     // 5632 x 2048, 131 / 200 / 400 rows: 36.7 / 38.7 / 48.1 -> 22.4 / 22.6 / 36.7; 7B shape, 131 / 160 / 192 / 256: 96 / 95 / 95 / 97 -> 62 / 60 /
     // 65 / 80; 13B shape: 124 / 123 / 129 / 132 -> 91 / 91 / 96 / 115.  Beyond one round (65B shape, 344 workgroups) it gains 4 % up to
     // 192 rows and loses 16 % at 256.
+    // Long rows of few columns are faster as two products cut along K where the cut makes exactly one round: it divides K, the pass does not
+    // (us, two launches -> pass: 1024 x 8192 weights, 131 / 512 rows 39 / 50 -> 54 / 56; 4096 x 11008, 131 / 200 rows 74 / 79 -> 93 / 96;
+    // 8192 x 13824, 131 rows 147 -> 166; but 4096 x 5120, 131 rows 49 -> 46, 2816 x 11008 83 -> 73 and 8192 x 8192 101 -> 99).
+    const long tiles128 = (long)((p.n + 127) / 128) * ((p.m + 127) / 128);
+    const int n_cu = p.compute_units;
+    if (p.m > 128 && n_cu % tiles128 == 0 && p.k > (tiles128 <= n_cu / 4 ? 5120 : 11264) && choose_split_k(p, choose_tile(p)) > 1) return 0;
     const int heights[5] = {32, 64, 128, 192, 256};
     for (int i = 0; i < 5 && (p.m <= 128 || p.k >= 512); i++) // (measured from k = 512 on beyond 128 rows)
-        if ((long)((p.n + 63) / 64) * ((p.m + heights[i] - 1) / heights[i]) <= p.compute_units) return 3 + i;
+        if ((long)((p.n + 63) / 64) * ((p.m + heights[i] - 1) / heights[i]) <= n_cu) return 3 + i;
     double single = 0.0;
     const int tile = choose_tile(p, &single);
     if (tile < 0 || tile > 3 || choose_split_k(p, tile) != 1) return 0;
-    const int n_cu = p.compute_units;
     const long cols = (p.n + 191) / 192;
     const long blocks256 = cols * ((p.m + 255) / 256), blocks128 = cols * ((p.m + 127) / 128);
     const double unit256 = 2.0 * 256 * 192 / (1.23 * 1.18);

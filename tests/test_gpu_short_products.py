@@ -101,6 +101,18 @@ def test_lowest_row_tile_in_one_round(ctx, m, n, k):
         assert np.array_equal(got, A.ffn_gate(B, W3).to_numpy())
 
 
+@pytest.mark.parametrize("m,n,k,cut", [(131, 1024, 8192, True), (400, 1024, 5184, True), (131, 1024, 5120, False), (131, 704, 8192, False)])
+def test_two_products_of_long_rows_are_cut(ctx, m, n, k, cut):
+    rng = np.random.default_rng(m + n)
+    A, W1, W3 = (Tensor.from_numpy(ctx, _f16(rng, r, k, std)) for r, std in ((m, 1.0), (n, 0.02), (n, 0.02)))
+    got = A.ffn_gate(W1, W3).to_numpy()
+    same = {}
+    for mode in ("0", "3"):  # two launches, cut along K; one pass, whole sums
+        with options(ctx, GEMM_DUAL=mode):
+            same[mode] = np.array_equal(got, A.ffn_gate(W1, W3).to_numpy())
+    assert same == {"0": cut, "3": not cut}
+
+
 # wq|wk|wv, wo and w2 of whole prompts on the narrow tiles: dim 1024 has 48, 16 and 16 column tiles (row tiles of 32 up to 160 and 512 rows, of
 # 64 up to 320 and 1024, of 128 up to 640), 2048 has 96 and 32, 3072 has 144 and 48.  RoPE, cache rows and V^T over several row tiles, the
 # residual, and the RMSNorm as a launch of its own; head dimensions 64, 128, 16 and 32
