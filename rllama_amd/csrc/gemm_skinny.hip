@@ -11,7 +11,7 @@
 //
 // What bounds it: small products by the latency of their launches, larger ones by what the memory path takes in 64-byte pieces.
 // Time to the first token at 2 / 8 / 16 rows, ms, tiled kernels -> this: dim 1024, 8 layers 0.50 / 0.52 / 0.53 -> 0.41 / 0.43 / 0.44; dim 2048,
-// 16 layers 1.30 / 1.28 / 1.32 -> 0.99 / 1.05 / 1.16; 7B shape (wo only) 3.70 / 3.69 / 3.75 -> 3.61 / 3.61 / 3.70.  At 17 to 32 rows the second
+// 16 layers 1.30 / 1.28 / 1.32 -> 0.99 / 1.05 / 1.16; 7B shape (wo only) 1 to 2 %.  At 17 to 32 rows the second
 // fragment of A per fragment of B costs more than it saves (dim 2048, 32 rows: 1.44 against 1.54).
 #include "kernels.h"
 #include "device_utils.h"
@@ -124,7 +124,7 @@ __global__ __launch_bounds__(64 * kSkWaves, 4) void gemm_f16_skinny_kernel(GemmP
 bool gemm_f16_skinny_supported(const GemmParams &p, int epilogue) {
     if (p.tune.no_skinny || p.tune.dual_plus1 != 0 || p.tune.tile_plus1 != 0 || p.tune.split_k != 0 || p.f32_operands || p.batch != 1 || p.split_k > 1 || p.k_seg != 0 || p.causal != 0) return false;
     if (p.m < 1 || p.m > 16 || p.n < 1 || p.k < 1024 || p.k % 32 != 0 || p.lda % 8 != 0 || p.ldb % 8 != 0) return false;
-    // (rows shorter than 1024 are not measured: they leave sixteen wavefronts less than two K-steps each)
+    // (rows shorter than 1024 are not measured: they leave sixteen wavefronts less than two K-steps each; results are right there too)
     // Fragments of 16 rows are 64 bytes per row and load instruction, which the memory path takes at about 4.7 TB/s; large products
     // are faster through LDS in whole lines in spite of their second kernel (7B shape, 8 rows: w1|w3 42 us here, 36 there)
     if ((size_t)p.n * p.k * (p.b2 != nullptr ? 4 : 2) > ((size_t)48 << 20)) return false;

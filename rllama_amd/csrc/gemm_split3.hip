@@ -4,8 +4,9 @@
 // The fp32 matrix instruction (v_mfma_f32_32x32x2_f32, gemm_dma.hip) retires 64 flop per cycle and SIMD, the bf16 one 1024.
 // Every fp32 value is the sum of three bf16 values exactly -- hi = bf16(x), mid = bf16(x - hi), lo = bf16(x - hi - mid), 8 + 8 +
 // 8 significand bits plus the signs of mid and lo against the 24 of x -- and of the nine products of two such sums the six
-// largest are taken:  lo hi' + hi lo' + mid mid' + mid hi' + hi mid' + hi hi'.  What is left out (mid lo', lo mid', lo lo') is below
-// 2^-25 of a product, half a unit in the last place of fp32.  The sums are fp32 like before, and there are fewer of them: one
+// largest are taken:  lo hi' + hi lo' + mid mid' + mid hi' + hi mid' + hi hi' (the splitting of Henry, Tang and Heinecke, "Leveraging the
+// bfloat16 artificial intelligence datatype for higher-precision computations", 2019).  What is left out, mid lo' and lo mid' of up to
+// 2^-25 of a product each and lo lo' of 2^-34, is at most 2^-24 of it, one rounding of fp32.  The sums are fp32 like before, and there are fewer of them: one
 // addition to the accumulator per 16 values of k and product instead of one per 2.  Six bf16 products cost 6/16 of the fp32
 // instruction's cycles.
 //
@@ -30,10 +31,10 @@
 // stages of B, whose latency is the HBM's.  With an odd number of 32-row tiles the row groups are one tile apart; the K-groups
 // swap row groups, so that every SIMD gets one wavefront of each size.
 //
-// What bounds it: 1024 rows x 4096 x 11008 runs its matrix pipes 64 % busy at 1.88 GHz (power); with fewer rows, 58 % on the
+// What bounds it: 1024 rows x 4096 x 11008 runs its matrix pipes 65 % busy at 1.93 GHz (power); with fewer rows, 58 % on the
 // compute units that have a tile.  Against the fp32 instruction, decomposition of A and sum of the pieces included, us:
-// 11008 x 4096 weights, 16 / 64 / 128 / 200 / 300 / 1024 rows: 84 / 142 / 157 / 271 / 443 / 746 -> 53 / 83 / 110 / 154 / 211 / 515;
-// 4096 x 11008: 64 / 107 / 123 / 206 / 395 / 707 -> 51 / 77 / 99 / 140 / 186 / 472.  7B shape, 200 prompt rows: 38.0 -> 21.6 ms.
+// 11008 x 4096 weights, 16 / 64 / 128 / 200 / 300 / 1024 rows: 87 / 143 / 155 / 270 / 445 / 795 -> 52 / 74 / 97 / 139 / 192 / 541;
+// 4096 x 11008: 68 / 105 / 125 / 205 / 394 / 705 -> 53 / 65 / 87 / 121 / 163 / 448.  7B shape, 200 prompt rows: 38.0 -> 21.0 ms.
 // Error against float64 (2-norm, 200 x 12288 x 4096): 5.0e-7 where the fp32 instruction has 1.15e-6 (fewer additions).
 // Products whose tiles do not fill the compute units are cut along K (partial sums in the workspace, added in order of the
 // pieces by gemm_split_finish_kernel).
