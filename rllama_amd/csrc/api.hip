@@ -1162,7 +1162,8 @@ static bool prefill_f32_supported(const rlh_model *m) {
 }
 
 // Multi-token forward at start_pos == 0 in f32 mode: the same structure as enqueue_prefill on fp32 operands
-// (products of weights as bf16 parts or on the fp32 matrix instruction, whichever is faster; attention on the latter), no rounding points, residual adds as accumulating GEMM epilogues on x in place.
+// (products of weights as bf16 parts or on the fp32 matrix instruction, whichever is faster; attention on the latter), no rounding
+// points, residual adds as accumulating GEMM epilogues on x in place.
 static int enqueue_prefill_f32(rlh_model *m, rlh_caches *c, const int32_t *tokens, int n, const LayerSpan *span = nullptr) {
     int rc = ensure_prefill_scratch(m, n);
     if (rc != RLH_OK) return rc;
