@@ -4,8 +4,8 @@
 // built as a streaming reader:
 //   * a wavefront produces one output row at a time with 16-byte loads per lane (one load instruction
 //     covers 1 KiB of the row), issued in bursts of 8 independent loads (7 to 11 where that divides the row
-//     and 8 does not) whose addresses differ by compile-time offsets, so the per-load instruction overhead
-//     is one VMEM instruction;
+//     and 8 does not; several whole rows where a row is shorter than a burst) whose addresses differ by
+//     compile-time offsets, so the per-load instruction overhead is one VMEM instruction;
 //   * rows are interleaved over all wavefronts of the grid (wave w takes rows w, w + W, ...), so that at
 //     any moment the grid reads one dense window of the matrix, and the launch is sized so that all
 //     wavefronts are resident at once (about 8 per CU);
@@ -31,7 +31,8 @@ size_t gemv_lds_bytes(int k, int w_is_f16, int x_f16) {
     return (size_t)gemv_iters(k, vec) * kWave * vec * (x_f16 ? 2 : 4);
 }
 
-template <typename WT, typename XT, int kEpi, bool kStream, int kBurst = kGemvBurst, bool kEmbed = false, bool kStamp = false>
+template <typename WT, typename XT, int kEpi, bool kStream, int kBurst = kGemvBurst, bool kEmbed = false, bool kStamp = false, int kGroup = 0,
+          int kPV = kGemvPrologueVecs>
 __global__ __launch_bounds__(kGemvThreads) void gemv_kernel(GemvParams p) {
     extern __shared__ uint4_t smem_raw[];
     __shared__ float red[16];
@@ -46,7 +47,7 @@ __global__ __launch_bounds__(kGemvThreads) void gemv_kernel(GemvParams p) {
     // greedy pick gains nothing from it and does not do it.
     // (The stamped measurement build keeps the burst behind the prologue, so that "x staged" and "first burst" stay two phases.)
     constexpr int kPre = (!kStamp && ((RLH_GEMV_PRELOAD_EPIS >> kEpi) & 1)) ? kPreSelf : kPreNone;
-    gemv_body<WT, XT, kEpi, kStream, kPre, kBurst, kEmbed, kStamp>(p, smem_raw, red, rope_f);
+    gemv_body<WT, XT, kEpi, kStream, kPre, kBurst, kEmbed, kStamp, kGroup, kPV>(p, smem_raw, red, rope_f);
 }
 
 static int gemv_blocks(int n_units) {
@@ -69,13 +70,44 @@ static hipError_t launch_gemv_t(GemvParams p, hipStream_t s) {
         hipLaunchKernelGGL(kern, dim3(blocks), dim3(kGemvThreads), lds, s, p);
         return hipGetLastError();
     };
+    // Short rows (up to 8 pieces: k <= 4096 halves or 2048 floats) are bound by latency when they are walked like long ones: a row
+    // of 1024 halves is two of a wavefront's eight load slots, so 32000 rows on 2048 wavefronts are 16 memory round trips one after
+    // the other, and the prologue has no whole burst to request.  Here a burst holds as many whole row units as make about eight loads
+    // (one unit from 8 loads on, 16 at most), the length is a compile-time constant and the prologue loads only the vectors that
+    // exist.  Measured, us per launch (f16):  dim 1024: wq|wk|wv 5.9 -> 4.8, w1|w3 6.5 -> 5.1, wo 3.6 -> 2.95, w2 4.8 -> 3.55, head
+    // 22.8 -> 12.3; dim 2048: 7.7 -> 6.9, 10.8 -> 9.6, 4.5 -> 3.9, head 28.1 -> 21.5; dim 3072: 13.6 -> 11.9, 19.4 -> 17.6, 7.6 -> 5.1,
+    // head 39.6 -> 31.4; dim 4096: 19.0 -> 18.7, 30.2 -> 29.6, 7.5 -> 7.5, head 40.7 -> 40.4.  From 10 pieces on (dim 5120) one burst per
+    // unit is no faster than bursts of 8 (w1|w3 44.6 against 44.9), so longer rows are walked burst by burst.  A lane adds its products in
+    // the same order either way: same bits.
+    const int pieces = gemv_iters(p.k, WVec<WT>::kVec);
+    if (p.stream_weights && !p.burst_fixed && pieces <= kGemvShortPieces) {
+        auto short_rows = [&](auto n_pieces) -> hipError_t {
+            constexpr int kP = decltype(n_pieces)::value;
+            constexpr int kUnit = kP * ((kEpi == kEpiSilu || kEpi == kEpiRopeKv) ? 2 : 1); // loads of one row unit
+            constexpr int kG = kUnit >= kGemvBurst ? 1 : kGemvBurst / kUnit;
+            constexpr int kPV = (kP * kWave * WVec<WT>::kVec + 4 * kGemvThreads - 1) / (4 * kGemvThreads);
+            if constexpr (kEpi == kEpiRopeKv) {
+                if (p.embed_table != nullptr) return launch(gemv_kernel<WT, XT, kEpi, true, kUnit * kG, true, false, kG, kPV>);
+            }
+            return launch(gemv_kernel<WT, XT, kEpi, true, kUnit * kG, false, false, kG, kPV>);
+        };
+        switch (pieces) {
+        case 1: return short_rows(std::integral_constant<int, 1>{});
+        case 2: return short_rows(std::integral_constant<int, 2>{});
+        case 3: return short_rows(std::integral_constant<int, 3>{});
+        case 4: return short_rows(std::integral_constant<int, 4>{});
+        case 5: return short_rows(std::integral_constant<int, 5>{});
+        case 6: return short_rows(std::integral_constant<int, 6>{});
+        case 7: return short_rows(std::integral_constant<int, 7>{});
+        default: return short_rows(std::integral_constant<int, 8>{});
+        }
+    }
     // f16 weights: a burst length that divides the row into whole bursts, where one of these does (pieces of 512 halves per row,
     // LLaMA shapes: 8 / 10 / 16 for dim 4096 / 5120 / 8192, 21.5 -> 22 / 27 / 35 for ffn 11008 / 13824 / 17920; 13 and 43 --
     // dim 6656, ffn 22016 -- have no divisor here and keep the default with its partial last burst).  Same order of additions
     // per lane whatever the burst length, so the same bits.  Measured: w2 of the 7B shape 18.8 -> 17.3 us, wo of the 13B shape
     // 12.2 -> 11.1 us, w2 of the 13B shape 25.7 -> 25.4 us.
     if constexpr (std::is_same<WT, half_t>::value && (kEpi == kEpiStore || kEpi == kEpiStoreArgmax)) {
-        const int pieces = gemv_iters(p.k, WVec<WT>::kVec);
         auto pick = [&](auto burst) -> hipError_t {
             constexpr int kB = decltype(burst)::value;
             if (p.stream_weights) return launch(gemv_kernel<WT, XT, kEpi, true, kB>);

@@ -48,6 +48,8 @@ constexpr int kGemvBurst = RLH_GEMV_BURST; // 16-byte loads per lane issued back
 #define RLH_GEMV_PROLOGUE_VECS 8
 #endif
 constexpr int kGemvPrologueVecs = RLH_GEMV_PROLOGUE_VECS; // float4 loads per thread per prologue batch (one batch covers k <= 1024 * this)
+// Rows of up to this many pieces are short: one burst holds one or more whole row units (gemv.hip has the rule and its figures).
+constexpr int kGemvShortPieces = 8;
 
 template <typename WT>
 struct WVec;
@@ -117,12 +119,12 @@ enum GemvPreload {
 // kBurst: 16-byte loads per lane and burst.  Rows that divide into whole bursts stream about 1 us faster per product than rows
 // whose last burst is a partial one (7B shape, k = 11008 = 21.5 pieces: 18.4 us with bursts of 8 + 8 + 6, 17.3 us with 11 + 11),
 // so the launcher picks a burst length that divides the row where one of the instantiated lengths does.
-template <typename WT, int kEpi, int kBurst = kGemvBurst>
+template <typename WT, int kEpi, int kBurst = kGemvBurst, int kGroup = 0>
 struct GemvShape {
     static constexpr int kVec = WVec<WT>::kVec;
     static constexpr int kMats = (kEpi == kEpiSilu) ? 2 : 1;    // w1 and w3 share x and the epilogue
     static constexpr int kRows = (kEpi == kEpiRopeKv) ? 2 : 1;  // a RoPE pair (2j, 2j+1) is produced by one wave
-    static constexpr int kU = kBurst / (kMats * kRows);         // pieces of one row per burst
+    static constexpr int kU = kBurst / (kMats * kRows * (kGroup > 0 ? kGroup : 1)); // pieces of one row per burst
     static constexpr int kPiece = kWave * kVec;                  // elements one wave-wide load covers
 };
 
@@ -148,6 +150,33 @@ __device__ __forceinline__ bool gemv_issue_first_burst(const GemvParams &p, uint
                 wpre[(u * S::kMats + m) * S::kRows + r] =
                     load16<kStream>(wmat[m] + (size_t)(unit * S::kRows + r) * K + (size_t)u * S::kPiece + lane * S::kVec);
     return true;
+}
+
+// Requests the kGroup whole row units first, first + W, ... of a short-row product (those that exist) into w: entry
+// ((g * kU + u) * kMats + m) * kRows + r is piece u of row r of matrix m of unit g.  Lanes past the end of a row in its last piece are
+// clamped to valid weights (they meet zeros of the padded x).
+template <typename WT, int kEpi, bool kStream, int kBurst, int kGroup>
+__device__ __forceinline__ void gemv_fetch_group(const GemvParams &p, int first, uint4_t (&w)[kBurst]) {
+    using S = GemvShape<WT, kEpi, kBurst, kGroup>;
+    const int lane = threadIdx.x & (kWave - 1);
+    const int n_units = p.n_rows / S::kRows;
+    const int W = gridDim.x * kGemvWaves;
+    const WT *wmat[2] = {reinterpret_cast<const WT *>(p.w), reinterpret_cast<const WT *>(p.w_b)};
+    const int last = min((S::kU - 1) * S::kPiece + lane * S::kVec, p.k - S::kVec); // lane's element in the last piece
+#pragma unroll
+    for (int g = 0; g < kGroup; g++) {
+        const int unit = first + g * W;
+        if (unit < n_units) {
+#pragma unroll
+            for (int u = 0; u < S::kU; u++)
+#pragma unroll
+                for (int m = 0; m < S::kMats; m++)
+#pragma unroll
+                    for (int r = 0; r < S::kRows; r++)
+                        w[((g * S::kU + u) * S::kMats + m) * S::kRows + r] =
+                            load16<kStream>(wmat[m] + (size_t)(unit * S::kRows + r) * p.k + (u == S::kU - 1 ? last : u * S::kPiece + lane * S::kVec));
+        }
+    }
 }
 
 // A running greedy candidate: the largest value seen and the lowest id that holds it, and whether a NaN was seen
@@ -178,12 +207,16 @@ __device__ __forceinline__ void greedy_merge(GreedyBest &g, float ov, int oi, in
 // kEmbed (kEpiRopeKv only): the input row comes from the embedding table (GemvParams::embed_table) instead of p.x.
 // kStamp (measurement builds only): every wavefront records the 100 MHz wall clock at five points into p.stamps.
 constexpr int kGemvStamps = 5; // entry, x staged, first burst consumed, last burst consumed, exit
-template <typename WT, typename XT, int kEpi, bool kStream, int kPre, int kBurst = kGemvBurst, bool kEmbed = false, bool kStamp = false>
+// kGroup: 0 for rows of any length, walked burst by burst; > 0 for short rows, where a burst holds kGroup whole row units.
+// kPV: float4 loads per thread and prologue batch.
+template <typename WT, typename XT, int kEpi, bool kStream, int kPre, int kBurst = kGemvBurst, bool kEmbed = false, bool kStamp = false, int kGroup = 0,
+          int kPV = kGemvPrologueVecs>
 __device__ __forceinline__ void gemv_body(const GemvParams &p, uint4_t *smem_raw, float *red, float2 *rope_f) {
     [[maybe_unused]] unsigned long long stamp[kGemvStamps] = {0, 0, 0, 0, 0};
     if constexpr (kStamp) stamp[0] = wall_clock64();
-    using S = GemvShape<WT, kEpi, kBurst>;
+    using S = GemvShape<WT, kEpi, kBurst, kGroup>;
     constexpr int kVec = S::kVec, kMats = S::kMats, kRows = S::kRows, kU = S::kU, kPiece = S::kPiece;
+    static_assert(kGroup == 0 || !kStamp, "the stamped build walks long rows");
     constexpr bool kArgmax = kEpi == kEpiStoreArgmax;
     XT *xs = reinterpret_cast<XT *>(smem_raw);
 
@@ -199,10 +232,15 @@ __device__ __forceinline__ void gemv_body(const GemvParams &p, uint4_t *smem_raw
     wmat[0] = reinterpret_cast<const WT *>(p.w);
     if constexpr (kMats == 2) wmat[1] = reinterpret_cast<const WT *>(p.w_b);
     const int unit_first = blockIdx.x * kGemvWaves + wave;
-    uint4_t wpre[kBurst];
+    uint4_t wpre[kBurst] = {};
     bool have_pre = false;
     auto preload = [&]() {
-        if constexpr (kPre == kPreSelf) have_pre = gemv_issue_first_burst<WT, kEpi, kStream, kBurst>(p, wpre);
+        if constexpr (kGroup > 0) {
+            gemv_fetch_group<WT, kEpi, kStream, kBurst, kGroup>(p, unit_first, wpre);
+            have_pre = true;
+        } else if constexpr (kPre == kPreSelf) {
+            have_pre = gemv_issue_first_burst<WT, kEpi, kStream, kBurst>(p, wpre);
+        }
         __builtin_amdgcn_sched_barrier(0);
     };
 
@@ -225,24 +263,24 @@ __device__ __forceinline__ void gemv_body(const GemvParams &p, uint4_t *smem_raw
         const int half_hd = p.head_dim / 2;
         if (tid < half_hd) rope_early = p.freqs[(size_t)pos * half_hd + tid];
     }
-    // one prologue batch of the input vector: kGemvPrologueVecs float4 per thread starting at float4 index `base`; the source is
+    // one prologue batch of the input vector: kPV float4 per thread starting at float4 index `base`; the source is
     // chosen once, outside the unrolled loads, so that all loads of the batch are issued back to back
-    auto load_batch = [&](int base, int n4, float4_t (&xv)[kGemvPrologueVecs]) {
+    auto load_batch = [&](int base, int n4, float4_t (&xv)[kPV]) {
         const float4_t *x4 = reinterpret_cast<const float4_t *>(p.x);
         if constexpr (kEmbed) {
             if (emb_h != nullptr) {
                 typedef __attribute__((ext_vector_type(4))) _Float16 half4_t;
-                half4_t hv[kGemvPrologueVecs];
+                half4_t hv[kPV];
 #pragma unroll
-                for (int j = 0; j < kGemvPrologueVecs; j++) hv[j] = *reinterpret_cast<const half4_t *>(emb_h + (size_t)min(base + tid + j * kGemvThreads, n4 - 1) * 4);
+                for (int j = 0; j < kPV; j++) hv[j] = *reinterpret_cast<const half4_t *>(emb_h + (size_t)min(base + tid + j * kGemvThreads, n4 - 1) * 4);
 #pragma unroll
-                for (int j = 0; j < kGemvPrologueVecs; j++) xv[j] = float4_t{(float)hv[j][0], (float)hv[j][1], (float)hv[j][2], (float)hv[j][3]};
+                for (int j = 0; j < kPV; j++) xv[j] = float4_t{(float)hv[j][0], (float)hv[j][1], (float)hv[j][2], (float)hv[j][3]};
                 return;
             }
             if (emb_f != nullptr) x4 = reinterpret_cast<const float4_t *>(emb_f);
         }
 #pragma unroll
-        for (int j = 0; j < kGemvPrologueVecs; j++) xv[j] = x4[min(base + tid + j * kGemvThreads, n4 - 1)];
+        for (int j = 0; j < kPV; j++) xv[j] = x4[min(base + tid + j * kGemvThreads, n4 - 1)];
     };
     auto load_in1 = [&](int i) -> float {
         if constexpr (kEmbed) {
@@ -259,26 +297,26 @@ __device__ __forceinline__ void gemv_body(const GemvParams &p, uint4_t *smem_raw
     const float4_t *a4 = reinterpret_cast<const float4_t *>(p.x_add);
     float4_t *o4 = reinterpret_cast<float4_t *>(p.x_out);
     for (int i = K + tid; i < kpad; i += kGemvThreads) xs[i] = (XT)0.0f;
-    if (p.norm_w != nullptr && n4 <= kGemvPrologueVecs * kGemvThreads) {
+    if (p.norm_w != nullptr && n4 <= kPV * kGemvThreads) {
         // RMSNorm::forward (transformer.rs:476-480): (x * rsqrt(mean(x^2) + eps)) * w, x kept in registers
         const float4_t *w4 = reinterpret_cast<const float4_t *>(p.norm_w);
-        float4_t xv[kGemvPrologueVecs], av[kGemvPrologueVecs], wv[kGemvPrologueVecs];
+        float4_t xv[kPV], av[kPV], wv[kPV];
         load_batch(0, n4, xv);
         if (a4 != nullptr) {
 #pragma unroll
-            for (int j = 0; j < kGemvPrologueVecs; j++) av[j] = a4[min(tid + j * kGemvThreads, n4 - 1)];
+            for (int j = 0; j < kPV; j++) av[j] = a4[min(tid + j * kGemvThreads, n4 - 1)];
         }
 #pragma unroll
-        for (int j = 0; j < kGemvPrologueVecs; j++) wv[j] = w4[min(tid + j * kGemvThreads, n4 - 1)];
+        for (int j = 0; j < kPV; j++) wv[j] = w4[min(tid + j * kGemvThreads, n4 - 1)];
         if (a4 != nullptr) {
 #pragma unroll
-            for (int j = 0; j < kGemvPrologueVecs; j++) xv[j] = xv[j] + av[j]; // transformer.rs:442 / :445
+            for (int j = 0; j < kPV; j++) xv[j] = xv[j] + av[j]; // transformer.rs:442 / :445
         }
         __builtin_amdgcn_sched_barrier(0);
         preload();
         float ss = 0.0f;
 #pragma unroll
-        for (int j = 0; j < kGemvPrologueVecs; j++) {
+        for (int j = 0; j < kPV; j++) {
             const int i = tid + j * kGemvThreads;
             if (i < n4) {
                 if (writes_sum) o4[i] = xv[j];
@@ -289,7 +327,7 @@ __device__ __forceinline__ void gemv_body(const GemvParams &p, uint4_t *smem_raw
         ss = block_sum(ss, red);
         const float rs = 1.0f / sqrtf(ss / (float)K + p.eps);
 #pragma unroll
-        for (int j = 0; j < kGemvPrologueVecs; j++) {
+        for (int j = 0; j < kPV; j++) {
             const int i = tid + j * kGemvThreads;
             if (i < n4) {
 #pragma unroll
@@ -314,21 +352,21 @@ __device__ __forceinline__ void gemv_body(const GemvParams &p, uint4_t *smem_raw
             xs[i] = (XT)as_f32((v * rs) * p.norm_w[i]);
         }
     } else {
-        for (int base = 0; base < n4; base += kGemvPrologueVecs * kGemvThreads) {
-            float4_t xv[kGemvPrologueVecs], av[kGemvPrologueVecs];
+        for (int base = 0; base < n4; base += kPV * kGemvThreads) {
+            float4_t xv[kPV], av[kPV];
             load_batch(base, n4, xv);
             if (a4 != nullptr) {
 #pragma unroll
-                for (int j = 0; j < kGemvPrologueVecs; j++) av[j] = a4[min(base + tid + j * kGemvThreads, n4 - 1)];
+                for (int j = 0; j < kPV; j++) av[j] = a4[min(base + tid + j * kGemvThreads, n4 - 1)];
 #pragma unroll
-                for (int j = 0; j < kGemvPrologueVecs; j++) xv[j] = xv[j] + av[j];
+                for (int j = 0; j < kPV; j++) xv[j] = xv[j] + av[j];
             }
-            if (base + kGemvPrologueVecs * kGemvThreads >= n4) { // behind the loads of the last batch: x stays ahead of it in the return queue
+            if (base + kPV * kGemvThreads >= n4) { // behind the loads of the last batch: x stays ahead of it in the return queue
                 __builtin_amdgcn_sched_barrier(0);
                 preload();
             }
 #pragma unroll
-            for (int j = 0; j < kGemvPrologueVecs; j++) {
+            for (int j = 0; j < kPV; j++) {
                 const int i = base + tid + j * kGemvThreads;
                 if (i < n4) {
                     if (writes_sum) o4[i] = xv[j];
@@ -348,7 +386,6 @@ __device__ __forceinline__ void gemv_body(const GemvParams &p, uint4_t *smem_raw
     //      grid reads one dense window of the matrix ----
     const int n_units = p.n_rows / kRows; // n_rows is a multiple of kRows (checked on the host)
     const int W = gridDim.x * kGemvWaves;
-    float acc[kMats][kRows];
     [[maybe_unused]] GreedyBest gb{-INFINITY, -1, 0}; // kArgmax: this wavefront's candidate (meaningful in lane 63)
     // the loads of the burst that starts at piece c of row unit `unit`
     auto fetch = [&](int unit, int c, uint4_t (&wv)[kU][kMats][kRows]) {
@@ -390,7 +427,7 @@ __device__ __forceinline__ void gemv_body(const GemvParams &p, uint4_t *smem_raw
         }
     };
     // products of one burst against x from LDS
-    auto mac = [&](int c, const uint4_t (&wv)[kU][kMats][kRows]) {
+    auto mac = [&](int c, const uint4_t (&wv)[kU][kMats][kRows], float (&acc)[kMats][kRows]) {
 #pragma unroll
         for (int u = 0; u < kU; u++) {
             if (c + u < pieces) {
@@ -409,7 +446,7 @@ __device__ __forceinline__ void gemv_body(const GemvParams &p, uint4_t *smem_raw
         }
     };
     // reduce (valid in lane 63) and epilogue of one row unit
-    auto finish = [&](int unit) {
+    auto finish = [&](int unit, const float (&acc)[kMats][kRows]) {
         const int row0 = unit * kRows;
         float v[kMats][kRows];
 #pragma unroll
@@ -463,65 +500,104 @@ __device__ __forceinline__ void gemv_body(const GemvParams &p, uint4_t *smem_raw
         }
     };
 
-    // (Measured and not kept: a wavefront requesting the first burst of its last row unit together with the last burst of the
-    // unit before, so that the partial last round of units -- 768 of 2048 wavefronts on the 7B shape's 11008 rows -- costs no
-    // memory latency of its own: the isolated 11008 x 4096 product 16.45 -> 17.25 us, w1|w3 30.1 -> 30.6 us, and with the code
-    // in place but switched off w2 17.1 -> 17.7 us.)
-    // The burst the prologue requested (pieces 0 .. kU - 1 of the first row unit) is consumed at the head of that unit.  With
-    // kAhead the first burst of the *next* unit is requested before the reduction and epilogue of the current one run, so
-    // that those run under its memory latency.
-    constexpr bool kAhead = !kStamp && ((RLH_GEMV_AHEAD_EPIS >> kEpi) & 1);
-    const bool burst0_full = kU <= pieces_full;
-    bool have = false;
-    if constexpr (kPre != kPreNone) have = have_pre;
-    for (int unit = unit_first; unit < n_units; unit += W) {
+    if constexpr (kGroup > 0) {
+        // ---- short rows: a burst is kGroup whole units, so that a wavefront has as many loads in flight as on long rows and the
+        //      next burst is requested in front of the reductions of the current one.  The units of a wavefront stay W apart (the
+        //      grid sweeps one dense window), the additions of a lane keep the order of the pieces. ----
+        static_assert(kU * kMats * kRows * kGroup == kBurst, "whole units per burst");
+        for (int unit = unit_first; unit < n_units; unit += W * kGroup) {
+            float acc[kGroup][kMats][kRows];
 #pragma unroll
-        for (int m = 0; m < kMats; m++)
+            for (int g = 0; g < kGroup; g++)
 #pragma unroll
-            for (int r = 0; r < kRows; r++) acc[m][r] = 0.0f;
-        int c_first = 0;
-        if constexpr (kPre != kPreNone || kAhead) {
-            if (have) {
+                for (int m = 0; m < kMats; m++)
+#pragma unroll
+                    for (int r = 0; r < kRows; r++) acc[g][m][r] = 0.0f;
+#pragma unroll
+            for (int u = 0; u < kU; u++) {
+                float xv[kVec];
+                load_x<XT, kVec>(xs + u * kPiece + lane * kVec, xv);
+#pragma unroll
+                for (int g = 0; g < kGroup; g++)
+#pragma unroll
+                    for (int m = 0; m < kMats; m++)
+#pragma unroll
+                        for (int r = 0; r < kRows; r++) {
+                            float wf[kVec];
+                            WVec<WT>::unpack(wpre[((g * kU + u) * kMats + m) * kRows + r], wf);
+#pragma unroll
+                            for (int i = 0; i < kVec; i++) acc[g][m][r] = fmaf(wf[i], xv[i], acc[g][m][r]);
+                        }
+            }
+            __builtin_amdgcn_sched_barrier(0); // the registers of the burst are free
+            gemv_fetch_group<WT, kEpi, kStream, kBurst, kGroup>(p, unit + W * kGroup, wpre);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int g = 0; g < kGroup; g++)
+                if (unit + g * W < n_units) finish(unit + g * W, acc[g]);
+        }
+    } else {
+        // (Measured and not kept: a wavefront requesting the first burst of its last row unit together with the last burst of the
+        // unit before, so that the partial last round of units -- 768 of 2048 wavefronts on the 7B shape's 11008 rows -- costs no
+        // memory latency of its own: the isolated 11008 x 4096 product 16.45 -> 17.25 us, w1|w3 30.1 -> 30.6 us, and with the code
+        // in place but switched off w2 17.1 -> 17.7 us.)
+        // The burst the prologue requested (pieces 0 .. kU - 1 of the first row unit) is consumed at the head of that unit.  With
+        // kAhead the first burst of the *next* unit is requested before the reduction and epilogue of the current one run, so
+        // that those run under its memory latency.
+        constexpr bool kAhead = !kStamp && ((RLH_GEMV_AHEAD_EPIS >> kEpi) & 1);
+        const bool burst0_full = kU <= pieces_full;
+        bool have = false;
+        if constexpr (kPre != kPreNone) have = have_pre;
+        for (int unit = unit_first; unit < n_units; unit += W) {
+            float acc[kMats][kRows];
+#pragma unroll
+            for (int m = 0; m < kMats; m++)
+#pragma unroll
+                for (int r = 0; r < kRows; r++) acc[m][r] = 0.0f;
+            int c_first = 0;
+            if constexpr (kPre != kPreNone || kAhead) {
+                if (have) {
+                    uint4_t wv[kU][kMats][kRows];
+#pragma unroll
+                    for (int u = 0; u < kU; u++)
+#pragma unroll
+                        for (int m = 0; m < kMats; m++)
+#pragma unroll
+                            for (int r = 0; r < kRows; r++) wv[u][m][r] = wpre[(u * kMats + m) * kRows + r];
+                    mac(0, wv, acc);
+                    c_first = kU;
+                    have = false;
+                }
+            }
+            for (int c = c_first; c < pieces; c += kU) {
                 uint4_t wv[kU][kMats][kRows];
-#pragma unroll
-                for (int u = 0; u < kU; u++)
-#pragma unroll
-                    for (int m = 0; m < kMats; m++)
-#pragma unroll
-                        for (int r = 0; r < kRows; r++) wv[u][m][r] = wpre[(u * kMats + m) * kRows + r];
-                mac(0, wv);
-                c_first = kU;
-                have = false;
+                fetch(unit, c, wv);
+                mac(c, wv, acc);
+                if constexpr (kStamp) {
+                    // (the products depend on the loaded data, and the clock is read behind them)
+                    asm volatile("" : "+v"(acc[0][0]));
+                    const unsigned long long now = wall_clock64();
+                    if (stamp[2] == 0) stamp[2] = now;
+                    stamp[3] = now;
+                }
             }
-        }
-        for (int c = c_first; c < pieces; c += kU) {
-            uint4_t wv[kU][kMats][kRows];
-            fetch(unit, c, wv);
-            mac(c, wv);
-            if constexpr (kStamp) {
-                // (the products depend on the loaded data, and the clock is read behind them)
-                asm volatile("" : "+v"(acc[0][0]));
-                const unsigned long long now = wall_clock64();
-                if (stamp[2] == 0) stamp[2] = now;
-                stamp[3] = now;
+            if constexpr (kAhead) {
+                const int next = unit + W;
+                if (next < n_units && burst0_full) {
+#pragma unroll
+                    for (int u = 0; u < kU; u++)
+#pragma unroll
+                        for (int m = 0; m < kMats; m++)
+#pragma unroll
+                            for (int r = 0; r < kRows; r++)
+                                wpre[(u * kMats + m) * kRows + r] =
+                                    load16<kStream>(wmat[m] + (size_t)(next * kRows + r) * K + (size_t)u * kPiece + lane * kVec);
+                    have = true;
+                    __builtin_amdgcn_sched_barrier(0);
+                }
             }
+            finish(unit, acc);
         }
-        if constexpr (kAhead) {
-            const int next = unit + W;
-            if (next < n_units && burst0_full) {
-#pragma unroll
-                for (int u = 0; u < kU; u++)
-#pragma unroll
-                    for (int m = 0; m < kMats; m++)
-#pragma unroll
-                        for (int r = 0; r < kRows; r++)
-                            wpre[(u * kMats + m) * kRows + r] =
-                                load16<kStream>(wmat[m] + (size_t)(next * kRows + r) * K + (size_t)u * kPiece + lane * kVec);
-                have = true;
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        }
-        finish(unit);
     }
     if constexpr (kStamp) {
         stamp[4] = wall_clock64();
