@@ -17,8 +17,8 @@ CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "_obj")
 LIB = os.path.join(HERE, "librllama_hip.so")
 
-SOURCES = ["gemv.hip", "attention.hip", "gemm.hip", "gemm_dma.hip", "gemm_kgroup.hip", "gemm_split3.hip", "gemm_skinny.hip", "attn_prefill.hip", "prefill.hip", "prefill_f32.hip", "misc.hip", "sampler.hip", "api.hip", "api_ops.hip"]
-HEADERS = ["kernels.h", "device_utils.h", "gemv_device.h", "gemm_epilogue.h", "split3_plan.h", "tensor_pool.h", "synth.h", "api_internal.h", os.path.join("..", "..", "include", "rllama_hip.h")]  # relative to csrc/
+SOURCES = ["gemv.hip", "attention.hip", "gemm.hip", "gemm_dma.hip", "gemm_kgroup.hip", "gemm_split3.hip", "gemm_skinny.hip", "gemm_rows.hip", "gemm_rows_fused.hip", "attn_prefill.hip", "prefill.hip", "prefill_f32.hip", "misc.hip", "sampler.hip", "api.hip", "api_ops.hip"]
+HEADERS = ["kernels.h", "device_utils.h", "gemv_device.h", "gemm_epilogue.h", "gemm_rows_device.h", "split3_plan.h", "tensor_pool.h", "synth.h", "api_internal.h", os.path.join("..", "..", "include", "rllama_hip.h")]  # relative to csrc/
 
 HIPCC = os.environ.get("HIPCC") or shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
 FLAGS = [
@@ -61,7 +61,7 @@ def build(force: bool = False) -> str:
     if not force and not _stale():
         return LIB
     os.makedirs(OBJ, exist_ok=True)
-    with ThreadPoolExecutor(max_workers=4) as ex:
+    with ThreadPoolExecutor(max_workers=8) as ex:
         objs = list(ex.map(_compile, _sources()))
     cmd = [HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB, *objs, "-lpthread"]
     r = subprocess.run(cmd, capture_output=True, text=True)

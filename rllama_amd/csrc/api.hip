@@ -168,6 +168,7 @@ bool tunables_set(Tunables &t, const char *name, const char *value) {
     if (n == "FINISH_NORM") return flag_off(t.gemm.no_finish_norm);
     if (n == "GEMM_KGROUP") return flag_off(t.gemm.no_kgroup);
     if (n == "GEMM_SKINNY") return flag_off(t.gemm.no_skinny);
+    if (n == "GEMM_ROWS") return flag_off(t.gemm.no_rows);
     if (n == "GEMM_SPLIT3") { t.gemm.split3_plus1 = reset ? 0 : (v != 0) + 1; return true; }
     return false;
 }
@@ -175,7 +176,7 @@ bool tunables_set(Tunables &t, const char *name, const char *value) {
 void tunables_from_env(Tunables &t) {
     static const char *const names[] = {"GEMV_BURST", "ATTN_CHUNK", "ATTN_SINGLE_MAX", "ATTN_MERGE", "ATTN_LDS", "PREFILL_ATTN", "PREFILL_ATTN_ORDER",
                                         "DECODE_GRAPH", "DECODE_FOLD", "GEMM_TILE", "GEMM_SPLIT_K", "GEMM_SPLIT_HALF", "GEMM_DUAL", "GEMM_DUAL_CUT",
-                                        "GEMM_ROPE", "FINISH_NORM", "GEMM_KGROUP", "GEMM_SKINNY", "GEMM_SPLIT3"};
+                                        "GEMM_ROPE", "FINISH_NORM", "GEMM_KGROUP", "GEMM_SKINNY", "GEMM_ROWS", "GEMM_SPLIT3"};
     for (const char *name : names) {
         const std::string env = std::string("RLLAMA_HIP_") + name;
         const char *val = getenv(env.c_str());
@@ -1123,7 +1124,7 @@ static int enqueue_prefill(rlh_model *m, rlh_caches *c, const int32_t *tokens, i
             g.lda = g.ldb = d;
             g.ldc = F;
             g.batch = 1;
-            g.workspace = S.gemm_ws; // the same policy as rlh_ffn_gate: whether the pass runs is decided with the work memory in place
+            g.workspace = S.gemm_ws; // whether the pass runs is decided with the work memory in place, as for rlh_ffn_gate
             g.workspace_bytes = S.gemm_ws_bytes;
             if (gemm_f16_dual_gate_supported(g)) {
                 HIP_TRY(launch_gemm_f16(g, kGemmEpiSiluGateF16, st));

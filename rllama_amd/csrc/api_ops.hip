@@ -334,6 +334,7 @@ extern "C" int rlh_ffn_gate(rlh_tensor *dst, const rlh_tensor *x, const rlh_tens
     g.lda = g.ldb = x->cols;
     g.ldc = w1->rows;
     g.batch = 1;
+    g.keep_order = 1;
     OpScratch &o = dst->ctx->ops;
     HIP_TRY(gemm_work_reserve(dst->ctx, &o.gemm_ws, &o.gemm_ws_bytes, 0));
     g.workspace = o.gemm_ws;

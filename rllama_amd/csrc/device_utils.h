@@ -4,6 +4,9 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+#include <utility>
+
 namespace rlh {
 
 typedef _Float16 half_t;
@@ -135,6 +138,17 @@ __device__ __forceinline__ void dma16(const half_t *src, unsigned dst) {
 // registers per load address of the form above.
 __device__ __forceinline__ void dma16_base(const half_t *base, unsigned byte_off, unsigned dst) {
     asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(byte_off), "s"(base), "s"(dst) : "memory");
+}
+
+// f(integral_constant<int, 0>), f(integral_constant<int, 1>), ...: a loop whose index is a compile-time constant in every
+// iteration (register arrays indexed by it stay in registers)
+template <typename F, int... I>
+__device__ __forceinline__ void static_for_impl(F &&f, std::integer_sequence<int, I...>) {
+    (f(std::integral_constant<int, I>{}), ...);
+}
+template <int kN, typename F>
+__device__ __forceinline__ void static_for(F &&f) {
+    static_for_impl(static_cast<F &&>(f), std::make_integer_sequence<int, kN>{});
 }
 
 template <int kN>

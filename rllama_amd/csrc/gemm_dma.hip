@@ -797,6 +797,14 @@ hipError_t launch_gemm_split_finish_f32(const GemmParams &p, const float *partia
     return hipGetLastError();
 }
 
+// Long rows of few columns are faster as two products cut along K where the cut makes exactly one round: it divides K, the pass does not
+// (us, two launches -> pass: 1024 x 8192 weights, 131 / 512 rows 39 / 50 -> 54 / 56; 4096 x 11008, 131 / 200 rows 74 / 79 -> 93 / 96;
+// 8192 x 13824, 131 rows 147 -> 166; but 4096 x 5120, 131 rows 49 -> 46, 2816 x 11008 83 -> 73 and 8192 x 8192 101 -> 99).
+bool gemm_f16_gate_cut(const GemmParams &p) {
+    const long tiles128 = (long)((p.n + 127) / 128) * ((p.m + 127) / 128);
+    return p.m > 128 && p.compute_units % tiles128 == 0 && p.k > (tiles128 <= p.compute_units / 4 ? 5120 : 11264) && choose_split_k(p, choose_tile(p)) > 1;
+}
+
 // Two products in one pass pay off where their workgroups fill the compute units about as well as the best single-product
 // tile does.  Returns 0 (two launches), 1 (workgroups of 256 x 192 of both products, eight wavefronts, all of the LDS),
 // 2 (128 x 192 of both, four wavefronts: prompts of about 300 to 512 rows, where the 128 x 128 tile of a single product needs two
@@ -825,12 +833,8 @@ static int choose_dual(const GemmParams &p, int *cut_cols = nullptr) {
     // 5632 x 2048, 131 / 200 / 400 rows: 36.7 / 38.7 / 48.1 -> 22.4 / 22.6 / 36.7; 7B shape, 131 / 160 / 192 / 256: 96 / 95 / 95 / 97 -> 62 / 60 /
     // 65 / 80; 13B shape: 124 / 123 / 129 / 132 -> 91 / 91 / 96 / 115.  Beyond one round (65B shape, 344 workgroups) it gains 4 % up to
     // 192 rows and loses 16 % at 256.
-    // Long rows of few columns are faster as two products cut along K where the cut makes exactly one round: it divides K, the pass does not
-    // (us, two launches -> pass: 1024 x 8192 weights, 131 / 512 rows 39 / 50 -> 54 / 56; 4096 x 11008, 131 / 200 rows 74 / 79 -> 93 / 96;
-    // 8192 x 13824, 131 rows 147 -> 166; but 4096 x 5120, 131 rows 49 -> 46, 2816 x 11008 83 -> 73 and 8192 x 8192 101 -> 99).
-    const long tiles128 = (long)((p.n + 127) / 128) * ((p.m + 127) / 128);
+    if (gemm_f16_gate_cut(p)) return 0;
     const int n_cu = p.compute_units;
-    if (p.m > 128 && n_cu % tiles128 == 0 && p.k > (tiles128 <= n_cu / 4 ? 5120 : 11264) && choose_split_k(p, choose_tile(p)) > 1) return 0;
     const int heights[5] = {32, 64, 128, 192, 256};
     for (int i = 0; i < 5 && (p.m <= 128 || p.k >= 512); i++) // (measured from k = 512 on beyond 128 rows)
         if ((long)((p.n + 63) / 64) * ((p.m + heights[i] - 1) / heights[i]) <= n_cu) return 3 + i;
@@ -871,7 +875,7 @@ static int choose_dual(const GemmParams &p, int *cut_cols = nullptr) {
 
 bool gemm_f16_dual_gate_supported(const GemmParams &p) {
     int n1 = 0;
-    if (gemm_f16_skinny_supported(p, kGemmEpiSiluGateF16)) return true;
+    if (gemm_f16_rows_pieces(p, kGemmEpiSiluGateF16) == 1 || gemm_f16_skinny_supported(p, kGemmEpiSiluGateF16)) return true;
     return choose_dual(p, &n1) != 0;
 }
 
@@ -886,14 +890,16 @@ bool gemm_f16_rope_supported(const GemmParams &p) {
     for (const void *q : {(const void *)R.q_hi, (const void *)R.q_lo, (const void *)R.cache_k, (const void *)R.cache_v, (const void *)R.v_t})
         if (q == nullptr || (reinterpret_cast<uintptr_t>(q) % 16) != 0) return false;
     if (R.freqs == nullptr || (reinterpret_cast<uintptr_t>(R.freqs) % 8) != 0) return false;
-    return gemm_f16_skinny_supported(p, kGemmEpiRopeQkv) || choose_split_k(p, choose_tile(p)) == 1;
+    return gemm_f16_rows_pieces(p, kGemmEpiRopeQkv) == 1 || gemm_f16_skinny_supported(p, kGemmEpiRopeQkv) || choose_split_k(p, choose_tile(p)) == 1;
 }
 
 hipError_t launch_gemm_f16_dma(const GemmParams &p_in, int epilogue, hipStream_t s) {
     if (!gemm_f16_dma_supported(p_in) || p_in.m <= 0 || p_in.n <= 0 || p_in.batch < 1) return hipErrorInvalidValue;
     if (epilogue == kGemmEpiResAddF32 && (p_in.residual == nullptr || p_in.batch != 1)) return hipErrorInvalidValue;
     if (epilogue == kGemmEpiRopeQkv && !gemm_f16_rope_supported(p_in)) return hipErrorInvalidValue;
-    if (gemm_f16_skinny_supported(p_in, epilogue)) return launch_gemm_f16_skinny(p_in, epilogue, s);
+    const int rows_pieces = gemm_f16_rows_pieces(p_in, epilogue);
+    if (rows_pieces == 1) return launch_gemm_f16_rows(p_in, epilogue, s);
+    if (rows_pieces == 0 && gemm_f16_skinny_supported(p_in, epilogue)) return launch_gemm_f16_skinny(p_in, epilogue, s);
     if (p_in.b2 != nullptr) {
         int n1 = 0;
         const int dual = epilogue == kGemmEpiSiluGateF16 ? choose_dual(p_in, &n1) : 0;
@@ -924,7 +930,7 @@ hipError_t launch_gemm_f16_dma(const GemmParams &p_in, int epilogue, hipStream_t
         return hipErrorInvalidValue;
     }
     if (epilogue == kGemmEpiSiluGateF16 && (p_in.gate == nullptr || p_in.batch != 1 || p_in.f32_operands)) return hipErrorInvalidValue;
-    const int splits = choose_split_k(p_in, choose_tile(p_in));
+    const int splits = rows_pieces > 1 ? rows_pieces : choose_split_k(p_in, choose_tile(p_in));
     if (splits > 1) {
         GemmParams q = p_in;            // the partial sums: split_k pieces as grid.z, fp32 store, C item z = workspace slice z
         q.c = p_in.workspace;
@@ -936,7 +942,7 @@ hipError_t launch_gemm_f16_dma(const GemmParams &p_in, int epilogue, hipStream_t
         q.ldc = p_in.n;
         q.stride_c = (size_t)p_in.m * p_in.n;
         q.workspace = nullptr;
-        hipError_t e = launch_gemm_f16_dma(q, kGemmEpiF32, s);
+        hipError_t e = rows_pieces > 1 ? launch_gemm_f16_rows(q, kGemmEpiF32, s) : launch_gemm_f16_dma(q, kGemmEpiF32, s);
         if (e != hipSuccess) return e;
         if (epilogue == kGemmEpiResAddF32 && p_in.norm_w != nullptr && p_in.norm_out != nullptr && p_in.norm_done != nullptr &&
             p_in.n <= 256 * 4 * kFinishNormVecs && !p_in.tune.no_finish_norm) {

@@ -11,18 +11,19 @@ namespace rlh {
 // consecutive columns, each of which lies within q, k or v of one head -- RoPE on q and k in fp32 (transformer.rs:823-856), q
 // as hi + lo f16 halves for the attention kernel, k and v rounded into the cache (tensor.rs:373-376), and v once more
 // transposed, 8 positions per piece.  rows_end: the end of the rows that all tiles of the launch cover together.
-template <int kRows, int kTW, int kTS>
+// kLanes threads share the work; `lane` is the thread's number among them.
+template <int kRows, int kTW, int kTS, int kLanes = 64>
 __device__ __forceinline__ void rope_qkv_from_tile(const half_t *tile, int lane, int wr0, int wc0, int M, int N, int rows_end, const PrefillRopeParams &R) {
     constexpr int kChunks = kTW / 8;
     const int d = R.dim, hd = R.head_dim, half_hd = hd / 2;
     half_t *qhi = reinterpret_cast<half_t *>(R.q_hi), *qlo = reinterpret_cast<half_t *>(R.q_lo);
     half_t *ck = reinterpret_cast<half_t *>(R.cache_k), *cv = reinterpret_cast<half_t *>(R.cache_v);
 #pragma unroll
-    for (int it = 0; it < kChunks * kRows / 64; it++) {
-        const int idx = it * 64 + lane;
+    for (int it = 0; it < (kChunks * kRows + kLanes - 1) / kLanes; it++) {
+        const int idx = it * kLanes + lane;
         const int rr = idx / kChunks, ch = idx - rr * kChunks;
         const int r = wr0 + rr, c = wc0 + ch * 8;
-        if (r < M && c < N) {
+        if (rr < kRows && r < M && c < N) {
             const half8_t o = *reinterpret_cast<const half8_t *>(tile + rr * kTS + ch * 8);
             const int part = c / d, cin = c - part * d; // 0 q, 1 k, 2 v
             const int head = cin / hd, d0 = cin - head * hd;
@@ -58,11 +59,11 @@ __device__ __forceinline__ void rope_qkv_from_tile(const half_t *tile, int lane,
         half_t *vt = reinterpret_cast<half_t *>(R.v_t);
         constexpr int kPieces = kRows / 8;
 #pragma unroll
-        for (int it = 0; it < kTW * kPieces / 64; it++) {
-            const int idx = it * 64 + lane;
+        for (int it = 0; it < (kTW * kPieces + kLanes - 1) / kLanes; it++) {
+            const int idx = it * kLanes + lane;
             const int cc = idx / kPieces, j = idx - cc * kPieces;
             const int c = wc0 + cc, pos0 = wr0 + j * 8;
-            if (c >= 2 * d && c < N && pos0 < R.t_pad) {
+            if (cc < kTW && c >= 2 * d && c < N && pos0 < R.t_pad) {
                 half8_t o;
 #pragma unroll
                 for (int e = 0; e < 8; e++) {
@@ -77,7 +78,7 @@ __device__ __forceinline__ void rope_qkv_from_tile(const half_t *tile, int lane,
         // left behind the last row tile must not be infinite or NaN (tiles of 32 and 64 rows end before t_pad, a multiple of 128)
         if (wr0 + kRows == rows_end) {
             const int pieces = (R.t_pad - rows_end) / 8; // negative: nothing to do
-            for (int idx = lane; idx < kTW * pieces; idx += 64) {
+            for (int idx = lane; idx < kTW * pieces; idx += kLanes) {
                 const int cc = idx / pieces, c = wc0 + cc;
                 if (c >= 2 * d && c < N)
                     *reinterpret_cast<half8_t *>(vt + (size_t)(c - 2 * d) * R.t_pad + rows_end + (idx - cc * pieces) * 8) = half8_t{0, 0, 0, 0, 0, 0, 0, 0};

@@ -9,17 +9,6 @@
 
 namespace rlh {
 
-// f(integral_constant<int, 0>), f(integral_constant<int, 1>), ...: a loop whose index is a compile-time constant in every
-// iteration (register arrays indexed by it stay in registers)
-template <typename F, int... I>
-__device__ __forceinline__ void static_for_impl(F &&f, std::integer_sequence<int, I...>) {
-    (f(std::integral_constant<int, I>{}), ...);
-}
-template <int kN, typename F>
-__device__ __forceinline__ void static_for(F &&f) {
-    static_for_impl(static_cast<F &&>(f), std::make_integer_sequence<int, kN>{});
-}
-
 // Launch shape (overridable at compile time for tuning runs).
 #ifndef RLH_GEMV_WAVES
 #define RLH_GEMV_WAVES 4

@@ -135,7 +135,8 @@ struct GemmTune {
     int no_rope_epilogue; // GEMM_ROPE=0: RoPE, q hi/lo, cache rows and V^T as a kernel of their own on the stored wq|wk|wv product
     int no_finish_norm;   // FINISH_NORM=0: the RMSNorm after a split wo / w2 product as a kernel of its own
     int no_kgroup;        // GEMM_KGROUP=0: 128x128 products stay on the kernel whose wavefronts split the tile
-    int no_skinny;        // GEMM_SKINNY=0: f16 products of at most 16 rows stay on the tiled kernels
+    int no_skinny;        // GEMM_SKINNY=0: the kernel of gemm_skinny.hip takes nothing
+    int no_rows;          // GEMM_ROWS=0: f16 products of at most 160 rows stay on the kernels for any number of rows
     int split3_plus1;     // GEMM_SPLIT3=0 / 1: fp32 products never / wherever the kernel can run as three bf16 parts per value: stored as value + 1
 };
 
@@ -176,6 +177,8 @@ struct GemmParams {
     _Float16 *norm_out;     // [m x n], row stride n
     float norm_eps;
     int *norm_done;         // host flag
+    int keep_order;         // 1 (rlh_ffn_gate): beyond 16 rows only kernels that add in the order of gemm_dma.hip's, so that one pass and
+                            // two launches give the same bits
     GemmTune tune;          // the context's switches (zero = defaults)
     PrefillRopeParams rope; // kGemmEpiRopeQkv: the destinations (qkv unused; n = m, 3 dim = n, f16 cache, vt_swap as the reader expects)
 };
@@ -193,6 +196,12 @@ hipError_t launch_gemm_f16_kgroup(const GemmParams &p, int epilogue, int tile, h
 // at most 16 rows, one fragment (gemm_skinny.hip): one pass over the weights, wavefronts split K
 bool gemm_f16_skinny_supported(const GemmParams &p, int epilogue);
 hipError_t launch_gemm_f16_skinny(const GemmParams &p, int epilogue, hipStream_t s);
+// at most 160 rows (gemm_rows.hip), one row tile, wavefronts split K.  0: the product is for the other kernels; 1: in one launch; more: in that
+// many pieces along K, launched with the kGemmEpiF32 epilogue and split_k = batch = pieces
+int gemm_f16_rows_pieces(const GemmParams &p, int epilogue);
+// whether w1 and w3 are better as two products, each cut along K, than in one pass (gemm_dma.hip)
+bool gemm_f16_gate_cut(const GemmParams &p);
+hipError_t launch_gemm_f16_rows(const GemmParams &p, int epilogue, hipStream_t s); // p: one that gemm_f16_rows_pieces takes, or its pieces
 // fp32 operands as three bf16 parts each (gemm_split3.hip): launch_gemm_f16 picks it for unbatched fp32 products with work memory where it is faster than the fp32 instruction
 bool gemm_split3_supported(const GemmParams &p, int epilogue);
 hipError_t launch_gemm_split3(const GemmParams &p, hipStream_t s); // p: one that gemm_split3_supported takes

@@ -4,10 +4,20 @@ import numpy as np
 import pytest
 
 import oracle
+import rllama_amd
 from common import Shape, make_gpu, options, synth_weights
 from rllama_amd import Tensor
 
 pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture
+def ctx():
+    """A context of its own: what these tensors leave in the pool of freed buffers goes with it."""
+    c = rllama_amd.Context(0)
+    yield c
+    c.close()
+
 
 # row lengths around the pieces of 512 halves / 256 floats (1 to 8, and 9, which is walked); rows: fewer than wavefronts of the grid, one
 # round of a group and a rest, several groups and a rest
