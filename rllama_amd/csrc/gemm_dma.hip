@@ -24,6 +24,7 @@
 namespace rlh {
 
 constexpr int kDmaMinBK = 32;
+constexpr int kDmaEvery = 2; // fragment pairs per requested load (1 and 2 measured alike)
 
 typedef __attribute__((ext_vector_type(16))) float float16_t;
 
@@ -115,11 +116,11 @@ __global__ __launch_bounds__(128 * kWavesM) void gemm_f16_dma_kernel(GemmParams 
     }
     const unsigned lds_base = (unsigned)(uintptr_t)(__attribute__((address_space(3))) void *)lds_raw;
     int iss_t = 0, iss_ka = 0, iss_kb = 0; // the K-tile the next issue() loads: index within its segment, k offsets in A and B
-    auto issue = [&](int kt) {             // called for kt = 0, 1, 2, ... in this order
+    auto issue_load = [&](int kt, int i) { // load i of K-tile kt; the loads of kt = 0, 1, 2, ... in this order, issue_done behind each
         const unsigned dst = lds_base + (unsigned)(kt % kStages) * kStageBytes + (unsigned)wave * 1024;
-#pragma unroll
-        for (int i = 0; i < kLoadsMax; i++)
-            if (i < kLoadsMin || !short_wave) dma16(gsrc[i] + (src_is_b[i] ? iss_kb : iss_ka), dst + i * (kWaves * 1024));
+        if (i < kLoadsMin || !short_wave) dma16(gsrc[i] + (src_is_b[i] ? iss_kb : iss_ka), dst + i * (kWaves * 1024));
+    };
+    auto issue_done = [&](int kt) {
         if (kt + 1 < n_kt) { // past the end the last tile is loaded again (keeps the in-flight count constant)
             if (++iss_t == tps) {
                 iss_t = 0;
@@ -201,6 +202,12 @@ __global__ __launch_bounds__(128 * kWavesM) void gemm_f16_dma_kernel(GemmParams 
     // with K-tile t + kStages.  Registers: the operand fragments of K-step s + 1 are read from LDS while the MFMAs
     // of K-step s run (two fragment sets, selected by the parity of the unrolled K-step); the tile change sits in
     // the middle of the last K-step's MFMAs so that the barrier and the LDS latency behind it stay covered.
+    // Where the loads of a K-tile are requested: a wavefront that requests them all at once at the tile change stands in the queue of the
+    // memory path until the last is taken, its fragment reads and MFMAs behind it.  With four stages or more they are spread over the
+    // MFMAs instead, one per kDmaEvery fragment pairs (7B shape, 131 rows: wq|wk|wv on 128 x 64 44.4 -> 39.9 us, w1|w3 on 192 x 64 58.2 -> 54.4).
+    // With two or three, K-tile t + 1 has to arrive while K-tile t is consumed, and what counts is that it is requested early (256 x 192, 7B
+    // wq|wk|wv of 1024 rows 107 us at once, 114 - 117 spread).
+    constexpr bool kSpread = kStages >= 4;
     constexpr int kKS = kBK / 16;
     constexpr int kSplitJ = kNTs / 2; // column tiles of the last K-step whose MFMAs run before the tile change (0 .. kNT measured alike)
     static_assert(kKS % 2 == 0, "fragment sets alternate by K-step parity");
@@ -215,12 +222,11 @@ __global__ __launch_bounds__(128 * kWavesM) void gemm_f16_dma_kernel(GemmParams 
             c = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
         }
     };
-    auto read_frags = [&](int set, const unsigned char *stage, int ks) {
+    // fragment r of K-step ks: those of A, then those of B
+    auto read_frag = [&](int set, const unsigned char *stage, int ks, int r) {
         const int lc = ks * 2 + fch;
-#pragma unroll
-        for (int i = 0; i < kIT; i++) af[set][i] = *reinterpret_cast<const half8_t *>(stage + a_off[i] + ((lc ^ a_sw[i]) << 4));
-#pragma unroll
-        for (int j = 0; j < (kDual ? 0 : kNT); j++) bf[set][j] = *reinterpret_cast<const half8_t *>(stage + b_off[j] + ((lc ^ b_sw[j]) << 4));
+        if (r < kIT) af[set][r] = *reinterpret_cast<const half8_t *>(stage + a_off[r] + ((lc ^ a_sw[r]) << 4));
+        else bf[set][r - kIT] = *reinterpret_cast<const half8_t *>(stage + b_off[r - kIT] + ((lc ^ b_sw[r - kIT]) << 4));
     };
     if constexpr (kDual) {
         // Two products: 192 accumulator registers of the 256 a wavefront has here, so everything else is kept small.  Staging
@@ -246,131 +252,162 @@ __global__ __launch_bounds__(128 * kWavesM) void gemm_f16_dma_kernel(GemmParams 
         }
         const half_t *s_a = A + (size_t)bm0 * p.lda, *s_b = B + (size_t)bn0 * p.ldb, *s_b2 = p.b2 + (size_t)bn0 * p.ldb;
         int iss_k = 0;
-        auto issue2 = [&](int kt) {
-            const unsigned dst = lds_base + (unsigned)(kt % kStages) * kStageBytes + (unsigned)wave * 1024;
-#pragma unroll
-            for (int i = 0; i < kLA; i++) dma16_base(s_a + iss_k, voff_a[i], dst + i * (kWaves * 1024));
-#pragma unroll
-            for (int i = 0; i < kLB; i++) dma16_base(s_b + iss_k, voff_b[i], dst + (kLA + i) * (kWaves * 1024));
-#pragma unroll
-            for (int i = 0; i < kLB; i++) dma16_base(s_b2 + iss_k, voff_b[i], dst + (kLA + kLB + i) * (kWaves * 1024));
+        auto issue2_load = [&](int kt, int i) {
+            const unsigned dst = lds_base + (unsigned)(kt % kStages) * kStageBytes + (unsigned)wave * 1024 + i * (kWaves * 1024);
+            if (i < kLA) dma16_base(s_a + iss_k, voff_a[i], dst);
+            else if (i < kLA + kLB) dma16_base(s_b + iss_k, voff_b[i - kLA], dst);
+            else dma16_base(s_b2 + iss_k, voff_b[i - kLA - kLB], dst);
+        };
+        auto issue2_done = [&](int kt) {
             if (kt + 1 < n_kt) iss_k += kBK; // past the end the last tile is loaded again (keeps the in-flight count constant)
         };
         const int sw = (frow / kSwzDiv) % kCpr;
         const int xa = (wm * kWR + frow) * kRowBytes, xb = (kBM + wn * (32 * kNT) + frow) * kRowBytes;
         half8_t b0[kNT], b1[kNT];
-        auto read_a = [&](int set, const unsigned char *stage, int ks) {
+        auto read_a = [&](int set, const unsigned char *stage, int ks, int i) {
             const int c = ((ks * 2 + fch) ^ sw) << 4;
-#pragma unroll
-            for (int i = 0; i < kIT; i++) af[set][i] = *reinterpret_cast<const half8_t *>(stage + xa + i * (32 * kRowBytes) + c);
+            af[set][i] = *reinterpret_cast<const half8_t *>(stage + xa + i * (32 * kRowBytes) + c);
         };
-        auto read_b = [&](half8_t (&b)[kNT], const unsigned char *stage, int ks, int q) {
+        auto read_b = [&](half8_t (&b)[kNT], const unsigned char *stage, int ks, int q, int j) {
             const int c = ((ks * 2 + fch) ^ sw) << 4;
-#pragma unroll
-            for (int j = 0; j < kNT; j++) b[j] = *reinterpret_cast<const half8_t *>(stage + xb + (q * kBN + j * 32) * kRowBytes + c);
+            b[j] = *reinterpret_cast<const half8_t *>(stage + xb + (q * kBN + j * 32) * kRowBytes + c);
         };
+        constexpr int kSlots = kIT * kNT, kReads = kIT + kNT;  // per product and K-step
+        constexpr int kDmaSlots = (kKS - 1) * 2 * kSlots + kSlots; // up to the tile change
+        constexpr int kSpan = kDmaSlots < kDmaEvery * kLoads ? kDmaSlots : kDmaEvery * kLoads;
+        for (int t = 0; t < kStages; t++) {
 #pragma unroll
-        for (int t = 0; t < kStages; t++) issue2(t);
+            for (int i = 0; i < kLoads; i++) issue2_load(t, i);
+            issue2_done(t);
+        }
         wait_vmcnt<(kStages - 1) * kLoads>();
         __syncthreads();
-        read_a(0, lds_raw, 0);
-        read_b(b0, lds_raw, 0, 0);
+#pragma unroll
+        for (int i = 0; i < kIT; i++) read_a(0, lds_raw, 0, i);
+#pragma unroll
+        for (int j = 0; j < kNT; j++) read_b(b0, lds_raw, 0, 0, j);
         for (int kt = 0; kt < n_kt; kt++) {
             const unsigned char *stage = lds_raw + (kt % kStages) * kStageBytes;
+            const int kt_in = kt + kStages - 1; // the K-tile requested during this one, into the stage that the tile change before freed
+            auto dma_at = [&](auto atc) {
+                constexpr int at = decltype(atc)::value;
+                if constexpr (kSpread && at < kSpan) {
+                    constexpr int lo = at * kLoads / kSpan, hi = (at + 1) * kLoads / kSpan;
+                    if constexpr (hi > lo) {
+                        if (kt > 0) {
 #pragma unroll
-            for (int ks = 0; ks < kKS; ks++) {
-                const int cur = ks & 1, nxt = cur ^ 1;
-                read_b(b1, stage, ks, 1);
-#pragma unroll
-                for (int j = 0; j < kNT; j++)
-#pragma unroll
-                    for (int i = 0; i < kIT; i++) mma(af[cur][i], b0[j], acc[i][j]);
-#pragma unroll
-                for (int r = 0; r < kNT; r++) {
-                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0); // MFMA
-                    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0); // DS read
-                }
-                if constexpr (kIT * kNT - kNT > 0) __builtin_amdgcn_sched_group_barrier(0x008, kIT * kNT - kNT, 0);
-                if (ks + 1 < kKS) {
-                    read_a(nxt, stage, ks + 1);
-                    read_b(b0, stage, ks + 1, 0);
-#pragma unroll
-                    for (int j = 0; j < kNT; j++)
-#pragma unroll
-                        for (int i = 0; i < kIT; i++) mma(af[cur][i], b1[j], acc[i][kNT + j]);
-                    constexpr int kMmas2 = kIT * kNT, kReads2 = kIT + kNT, kPairs2 = kMmas2 < kReads2 ? kMmas2 : kReads2;
-#pragma unroll
-                    for (int r = 0; r < kPairs2; r++) {
-                        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                            for (int i = lo; i < hi; i++) issue2_load(kt_in, i);
+                            if constexpr (hi == kLoads) issue2_done(kt_in);
+                        }
                     }
-                    if constexpr (kMmas2 > kPairs2) __builtin_amdgcn_sched_group_barrier(0x008, kMmas2 - kPairs2, 0);
-                    if constexpr (kReads2 > kPairs2) __builtin_amdgcn_sched_group_barrier(0x100, kReads2 - kPairs2, 0);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            static_for<kKS>([&](auto ksc) {
+                constexpr int ks = decltype(ksc)::value, cur = ks & 1, nxt = cur ^ 1;
+                static_for<kSlots>([&](auto slc) {
+                    constexpr int sl = decltype(slc)::value;
+                    mma(af[cur][sl % kIT], b0[sl / kIT], acc[sl % kIT][sl / kIT]);
+                    if constexpr (sl < kNT) read_b(b1, stage, ks, 1, sl);
+                    dma_at(std::integral_constant<int, ks * 2 * kSlots + sl>{});
+                });
+                if constexpr (ks + 1 < kKS) {
+                    static_for<kSlots>([&](auto slc) {
+                        constexpr int sl = decltype(slc)::value;
+                        mma(af[cur][sl % kIT], b1[sl / kIT], acc[sl % kIT][kNT + sl / kIT]);
+                        if constexpr (sl < kIT) read_a(nxt, stage, ks + 1, sl);
+                        else if constexpr (sl < kReads) read_b(b0, stage, ks + 1, 0, sl - kIT);
+                        if constexpr (sl + 1 == kSlots && kReads > kSlots) {
+#pragma unroll
+                            for (int r = kSlots; r < kReads; r++) {
+                                if (r < kIT) read_a(nxt, stage, ks + 1, r);
+                                else read_b(b0, stage, ks + 1, 0, r - kIT);
+                            }
+                        }
+                        dma_at(std::integral_constant<int, (ks * 2 + 1) * kSlots + sl>{});
+                    });
                 } else {
-                    __builtin_amdgcn_sched_barrier(0);
                     wait_vmcnt<(kStages - 2) * kLoads>();
                     __syncthreads(); // K-tile kt + 1 is in LDS for everybody, and nobody reads K-tile kt any more
-                    issue2(kt + kStages);
+                    if constexpr (!kSpread) {
+#pragma unroll
+                        for (int i = 0; i < kLoads; i++) issue2_load(kt + kStages, i);
+                        issue2_done(kt + kStages);
+                    }
                     const unsigned char *next = lds_raw + ((kt + 1) % kStages) * kStageBytes;
-                    read_a(nxt, next, 0);
-                    read_b(b0, next, 0, 0);
+#pragma unroll
+                    for (int i = 0; i < kIT; i++) read_a(nxt, next, 0, i);
+#pragma unroll
+                    for (int j = 0; j < kNT; j++) read_b(b0, next, 0, 0, j);
                     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                    for (int j = 0; j < kNT; j++)
-#pragma unroll
-                        for (int i = 0; i < kIT; i++) mma(af[cur][i], b1[j], acc[i][kNT + j]);
+                    for (int sl = 0; sl < kSlots; sl++) mma(af[cur][sl % kIT], b1[sl / kIT], acc[sl % kIT][kNT + sl / kIT]);
+                    __builtin_amdgcn_sched_barrier(0);
                 }
-            }
+            });
         }
     } else {
+        constexpr int kSlots = kIT * kNTs, kReads = kIT + kNTs; // fragment pairs and fragments of a K-step
+        constexpr int kDmaSlots = (kKS - 1) * kSlots;           // of the K-steps in front of the tile change
+        constexpr int kSpan = kDmaSlots < kDmaEvery * kLoadsMax ? kDmaSlots : kDmaEvery * kLoadsMax;
+        auto slot_mma = [&](int set, int sl) { mma(af[set][sl % kIT], bf[set][sl / kIT], acc[sl % kIT][sl / kIT]); };
+        for (int t = 0; t < kStages; t++) {
 #pragma unroll
-        for (int t = 0; t < kStages; t++) issue(t);
+            for (int i = 0; i < kLoadsMax; i++) issue_load(t, i);
+            issue_done(t);
+        }
         if (short_wave) wait_vmcnt<(kStages - 1) * kLoadsMin>();
         else wait_vmcnt<(kStages - 1) * kLoadsMax>();
         __syncthreads();
-        read_frags(0, lds_raw, 0);
+#pragma unroll
+        for (int r = 0; r < kReads; r++) read_frag(0, lds_raw, 0, r);
         for (int kt = 0; kt < n_kt; kt++) {
             const unsigned char *stage = lds_raw + (kt % kStages) * kStageBytes;
+            const int kt_in = kt + kStages - 1; // the K-tile requested during this one, into the stage that the tile change before freed
+            static_for<kKS>([&](auto ksc) {
+                constexpr int ks = decltype(ksc)::value, cur = ks & 1, nxt = cur ^ 1;
+                if constexpr (ks + 1 < kKS) {
+                    static_for<kSlots>([&](auto slc) {
+                        constexpr int sl = decltype(slc)::value, at = ks * kSlots + sl;
+                        slot_mma(cur, sl);
+                        if constexpr (sl < kReads) read_frag(nxt, stage, ks + 1, sl);
+                        if constexpr (sl + 1 == kSlots && kReads > kSlots) {
 #pragma unroll
-            for (int ks = 0; ks < kKS; ks++) {
-                const int cur = ks & 1, nxt = cur ^ 1;
-                if (ks + 1 < kKS) {
-                    read_frags(nxt, stage, ks + 1);
-#pragma unroll
-                    for (int j = 0; j < kNTs; j++)
-#pragma unroll
-                        for (int i = 0; i < kIT; i++) mma(af[cur][i], bf[cur][j], acc[i][j]);
-                    {   // order within the step: an LDS fragment read of the next step behind each of the first MFMAs of this one,
-                        // so that the reads are in flight under the matrix pipe and none is left to wait for when the next step
-                        // begins (left to itself the scheduler issues the reads at the end of the step and the MFMAs wait for them)
-                        constexpr int kPerMma = kF32 ? 4 : 1; // MFMA instructions per fragment pair
-                        constexpr int kMmas = kIT * kNTs, kReads = kIT + kNTs, kPairs = kMmas < kReads ? kMmas : kReads;
-#pragma unroll
-                        for (int r = 0; r < kPairs; r++) {
-                            __builtin_amdgcn_sched_group_barrier(0x008, kPerMma, 0); // MFMA
-                            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);       // DS read
+                            for (int r = kSlots; r < kReads; r++) read_frag(nxt, stage, ks + 1, r);
                         }
-                        if constexpr (kMmas > kPairs) __builtin_amdgcn_sched_group_barrier(0x008, (kMmas - kPairs) * kPerMma, 0);
-                        if constexpr (kReads > kPairs) __builtin_amdgcn_sched_group_barrier(0x100, kReads - kPairs, 0);
-                    }
+                        if constexpr (kSpread && at < kSpan) {
+                            constexpr int lo = at * kLoadsMax / kSpan, hi = (at + 1) * kLoadsMax / kSpan;
+                            if constexpr (hi > lo) {
+                                if (kt > 0) {
+#pragma unroll
+                                    for (int i = lo; i < hi; i++) issue_load(kt_in, i);
+                                    if constexpr (hi == kLoadsMax) issue_done(kt_in);
+                                }
+                            }
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
+                    });
                 } else {
 #pragma unroll
-                    for (int j = 0; j < kSplitJ; j++)
-#pragma unroll
-                        for (int i = 0; i < kIT; i++) mma(af[cur][i], bf[cur][j], acc[i][j]);
+                    for (int sl = 0; sl < kSplitJ * kIT; sl++) slot_mma(cur, sl);
                     __builtin_amdgcn_sched_barrier(0);
                     if (short_wave) wait_vmcnt<(kStages - 2) * kLoadsMin>();
                     else wait_vmcnt<(kStages - 2) * kLoadsMax>();
                     __syncthreads(); // K-tile kt + 1 is in LDS for everybody, and nobody reads K-tile kt any more
-                    issue(kt + kStages);
-                    read_frags(nxt, lds_raw + ((kt + 1) % kStages) * kStageBytes, 0);
+                    if constexpr (!kSpread) {
+#pragma unroll
+                        for (int i = 0; i < kLoadsMax; i++) issue_load(kt + kStages, i);
+                        issue_done(kt + kStages);
+                    }
+                    const unsigned char *next = lds_raw + ((kt + 1) % kStages) * kStageBytes;
+#pragma unroll
+                    for (int r = 0; r < kReads; r++) read_frag(nxt, next, 0, r);
                     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                    for (int j = kSplitJ; j < kNTs; j++)
-#pragma unroll
-                        for (int i = 0; i < kIT; i++) mma(af[cur][i], bf[cur][j], acc[i][j]);
+                    for (int sl = kSplitJ * kIT; sl < kSlots; sl++) slot_mma(cur, sl);
+                    __builtin_amdgcn_sched_barrier(0);
                 }
-            }
+            });
         }
     }
     wait_vmcnt<0>(); // drain the clamped tail loads before the block's LDS is released
