@@ -17,7 +17,7 @@ CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "_obj")
 LIB = os.path.join(HERE, "librllama_hip.so")
 
-SOURCES = ["gemv.hip", "attention.hip", "gemm.hip", "gemm_dma.hip", "gemm_kgroup.hip", "gemm_split3.hip", "gemm_skinny.hip", "gemm_rows.hip", "gemm_rows_fused.hip", "attn_prefill.hip", "prefill.hip", "prefill_f32.hip", "misc.hip", "sampler.hip", "api.hip", "api_ops.hip"]
+SOURCES = ["gemv.hip", "attention.hip", "gemm.hip", "gemm_dma.hip", "gemm_kgroup.hip", "gemm_split3.hip", "gemm_skinny.hip", "gemm_rows.hip", "gemm_rows_fused.hip", "gemm_rows_f32.hip", "attn_prefill.hip", "prefill.hip", "prefill_f32.hip", "misc.hip", "sampler.hip", "api.hip", "api_ops.hip"]
 HEADERS = ["kernels.h", "device_utils.h", "gemv_device.h", "gemm_epilogue.h", "gemm_rows_device.h", "split3_plan.h", "tensor_pool.h", "synth.h", "api_internal.h", os.path.join("..", "..", "include", "rllama_hip.h")]  # relative to csrc/
 
 HIPCC = os.environ.get("HIPCC") or shutil.which("hipcc") or "/opt/rocm/bin/hipcc"

@@ -1270,9 +1270,30 @@ static int enqueue_prefill_f32(rlh_model *m, rlh_caches *c, const int32_t *token
         }
         if ((rc = gemm(att, d, L.wo.p, d, S.x, d, n, d, d, 1)) != RLH_OK) return rc;     // x += wo(att)   (transformer.rs:442)
         HIP_TRY(launch_rmsnorm_rows_f32(xn, S.x, (const float *)L.ffn_norm.p, n, d, eps, st));
-        if ((rc = gemm(xn, d, L.w1.p, d, gg, F, n, F, d, 0)) != RLH_OK) return rc;
-        if ((rc = gemm(xn, d, L.w3.p, d, uu, F, n, F, d, 0)) != RLH_OK) return rc;
-        HIP_TRY(launch_silu_mul_f32(gg, uu, mm, (size_t)n * F, st));
+        {
+            GemmParams g{};
+            g.tune = m->ctx->tun.gemm;
+            g.compute_units = m->ctx->prop.multiProcessorCount;
+            g.a = (const _Float16 *)xn;
+            g.b = (const _Float16 *)L.w1.p;
+            g.b2 = (const _Float16 *)L.w3.p;
+            g.c = mm;
+            g.m = n;
+            g.n = F;
+            g.k = g.lda = g.ldb = d;
+            g.ldc = F;
+            g.batch = 1;
+            g.f32_operands = 1;
+            g.workspace = S.gemm_ws;
+            g.workspace_bytes = S.gemm_ws_bytes;
+            if (gemm_f32_rows_pieces(g, kGemmEpiSiluGateF32) > 0) { // both products and SiLU * gate in one launch
+                HIP_TRY(launch_gemm_f32_rows(g, kGemmEpiSiluGateF32, st));
+            } else {
+                if ((rc = gemm(xn, d, L.w1.p, d, gg, F, n, F, d, 0)) != RLH_OK) return rc;
+                if ((rc = gemm(xn, d, L.w3.p, d, uu, F, n, F, d, 0)) != RLH_OK) return rc;
+                HIP_TRY(launch_silu_mul_f32(gg, uu, mm, (size_t)n * F, st));
+            }
+        }
         if ((rc = gemm(mm, F, L.w2.p, F, S.x, d, n, d, F, 1)) != RLH_OK) return rc;      // x += w2(...)   (transformer.rs:445)
     }
     if (span) {

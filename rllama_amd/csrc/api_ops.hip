@@ -226,7 +226,7 @@ extern "C" int rlh_matrix_mul_inplace_transposed(rlh_tensor *dst, const rlh_tens
         g.ldb = k;
         g.ldc = mrows;
         g.batch = 1;
-        g.f32_operands = f16 ? 0 : 1;
+        g.f32_operands = g.keep_order = f16 ? 0 : 1;
         OpScratch &o = dst->ctx->ops;
         HIP_TRY(gemm_work_reserve(dst->ctx, &o.gemm_ws, &o.gemm_ws_bytes, f16 ? 0 : split3_work_bytes(n, mrows, k)));
         g.workspace = o.gemm_ws;

@@ -132,6 +132,7 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_f16_kernel(GemmParams p) {
 hipError_t launch_gemm_f16(const GemmParams &p, int epilogue, hipStream_t s) {
     if (p.f32_operands) { // fp32 operands exist on the fast path only
         if (p.m <= 0 || p.n <= 0 || p.batch < 1 || !gemm_f16_dma_supported(p)) return hipErrorInvalidValue;
+        if (gemm_f32_rows_pieces(p, epilogue) > 0) return launch_gemm_f32_rows(p, epilogue, s);
         if (gemm_split3_supported(p, epilogue)) return launch_gemm_split3(p, s);
         return launch_gemm_f16_dma(p, epilogue, s);
     }

@@ -9,10 +9,8 @@ hipError_t launch_gemm_f16_rows_fused(const GemmParams &p, int epilogue, hipStre
 // Microseconds of a product in `pieces` pieces with what has to follow it: a launch, then what one compute unit stages at 45 GB/s or all of
 // the weights at 5.6 TB/s.  The kernel that adds the pieces brings the RMSNorm behind a residual product along.
 static double rows_us(const GemmParams &p, int epilogue, int pieces) {
-    long cost = 0;
-    rows_columns(p, pieces, &cost);
     const double k = ((p.k / 128 + pieces - 1) / pieces) * 128.0;
-    const double staged = k * 32.0 * (double)cost / 45e3, weights = 2.0 * p.n * (double)p.k * (p.b2 != nullptr ? 2 : 1) / 5.6e6;
+    const double staged = k / 1024 * rows_us_k(p, pieces, rows_columns(p, pieces)), weights = 2.0 * p.n * (double)p.k * (p.b2 != nullptr ? 2 : 1) / 5.6e6;
     double us = 3.0 + (staged > weights ? staged : weights);
     if (pieces > 1) us += 4.0 + 4.0 * pieces * (double)p.m * p.n / 4.7e6;
     if (epilogue == kGemmEpiResAddF32 && p.norm_w != nullptr) us += pieces > 1 ? 1.2 : 4.5;

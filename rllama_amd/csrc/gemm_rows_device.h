@@ -26,14 +26,14 @@
 
 namespace rlh {
 
-constexpr int kRowsMax = 160;
+constexpr int kRowsMax = 160, kRowsF32Max = 96;
 
 // kMF x kNF: 16 x 16 fragments of a workgroup's tile (rows x columns of one product; kGemmEpiSiluGateF16 computes two products).
 // kBK: halves of K per unit; K-group g of the kBK / 32 takes K-step g of every unit.  kRH x kCH: wavefronts of one K-group, over rows
 // and columns (of both products).  kStages: units in LDS.
 template <int kEpi, int kMF, int kNF, int kBK, int kRH, int kCH, int kStages>
 struct RowsShape {
-    static constexpr bool kDual = kEpi == kGemmEpiSiluGateF16;
+    static constexpr bool kDual = kEpi == kGemmEpiSiluGateF16 || kEpi == kGemmEpiSiluGateF32;
     static constexpr int kP = kDual ? 2 : 1;
     static constexpr int kKG = kBK / 32, kWaves = kKG * kRH * kCH, kThreads = 64 * kWaves;
     static constexpr int kNFt = kNF * kP, kMFw = kMF / kRH, kNFw = kNFt / kCH;
@@ -48,7 +48,10 @@ struct RowsShape {
     static_assert(kBK == 64 || kBK == 128 || kBK == 256, "K-steps of 32 halves");
 };
 
-template <int kEpi, int kMF, int kNF, int kBK, int kRH, int kCH, int kStages>
+// kF32: the operands are fp32 (f32 mode).  Staging moves bytes and is the same with units of kBK / 2 floats; a 16-byte fragment then holds
+// four consecutive k of a row and feeds four v_mfma_f32_16x16x4_f32 (k slot of lane group l / 16 in the j-th of them: float j of the group's
+// chunk, for A and B alike).
+template <int kEpi, int kMF, int kNF, int kBK, int kRH, int kCH, int kStages, bool kF32 = false>
 __global__ __launch_bounds__(2 * kBK * kRH * kCH) void gemm_f16_rows_kernel(GemmParams p) {
     using S = RowsShape<kEpi, kMF, kNF, kBK, kRH, kCH, kStages>;
     constexpr bool kDual = S::kDual;
@@ -61,7 +64,8 @@ __global__ __launch_bounds__(2 * kBK * kRH * kCH) void gemm_f16_rows_kernel(Gemm
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int pos = wave % (kRH * kCH), g = wave / (kRH * kCH), rh = pos % kRH, ch = pos / kRH;
     const int bx = blockIdx.x, bn0 = bx * kBN;
-    const int M = p.m, N = p.n, K = p.k;
+    constexpr int kE = kF32 ? 2 : 1; // halves per element: k and k offsets below are in halves
+    const int M = p.m, N = p.n, K = p.k * kE;
     // split_k > 1: grid.z counts ranges of units of one product, C item z (stride_c apart) gets its partial sums (kGemmEpiF32 only)
     int u0 = 0, cnt = K / kBK;
     if (p.split_k > 1) {
@@ -84,11 +88,11 @@ __global__ __launch_bounds__(2 * kBK * kRH * kCH) void gemm_f16_rows_kernel(Gemm
         const int lc = (lane % kCpr) ^ swz(row2);
         if (r0 >= 16 * kNFt) {
             gbase[i] = p.a;
-            voff[i] = (unsigned)((min(row2 - 16 * kNFt, M - 1) * p.lda + lc * 8) * 2); // rows past the edge: a valid row, never stored
+            voff[i] = (unsigned)((min(row2 - 16 * kNFt, M - 1) * p.lda * kE + lc * 8) * 2); // rows past the edge: a valid row, never stored
         } else {
             const bool second = kDual && r0 >= kBN;
-            gbase[i] = (second ? p.b2 : p.b) + (size_t)bn0 * p.ldb;
-            voff[i] = (unsigned)((min(second ? row2 - kBN : row2, N - 1 - bn0) * p.ldb + lc * 8) * 2);
+            gbase[i] = (second ? p.b2 : p.b) + (size_t)bn0 * p.ldb * kE;
+            voff[i] = (unsigned)((min(second ? row2 - kBN : row2, N - 1 - bn0) * p.ldb * kE + lc * 8) * 2);
         }
     }
     const unsigned lds_base = (unsigned)(uintptr_t)(__attribute__((address_space(3))) void *)lds_raw;
@@ -104,7 +108,11 @@ __global__ __launch_bounds__(2 * kBK * kRH * kCH) void gemm_f16_rows_kernel(Gemm
         if (++iss_slot == kStages) iss_slot = 0;
     };
 
+    // kF32: a unit's four MFMAs per fragment start from zero and are added to acc at its end, so that not all of K follows each other in
+    // one register: a block of 8 rows, 7B / 1024-dim shape, is 1.42e-6 / 4.8e-7 from float64 with one running
+    // sum and 6.0e-7 / 2.5e-7 like this (on the kernels for any number of rows 1.16e-6 / 3.3e-7).
     float4_t acc[kMFw][kNFw];
+    [[maybe_unused]] float4_t part[kF32 ? kMFw : 1][kF32 ? kNFw : 1] = {};
 #pragma unroll
     for (int i = 0; i < kMFw; i++)
 #pragma unroll
@@ -147,9 +155,17 @@ __global__ __launch_bounds__(2 * kBK * kRH * kCH) void gemm_f16_rows_kernel(Gemm
     __syncthreads();
 #pragma unroll
     for (int r = 0; r < kReads; r++) read_frag(std::integral_constant<int, 0>{}, lds_raw, r);
-    auto mma = [&](auto set, int sl) {
-        constexpr int s = decltype(set)::value;
-        acc[sl / kNFw][sl % kNFw] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fb[s][sl % kNFw], fa[s][sl / kNFw], acc[sl / kNFw][sl % kNFw], 0, 0, 0);
+    constexpr int kMmas = kF32 ? 4 * kSlots : kSlots; // of a unit; fp32: the first of every fragment pair, then the second of every pair, ...
+    auto mma = [&](auto set, auto index) {
+        constexpr int s = decltype(set)::value, x = decltype(index)::value, i = x % kSlots / kNFw, j = x % kNFw;
+        if constexpr (kF32) {
+            constexpr int e = x / kSlots;
+            const float4_t b4 = __builtin_bit_cast(float4_t, fb[s][j]), a4 = __builtin_bit_cast(float4_t, fa[s][i]);
+            if constexpr (e == 0) part[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(b4[e], a4[e], float4_t{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+            else part[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(b4[e], a4[e], part[i][j], 0, 0, 0);
+        } else {
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fb[s][j], fa[s][i], acc[i][j], 0, 0, 0);
+        }
     };
     // unit t: the fragments of unit t + 1 are read (kRead) and unit t + kStages is requested (kLoad) between its MFMAs
     auto step = [&](int t, auto set, auto rd, auto ld) {
@@ -162,21 +178,27 @@ __global__ __launch_bounds__(2 * kBK * kRH * kCH) void gemm_f16_rows_kernel(Gemm
             if (++slot == kStages) slot = 0;
         }
         const unsigned char *next = lds_raw + slot * kStageBytes;
-        static_for<kSlots>([&](auto slc) {
-            constexpr int sl = decltype(slc)::value;
-            if constexpr (kRead && sl < kReads) read_frag(std::integral_constant<int, s ^ 1>{}, next, sl);
-            if constexpr (kRead && sl == 0 && kReads > kSlots) {
+        static_for<kMmas>([&](auto index) {
+            constexpr int x = decltype(index)::value;
+            if constexpr (kRead && x < kReads) read_frag(std::integral_constant<int, s ^ 1>{}, next, x);
+            if constexpr (kRead && x == 0 && kReads > kMmas) {
 #pragma unroll
-                for (int r = kSlots; r < kReads; r++) read_frag(std::integral_constant<int, s ^ 1>{}, next, r);
+                for (int r = kMmas; r < kReads; r++) read_frag(std::integral_constant<int, s ^ 1>{}, next, r);
             }
-            mma(set, sl);
+            mma(set, index);
             if constexpr (kLoad) {
-                constexpr int lo = sl * kLMax / kSlots, hi = (sl + 1) * kLMax / kSlots;
+                constexpr int lo = x * kLMax / kMmas, hi = (x + 1) * kLMax / kMmas;
 #pragma unroll
                 for (int i = lo; i < hi; i++) issue_load(i);
             }
             __builtin_amdgcn_sched_barrier(0);
         });
+        if constexpr (kF32) {
+#pragma unroll
+            for (int i = 0; i < kMFw; i++)
+#pragma unroll
+                for (int j = 0; j < kNFw; j++) acc[i][j] += part[i][j];
+        }
         if constexpr (kLoad) issue_done();
     };
     constexpr std::integral_constant<int, 0> even{};
@@ -197,39 +219,73 @@ __global__ __launch_bounds__(2 * kBK * kRH * kCH) void gemm_f16_rows_kernel(Gemm
         else { step(t + 1, odd, no, no); break; }
     }
 
-    // ---- the K-groups' partial sums: fragment f of a position goes to K-group f % kKG, which adds them in the order of the groups
-    constexpr int kF = kMFw * kNFw, kOwn = (kF + kKG - 1) / kKG;
-    constexpr int kRoundMax = S::kLds / 1024 / kWaves / kKG * kKG;
-    static_assert(kKG == 1 || kRoundMax >= kKG, "a round of partial sums fits the stages");
-    constexpr int kRound = kRoundMax < kF ? kRoundMax : (kF + kKG - 1) / kKG * kKG;
+    // ---- the K-groups' partial sums: every fragment of a position goes to one K-group, which adds them in the order of the groups.  (The
+    //      fragments of both products at one place go to the same group where the epilogue works on registers.)
+    constexpr int kF = kMFw * kNFw;
+    constexpr bool kPairs = kEpi == kGemmEpiSiluGateF32;
+    static_assert(!kPairs || kCH == 1, "both products in one wavefront");
+    constexpr int kOwn = kPairs ? (kF / 2 + kKG - 1) / kKG * 2 : (kF + kKG - 1) / kKG;
+    constexpr auto owner = [](int f) { return (kPairs ? f / kNFw * kNF + f % kNFw % kNF : f) % kKG; };
+    constexpr auto slot_of = [](int f) { return kPairs ? (f / kNFw * kNF + f % kNFw % kNF) / kKG * 2 + f % kNFw / kNF : f / kKG; };
+    auto row_of = [&](int f) { return (rh * kMFw + f / kNFw) * 16 + frow; };
+    auto col_of = [&](int f) { return bn0 + (ch * kNFw + f % kNFw % (kPairs ? kNF : kNFw)) * 16 + (lane >> 4) * 4; };
     float4_t out[kOwn];
-    float4_t *xbuf = reinterpret_cast<float4_t *>(lds_raw);
-#pragma unroll
-    for (int f0 = 0; f0 < kF; f0 += kRound) {
-        __syncthreads(); // the stages (or the round before) have been read
-#pragma unroll
-        for (int f = f0; f < (f0 + kRound < kF ? f0 + kRound : kF); f++)
-            if (f % kKG != g) xbuf[((pos * kKG + g) * kRound + (f - f0)) * 64 + lane] = acc[f / kNFw][f % kNFw];
-        __syncthreads();
-#pragma unroll
-        for (int f = f0; f < (f0 + kRound < kF ? f0 + kRound : kF); f++)
-            if (f % kKG == g) {
-                float4_t sum;
-#pragma unroll
-                for (int q = 0; q < kKG; q++) {
-                    const float4_t term = q == f % kKG ? acc[f / kNFw][f % kNFw] : xbuf[((pos * kKG + q) * kRound + (f - f0)) * 64 + lane];
-                    sum = q == 0 ? term : sum + term;
-                }
-                out[f / kKG] = sum;
+    [[maybe_unused]] float4_t prev[kF32 && kEpi == kGemmEpiF32 ? kOwn : 1]; // what the sums are added to, requested ahead of the exchange
+    if constexpr (kF32 && kEpi == kGemmEpiF32) {
+        static_for<kF>([&](auto fc) {
+            constexpr int f = decltype(fc)::value;
+            if (owner(f) == g) {
+                const bool in = p.accumulate && row_of(f) < M && col_of(f) < N;
+                prev[slot_of(f)] = in ? *reinterpret_cast<const float4_t *>(reinterpret_cast<const float *>(p.c) + (size_t)row_of(f) * p.ldc + col_of(f)) : float4_t{0, 0, 0, 0};
             }
+        });
     }
-    if constexpr (kEpi == kGemmEpiF32) {
-#pragma unroll
-        for (int f = 0; f < kF; f++)
-            if (f % kKG == g) {
-                const int r = (rh * kMFw + f / kNFw) * 16 + frow, c = bn0 + (ch * kNFw + f % kNFw) * 16 + (lane >> 4) * 4;
-                if (r < M && c < N) *reinterpret_cast<float4_t *>(reinterpret_cast<float *>(p.c) + (size_t)blockIdx.z * p.stride_c + (size_t)r * p.ldc + c) = out[f / kKG];
+    constexpr int kRoundMax = S::kLds / 1024 / kWaves;
+    static_assert(kRoundMax >= 1, "a round of partial sums fits the stages");
+    constexpr int kRound = kRoundMax < kF ? kRoundMax : kF;
+    float4_t *xbuf = reinterpret_cast<float4_t *>(lds_raw);
+    static_for<(kF + kRound - 1) / kRound>([&](auto round) {
+        constexpr int f0 = decltype(round)::value * kRound, n_f = kF - f0 < kRound ? kF - f0 : kRound;
+        __syncthreads(); // the stages (or the round before) have been read
+        static_for<n_f>([&](auto fc) {
+            constexpr int i = decltype(fc)::value, f = f0 + i;
+            if (owner(f) != g) xbuf[((pos * kKG + g) * kRound + i) * 64 + lane] = acc[f / kNFw][f % kNFw];
+        });
+        __syncthreads();
+        static_for<n_f>([&](auto fc) {
+            constexpr int i = decltype(fc)::value, f = f0 + i;
+            if (owner(f) == g) {
+                float4_t sum;
+                static_for<kKG>([&](auto qc) {
+                    constexpr int q = decltype(qc)::value;
+                    float4_t term;
+                    if constexpr (q == owner(f)) term = acc[f / kNFw][f % kNFw];
+                    else term = xbuf[((pos * kKG + q) * kRound + i) * 64 + lane];
+                    if constexpr (q == 0) sum = term;
+                    else sum = sum + term;
+                });
+                out[slot_of(f)] = sum;
             }
+        });
+    });
+    if constexpr (kEpi == kGemmEpiF32 || kEpi == kGemmEpiSiluGateF32) {
+        static_for<kF>([&](auto fc) {
+            constexpr int f = decltype(fc)::value;
+            if constexpr (!kPairs || f % kNFw < kNF) {
+                if (owner(f) == g && row_of(f) < M && col_of(f) < N) {
+                    float4_t o = out[slot_of(f)];
+                    if constexpr (kPairs) {
+                        const float4_t u = out[slot_of(f) + 1];
+#pragma unroll
+                        for (int e = 0; e < 4; e++) o[e] = (o[e] / (1.0f + expf(-o[e]))) * u[e]; // transformer.rs:557-565; tensor.rs:822-832, 722-734
+                    }
+                    if constexpr (kF32 && kEpi == kGemmEpiF32) {
+                        if (p.accumulate) o = prev[slot_of(f)] + o;
+                    }
+                    *reinterpret_cast<float4_t *>(reinterpret_cast<float *>(p.c) + (size_t)blockIdx.z * p.stride_c + (size_t)row_of(f) * p.ldc + col_of(f)) = o;
+                }
+            }
+        });
         return;
     } else {
         constexpr int kTW = 16 * kNFt, kTS = kTW + 8;
@@ -238,12 +294,12 @@ __global__ __launch_bounds__(2 * kBK * kRH * kCH) void gemm_f16_rows_kernel(Gemm
         __syncthreads();
 #pragma unroll
         for (int f = 0; f < kF; f++)
-            if (f % kKG == g) {
+            if (owner(f) == g) {
                 typedef __attribute__((ext_vector_type(4))) _Float16 half4_t;
                 half4_t o;
 #pragma unroll
-                for (int e = 0; e < 4; e++) o[e] = (half_t)out[f / kKG][e]; // tensor.rs:1623-1643
-                const int rr = (rh * kMFw + f / kNFw) * 16 + frow;
+                for (int e = 0; e < 4; e++) o[e] = (half_t)out[slot_of(f)][e]; // tensor.rs:1623-1643
+                const int rr = row_of(f);
                 if (rr >= M) o = half4_t{0, 0, 0, 0}; // (the padding of V^T has to be finite)
                 *reinterpret_cast<half4_t *>(tile + rr * kTS + (ch * kNFw + f % kNFw) * 16 + (lane >> 4) * 4) = o;
             }
@@ -285,60 +341,66 @@ __global__ __launch_bounds__(2 * kBK * kRH * kCH) void gemm_f16_rows_kernel(Gemm
     }
 }
 
-inline int rows_fragments(int m) { return (m + 15) / 16; }
+inline int rows_fragments(const GemmParams &p) { return p.f32_operands && p.m > 64 ? 6 : (p.m + 15) / 16; }
 
-// Columns per workgroup: the number of 16-column fragments with the least (rounds of workgroups) x (bytes a workgroup stages per value of k).
-inline int rows_columns(const GemmParams &p, int pieces, long *cost_out = nullptr) {
-    const int mf = rows_fragments(p.m), products = p.b2 != nullptr ? 2 : 1;
+// Microseconds per 1024 values of k that the workgroups of a product of `pieces` pieces take on nf x 16 columns each: rounds of
+// workgroups x what a compute unit stages at 45 GB/s, or (fp32) what its matrix cores take at 0.45 TFLOP/s, whichever is longer.
+inline double rows_us_k(const GemmParams &p, int pieces, int nf) {
+    const int mf = rows_fragments(p), cols = nf * (p.b2 != nullptr ? 2 : 1);
+    const long blocks = (long)((p.n + 16 * nf - 1) / (16 * nf)) * pieces, rounds = (blocks + p.compute_units - 1) / p.compute_units;
+    const double staged = (mf + cols) * 16 * 1024.0 * (p.f32_operands ? 4 : 2) / 45e3;
+    const double mfma = p.f32_operands ? 2.0 * 256 * mf * cols * 1024 / 0.45e6 : 0.0;
+    return rounds * (staged > mfma ? staged : mfma);
+}
+
+// 16-column fragments per workgroup: the number that takes least (two fp32 products of many rows: as many as the registers hold).
+inline int rows_columns(const GemmParams &p, int pieces) {
+    const int most = p.f32_operands && p.b2 != nullptr ? (p.m > 64 ? 2 : p.m > 48 ? 3 : 4) : 4;
     int best = 1;
-    long best_cost = 0;
-    for (int nf = 1; nf <= 4; nf++) {
-        const long blocks = (long)((p.n + 16 * nf - 1) / (16 * nf)) * pieces;
-        const long cost = (blocks + p.compute_units - 1) / p.compute_units * (mf + nf * products);
-        if (nf == 1 || cost < best_cost) {
-            best = nf;
-            best_cost = cost;
-        }
-    }
-    if (cost_out != nullptr) *cost_out = best_cost;
+    for (int nf = 2; nf <= most; nf++)
+        if (rows_us_k(p, pieces, nf) < rows_us_k(p, pieces, best)) best = nf;
     return best;
 }
 
-template <int kEpi, int kMF, int kNF, int kBKFixed = 0>
+template <int kEpi, int kMF, int kNF, bool kF32, int kBKFixed = 0>
 hipError_t launch_rows(const GemmParams &p, hipStream_t s) {
     // Units of 128 halves (whole 256-byte pieces of rows) while at least three fit the LDS, else of 64.  One fragment of rows and few
     // columns: 80 KB, so that two workgroups share a compute unit, and for long rows units of 256, i.e. twice the wavefronts (8 rows,
     // 4096 x 4096: 9.1 us with units of 128, 10.8 with 256; 4096 x 11008: 19.7 and 17.2).
-    if constexpr (kMF == 1 && kNF <= 2 && kBKFixed == 0 && kEpi != kGemmEpiSiluGateF16) {
-        if (p.k >= 6144 && p.k % 256 == 0) return launch_rows<kEpi, kMF, kNF, 256>(p, s);
+    if constexpr (kMF == 1 && kNF <= 2 && kBKFixed == 0 && !kF32 && kEpi != kGemmEpiSiluGateF16) {
+        if (p.k >= 6144 && p.k % 256 == 0) return launch_rows<kEpi, kMF, kNF, kF32, 256>(p, s);
     }
-    constexpr int kFrags = kMF + kNF * (kEpi == kGemmEpiSiluGateF16 ? 2 : 1);
+    constexpr int kFrags = kMF + kNF * (kEpi == kGemmEpiSiluGateF16 || kEpi == kGemmEpiSiluGateF32 ? 2 : 1);
     constexpr int kBK = kBKFixed > 0 ? kBKFixed : kFrags <= 13 ? 128 : 64;
     constexpr int kFit = (kMF == 1 && kFrags <= 5 ? 80 : 160) * 32 / (kFrags * kBK); // units of kFrags * 32 * kBK bytes
     constexpr int kStages = kFit > 8 ? 8 : kFit > 6 && kMF > 1 ? 6 : kFit;
-    constexpr int kCH = kEpi == kGemmEpiSiluGateF16 || kBK == 64 ? 2 : 1;
+    constexpr int kCH = kEpi == kGemmEpiSiluGateF16 || (kBK == 64 && kEpi != kGemmEpiSiluGateF32) ? 2 : 1;
     constexpr int kRH = kMF % 2 == 0 && (kBK == 64 || (kMF >= 4 && kCH == 1)) ? 2 : 1;
     using S = RowsShape<kEpi, kMF, kNF, kBK, kRH, kCH, kStages>;
-    const auto kern = gemm_f16_rows_kernel<kEpi, kMF, kNF, kBK, kRH, kCH, kStages>;
+    const auto kern = gemm_f16_rows_kernel<kEpi, kMF, kNF, kBK, kRH, kCH, kStages, kF32>;
     static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, S::kLds);
     if (attr != hipSuccess) return attr;
     hipLaunchKernelGGL(kern, dim3((p.n + 16 * kNF - 1) / (16 * kNF), 1, p.split_k > 1 ? p.split_k : 1), dim3(S::kThreads), S::kLds, s, p);
     return hipGetLastError();
 }
 
-template <int kEpi, int kMF>
+template <int kEpi, int kMF, bool kF32 = false>
 hipError_t launch_rows_mf(const GemmParams &p, hipStream_t s) {
     switch (rows_columns(p, p.split_k > 1 ? p.split_k : 1)) {
-    case 1: return launch_rows<kEpi, kMF, 1>(p, s);
-    case 2: return launch_rows<kEpi, kMF, 2>(p, s);
-    case 3: return launch_rows<kEpi, kMF, 3>(p, s);
-    default: return launch_rows<kEpi, kMF, 4>(p, s);
+    case 1: return launch_rows<kEpi, kMF, 1, kF32>(p, s);
+    case 2: return launch_rows<kEpi, kMF, 2, kF32>(p, s);
+    case 3:
+        if constexpr (kEpi != kGemmEpiSiluGateF32 || kMF <= 4) return launch_rows<kEpi, kMF, 3, kF32>(p, s);
+        return hipErrorInvalidValue;
+    default:
+        if constexpr (kEpi != kGemmEpiSiluGateF32 || kMF <= 3) return launch_rows<kEpi, kMF, 4, kF32>(p, s);
+        return hipErrorInvalidValue;
     }
 }
 
 template <int kEpi>
 hipError_t launch_rows_epi(const GemmParams &p, hipStream_t s) {
-    switch (rows_fragments(p.m)) {
+    switch (rows_fragments(p)) {
     case 1: return launch_rows_mf<kEpi, 1>(p, s);
     case 2: return launch_rows_mf<kEpi, 2>(p, s);
     case 3: return launch_rows_mf<kEpi, 3>(p, s);

@@ -119,6 +119,7 @@ enum GemmEpilogue {
     kGemmEpiF32 = 1,        // C f32 = acc, or += acc when accumulate  (attention scores / P.V partial products)
     kGemmEpiResAddF32 = 2,  // C f32 = residual + f16r(acc)            (wo and w2 followed by transformer.rs:442 / :445)
     kGemmEpiSiluGateF16 = 3, // C f16 = round(silu(gate) * f16r(acc))  (w3 with w1's f16 output as the gate: transformer.rs:557-565)
+    kGemmEpiSiluGateF32 = 5, // fp32 operands, b2, at most kRowsF32Max rows: C f32 = silu(a * b^T) * (a * b2^T) (transformer.rs:557-565, no rounding point)
     kGemmEpiRopeQkv = 4     // fast path only: the f16-rounded [m x 3 dim] product of wq|wk|wv is not stored; RoPE on its q and k
                             // columns, q as hi + lo halves, k and v into the cache, v transposed (GemmParams::rope; what
                             // rope_kv_prefill_tiled_kernel does with the stored product: transformer.rs:704-761)
@@ -177,8 +178,8 @@ struct GemmParams {
     _Float16 *norm_out;     // [m x n], row stride n
     float norm_eps;
     int *norm_done;         // host flag
-    int keep_order;         // 1 (rlh_ffn_gate): beyond 16 rows only kernels that add in the order of gemm_dma.hip's, so that one pass and
-                            // two launches give the same bits
+    int keep_order;         // 1 (op-level fp32 products; rlh_ffn_gate beyond 16 rows): none of the kernels of gemm_rows_device.h, so that a fp32
+                            // product has the bits of one of the two ways that GEMM_SPLIT3 names, and one pass those of two launches
     GemmTune tune;          // the context's switches (zero = defaults)
     PrefillRopeParams rope; // kGemmEpiRopeQkv: the destinations (qkv unused; n = m, 3 dim = n, f16 cache, vt_swap as the reader expects)
 };
@@ -202,6 +203,9 @@ int gemm_f16_rows_pieces(const GemmParams &p, int epilogue);
 // whether w1 and w3 are better as two products, each cut along K, than in one pass (gemm_dma.hip)
 bool gemm_f16_gate_cut(const GemmParams &p);
 hipError_t launch_gemm_f16_rows(const GemmParams &p, int epilogue, hipStream_t s); // p: one that gemm_f16_rows_pieces takes, or its pieces
+// the same for fp32 operands (gemm_rows_f32.hip); 0: the product is for the other kernels
+int gemm_f32_rows_pieces(const GemmParams &p, int epilogue);
+hipError_t launch_gemm_f32_rows(const GemmParams &p, int epilogue, hipStream_t s); // p: one that gemm_f32_rows_pieces takes; cuts it and adds the pieces itself
 // fp32 operands as three bf16 parts each (gemm_split3.hip): launch_gemm_f16 picks it for unbatched fp32 products with work memory where it is faster than the fp32 instruction
 bool gemm_split3_supported(const GemmParams &p, int epilogue);
 hipError_t launch_gemm_split3(const GemmParams &p, hipStream_t s); // p: one that gemm_split3_supported takes

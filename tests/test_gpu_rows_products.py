@@ -1,9 +1,10 @@
-"""f16 products of at most 160 rows on the kernel whose wavefronts split K: plain, cut along K, w1 and w3 in one pass, and inside prompts."""
+"""Products of at most 160 (f16) or 96 (fp32) rows on the kernel whose wavefronts split K: plain, cut along K, w1 and w3 in one pass, and inside
+prompts of both modes."""
 import numpy as np
 import pytest
 
 import rllama_amd
-from common import Shape, make_gpu, make_oracle, max_rel_err, options, synth_weights
+from common import Shape, make_gpu, make_oracle, max_rel_err, options, random_f32_weights, synth_weights
 from rllama_amd import Tensor
 from test_gpu_short_products import TOL_F16, _check, _check_gate, _f16
 
@@ -59,4 +60,21 @@ def test_prompts(ctx, dim, heads, ffn):
         gc, oc = gm.make_caches(), om.make_caches()
         assert max_rel_err(gm.forward(toks[:n], 0, gc), om.forward(toks[:n], 0, oc)) < TOL_F16, n
         assert max_rel_err(gm.forward(toks[n:n + 1], n, gc), om.forward(toks[n:n + 1], n, oc)) < TOL_F16, n
+    gm.free()
+
+
+# f32 mode: no rounding points, so only the order of sums differs.  K of an odd number of units of 64 floats, fewer units than stages, pieces along K
+# (ffn 6144), column counts that leave a remainder, both products of w1 and w3 on one to four fragments of columns; up to 96 rows and beyond
+@pytest.mark.parametrize("dim,heads,ffn", [(64, 2, 192), (192, 3, 520), (1024, 16, 2816), (1088, 17, 2048), (2048, 32, 6144)])
+def test_prompts_in_f32_mode(ctx, dim, heads, ffn):
+    shape = Shape(dim=dim, n_layers=2, n_heads=heads, ffn_hidden=ffn // 32 * 32, vocab_size=64, max_seq_len=112)
+    W = random_f32_weights(shape, seed=63, std=0.7 / dim ** 0.5)
+    toks = np.random.default_rng(64).integers(0, shape.vocab_size, 112)
+    om, gm = make_oracle(shape, W, False), make_gpu(ctx, shape, W, False)
+    for n in (2, 16, 17, 33, 48, 49, 64, 65, 96, 97):
+        gm.forward(toks, 0, gm.make_caches())  # leaves other rows' values in the work buffers
+        gc, oc = gm.make_caches(), om.make_caches()
+        # (the oracle adds in another order too: a few 2^-24 times the square root of K per sum, 1e-6 of the largest logit measured)
+        assert max_rel_err(gm.forward(toks[:n], 0, gc), om.forward(toks[:n], 0, oc)) < 1e-5, n
+        assert max_rel_err(gm.forward(toks[n:n + 1], n, gc), om.forward(toks[n:n + 1], n, oc)) < 1e-5, n
     gm.free()
