@@ -204,7 +204,7 @@ __global__ __launch_bounds__(128 * kWavesM) void gemm_f16_dma_kernel(GemmParams 
     // the middle of the last K-step's MFMAs so that the barrier and the LDS latency behind it stay covered.
     // Where the loads of a K-tile are requested: a wavefront that requests them all at once at the tile change stands in the queue of the
     // memory path until the last is taken, its fragment reads and MFMAs behind it.  With four stages or more they are spread over the
-    // MFMAs instead, one per kDmaEvery fragment pairs (7B shape, 131 rows: wq|wk|wv on 128 x 64 44.4 -> 39.9 us, w1|w3 on 192 x 64 58.2 -> 54.4).
+    // MFMAs instead, one per kDmaEvery fragment pairs and in a fixed order (7B shape, 131 rows: wq|wk|wv on 128 x 64 44.4 -> 39.9 us, w1|w3 on 192 x 64 58.2 -> 54.4).
     // With two or three, K-tile t + 1 has to arrive while K-tile t is consumed, and what counts is that it is requested early (256 x 192, 7B
     // wq|wk|wv of 1024 rows 107 us at once, 114 - 117 spread).
     constexpr bool kSpread = kStages >= 4;
@@ -291,7 +291,7 @@ __global__ __launch_bounds__(128 * kWavesM) void gemm_f16_dma_kernel(GemmParams 
             const int kt_in = kt + kStages - 1; // the K-tile requested during this one, into the stage that the tile change before freed
             auto dma_at = [&](auto atc) {
                 constexpr int at = decltype(atc)::value;
-                if constexpr (kSpread && at < kSpan) {
+                if constexpr (at < kSpan) {
                     constexpr int lo = at * kLoads / kSpan, hi = (at + 1) * kLoads / kSpan;
                     if constexpr (hi > lo) {
                         if (kt > 0) {
@@ -305,13 +305,26 @@ __global__ __launch_bounds__(128 * kWavesM) void gemm_f16_dma_kernel(GemmParams 
             };
             static_for<kKS>([&](auto ksc) {
                 constexpr int ks = decltype(ksc)::value, cur = ks & 1, nxt = cur ^ 1;
-                static_for<kSlots>([&](auto slc) {
-                    constexpr int sl = decltype(slc)::value;
-                    mma(af[cur][sl % kIT], b0[sl / kIT], acc[sl % kIT][sl / kIT]);
-                    if constexpr (sl < kNT) read_b(b1, stage, ks, 1, sl);
-                    dma_at(std::integral_constant<int, ks * 2 * kSlots + sl>{});
-                });
-                if constexpr (ks + 1 < kKS) {
+                if constexpr (kSpread) {
+                    static_for<kSlots>([&](auto slc) {
+                        constexpr int sl = decltype(slc)::value;
+                        mma(af[cur][sl % kIT], b0[sl / kIT], acc[sl % kIT][sl / kIT]);
+                        if constexpr (sl < kNT) read_b(b1, stage, ks, 1, sl);
+                        dma_at(std::integral_constant<int, ks * 2 * kSlots + sl>{});
+                    });
+                } else {
+#pragma unroll
+                    for (int j = 0; j < kNT; j++) read_b(b1, stage, ks, 1, j);
+#pragma unroll
+                    for (int sl = 0; sl < kSlots; sl++) mma(af[cur][sl % kIT], b0[sl / kIT], acc[sl % kIT][sl / kIT]);
+#pragma unroll
+                    for (int r = 0; r < kNT; r++) {
+                        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0); // MFMA
+                        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0); // DS read
+                    }
+                    if constexpr (kSlots > kNT) __builtin_amdgcn_sched_group_barrier(0x008, kSlots - kNT, 0);
+                }
+                if constexpr (ks + 1 < kKS && kSpread) {
                     static_for<kSlots>([&](auto slc) {
                         constexpr int sl = decltype(slc)::value;
                         mma(af[cur][sl % kIT], b1[sl / kIT], acc[sl % kIT][kNT + sl / kIT]);
@@ -326,7 +339,23 @@ __global__ __launch_bounds__(128 * kWavesM) void gemm_f16_dma_kernel(GemmParams 
                         }
                         dma_at(std::integral_constant<int, (ks * 2 + 1) * kSlots + sl>{});
                     });
+                } else if constexpr (ks + 1 < kKS) {
+#pragma unroll
+                    for (int i = 0; i < kIT; i++) read_a(nxt, stage, ks + 1, i);
+#pragma unroll
+                    for (int j = 0; j < kNT; j++) read_b(b0, stage, ks + 1, 0, j);
+#pragma unroll
+                    for (int sl = 0; sl < kSlots; sl++) mma(af[cur][sl % kIT], b1[sl / kIT], acc[sl % kIT][kNT + sl / kIT]);
+                    constexpr int kPairs = kSlots < kReads ? kSlots : kReads;
+#pragma unroll
+                    for (int r = 0; r < kPairs; r++) {
+                        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                    }
+                    if constexpr (kSlots > kPairs) __builtin_amdgcn_sched_group_barrier(0x008, kSlots - kPairs, 0);
+                    if constexpr (kReads > kPairs) __builtin_amdgcn_sched_group_barrier(0x100, kReads - kPairs, 0);
                 } else {
+                    __builtin_amdgcn_sched_barrier(0);
                     wait_vmcnt<(kStages - 2) * kLoads>();
                     __syncthreads(); // K-tile kt + 1 is in LDS for everybody, and nobody reads K-tile kt any more
                     if constexpr (!kSpread) {
@@ -366,7 +395,7 @@ __global__ __launch_bounds__(128 * kWavesM) void gemm_f16_dma_kernel(GemmParams 
             const int kt_in = kt + kStages - 1; // the K-tile requested during this one, into the stage that the tile change before freed
             static_for<kKS>([&](auto ksc) {
                 constexpr int ks = decltype(ksc)::value, cur = ks & 1, nxt = cur ^ 1;
-                if constexpr (ks + 1 < kKS) {
+                if constexpr (ks + 1 < kKS && kSpread) {
                     static_for<kSlots>([&](auto slc) {
                         constexpr int sl = decltype(slc)::value, at = ks * kSlots + sl;
                         slot_mma(cur, sl);
@@ -375,7 +404,7 @@ __global__ __launch_bounds__(128 * kWavesM) void gemm_f16_dma_kernel(GemmParams 
 #pragma unroll
                             for (int r = kSlots; r < kReads; r++) read_frag(nxt, stage, ks + 1, r);
                         }
-                        if constexpr (kSpread && at < kSpan) {
+                        if constexpr (at < kSpan) {
                             constexpr int lo = at * kLoadsMax / kSpan, hi = (at + 1) * kLoadsMax / kSpan;
                             if constexpr (hi > lo) {
                                 if (kt > 0) {
@@ -387,6 +416,22 @@ __global__ __launch_bounds__(128 * kWavesM) void gemm_f16_dma_kernel(GemmParams 
                         }
                         __builtin_amdgcn_sched_barrier(0);
                     });
+                } else if constexpr (ks + 1 < kKS) {
+#pragma unroll
+                    for (int r = 0; r < kReads; r++) read_frag(nxt, stage, ks + 1, r);
+#pragma unroll
+                    for (int sl = 0; sl < kSlots; sl++) slot_mma(cur, sl);
+                    // an LDS fragment read of the next step behind each of the first MFMAs of this one, so that the reads are in flight under
+                    // the matrix pipe (left to itself the scheduler issues them at the end of the step and the MFMAs wait for them)
+                    constexpr int kPerMma = kF32 ? 4 : 1; // MFMA instructions per fragment pair
+                    constexpr int kPairs = kSlots < kReads ? kSlots : kReads;
+#pragma unroll
+                    for (int r = 0; r < kPairs; r++) {
+                        __builtin_amdgcn_sched_group_barrier(0x008, kPerMma, 0); // MFMA
+                        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);       // DS read
+                    }
+                    if constexpr (kSlots > kPairs) __builtin_amdgcn_sched_group_barrier(0x008, (kSlots - kPairs) * kPerMma, 0);
+                    if constexpr (kReads > kPairs) __builtin_amdgcn_sched_group_barrier(0x100, kReads - kPairs, 0);
                 } else {
 #pragma unroll
                     for (int sl = 0; sl < kSplitJ * kIT; sl++) slot_mma(cur, sl);

@@ -98,12 +98,12 @@ __global__ __launch_bounds__(64 * kWM * kWN * kKG) void gemm_f16_kgroup_kernel(G
     const half_t *s_a = p.a + (size_t)bm0 * p.lda + k_skip, *s_b = p.b + (size_t)bn0 * p.ldb + k_skip;
     const unsigned lds_base = (unsigned)(uintptr_t)(__attribute__((address_space(3))) void *)lds_raw;
     int iss_k = 0;
-    auto issue_load = [&](int kt, int i) { // load i of K-tile kt; the loads of kt = 0, 1, 2, ... in this order, issue_done behind each
-        const unsigned dst = lds_base + (unsigned)(kt % kStages) * kStageBytes + (unsigned)wave * 1024 + i * (kWaves * 1024);
-        if (i < kLA) dma16_base(s_a + iss_k, voff_a[i], dst);
-        else dma16_base(s_b + iss_k, voff_b[i - kLA], dst);
-    };
-    auto issue_done = [&](int kt) {
+    auto issue = [&](int kt) { // called for kt = 0, 1, 2, ... in this order
+        const unsigned dst = lds_base + (unsigned)(kt % kStages) * kStageBytes + (unsigned)wave * 1024;
+#pragma unroll
+        for (int i = 0; i < kLA; i++) dma16_base(s_a + iss_k, voff_a[i], dst + i * (kWaves * 1024));
+#pragma unroll
+        for (int i = 0; i < kLB; i++) dma16_base(s_b + iss_k, voff_b[i], dst + (kLA + i) * (kWaves * 1024));
         if (kt + 1 < n_kt) iss_k += kBK; // past the end the last tile is loaded again (keeps the in-flight count constant)
     };
 
@@ -154,11 +154,7 @@ __global__ __launch_bounds__(64 * kWM * kWN * kKG) void gemm_f16_kgroup_kernel(G
     // sits in the middle of the wavefront's last K-step of the tile.  `parity` is the parity of the wavefront's K-step count
     // so far (compile time: the loop over K-tiles is unrolled by two).
 #pragma unroll
-    for (int t = 0; t < kStages; t++) {
-#pragma unroll
-        for (int i = 0; i < kLoads; i++) issue_load(t, i);
-        issue_done(t);
-    }
+    for (int t = 0; t < kStages; t++) issue(t);
     wait_vmcnt<(kStages - 1) * kLoads>();
     __syncthreads();
     read_frags(0, lds_raw, 0);
@@ -180,23 +176,14 @@ __global__ __launch_bounds__(64 * kWM * kWN * kKG) void gemm_f16_kgroup_kernel(G
                 }
                 __builtin_amdgcn_sched_group_barrier(0x008, kIT * kNT - (kIT + kNT), 0);
             } else {
-                // the loads of K-tile kt + kStages - 1, into the stage that the tile change before freed, one behind each of the first
-                // MFMAs (all at once behind the barrier, the fragment reads and MFMAs stand behind them in the queue)
-                constexpr int kFirst = kNT / 2 * kIT;
-                static_for<kFirst>([&](auto slc) {
-                    constexpr int sl = decltype(slc)::value, lo = sl * kLoads / kFirst, hi = (sl + 1) * kLoads / kFirst;
-                    mma(cur, sl % kIT, sl / kIT);
-                    if constexpr (hi > lo) {
-                        if (kt > 0) {
 #pragma unroll
-                            for (int i = lo; i < hi; i++) issue_load(kt + kStages - 1, i);
-                            if constexpr (hi == kLoads) issue_done(kt + kStages - 1);
-                        }
-                    }
-                    __builtin_amdgcn_sched_barrier(0);
-                });
+                for (int j = 0; j < kNT / 2; j++)
+#pragma unroll
+                    for (int i = 0; i < kIT; i++) mma(cur, i, j);
+                __builtin_amdgcn_sched_barrier(0);
                 wait_vmcnt<(kStages - 2) * kLoads>();
                 __syncthreads(); // K-tile kt + 1 is in LDS for everybody, and nobody reads K-tile kt any more
+                issue(kt + kStages);
                 read_frags(nxt, lds_raw + ((kt + 1) % kStages) * kStageBytes, 0);
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
