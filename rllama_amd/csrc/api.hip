@@ -254,6 +254,7 @@ extern "C" void rlh_shutdown(rlh_ctx *ctx) {
         ctx->stream = nullptr;
     }
     ops_release(ctx);
+    if (ctx->stage) (void)hipHostFree(ctx->stage);
     delete ctx;
 }
 
@@ -271,6 +272,41 @@ extern "C" int rlh_device_info(rlh_ctx *ctx, char *name, int cap, int *compute_u
     if (hbm_bytes) *hbm_bytes = (uint64_t)ctx->prop.totalGlobalMem;
     return RLH_OK;
 }
+
+// A copy to or from pageable memory goes through staging of the runtime's own, which it waits for; through memory of ours the copy is one
+// command of the stream and the wait at the end of the call is the only one.  With the upload of a single token gone (it is a kernel argument
+// anyway): decode step of dim 1024, 8 layers 238 -> 219 us (f32 mode 367 -> 313), 7B shape, 8 layers 715 -> 700; results of 630 KB to 2.4 MB
+// of op-level tensors 114 -> 112 and, above the staging, unchanged.  1 MiB: larger copies are no faster through it.
+namespace rlh {
+static bool stage_ready(rlh_ctx *ctx, size_t bytes) {
+    if (bytes > kStageBytes) return false;
+    if (ctx->stage == nullptr && hipHostMalloc((void **)&ctx->stage, 2 * kStageBytes, hipHostMallocDefault) != hipSuccess) {
+        ctx->stage = nullptr;
+        (void)hipGetLastError();
+    }
+    return ctx->stage != nullptr;
+}
+
+hipError_t stage_upload(rlh_ctx *ctx, void *dev, const void *host, size_t bytes) {
+    if (!stage_ready(ctx, bytes)) return hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, ctx->stream);
+    if (ctx->stage_busy) { // the call before ended without stage_download, maybe with an error
+        const hipError_t e = hipStreamSynchronize(ctx->stream);
+        if (e != hipSuccess) return e;
+    }
+    memcpy(ctx->stage, host, bytes);
+    ctx->stage_busy = true;
+    return hipMemcpyAsync(dev, ctx->stage, bytes, hipMemcpyHostToDevice, ctx->stream);
+}
+
+hipError_t stage_download(rlh_ctx *ctx, void *host, const void *dev, size_t bytes) {
+    const bool staged = stage_ready(ctx, bytes);
+    hipError_t e = hipMemcpyAsync(staged ? ctx->stage + kStageBytes : host, dev, bytes, hipMemcpyDeviceToHost, ctx->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
+    if (e == hipSuccess) ctx->stage_busy = false;
+    if (e == hipSuccess && staged) memcpy(host, ctx->stage + kStageBytes, bytes);
+    return e;
+}
+} // namespace rlh
 
 // ------------------------------------------------------------------------------------------------
 // model
@@ -958,7 +994,7 @@ static int enqueue_prefill(rlh_model *m, rlh_caches *c, const int32_t *tokens, i
     if (span) {
         HIP_TRY(hipMemcpyAsync(S.x, span->x_in, sizeof(float) * (size_t)n * d, hipMemcpyHostToDevice, st));
     } else {
-        HIP_TRY(hipMemcpyAsync(m->prompt_dev, tokens, sizeof(int32_t) * (size_t)n, hipMemcpyHostToDevice, st));
+        HIP_TRY(stage_upload(m->ctx, m->prompt_dev, tokens, sizeof(int32_t) * (size_t)n));
         HIP_TRY(launch_set_state(m->state, n - 1, tokens[n - 1], 1, st));
         HIP_TRY(launch_embed_rows(m->tok_emb.p, m->tok_emb.f16, m->prompt_dev, n, d, S.x, st));
     }
@@ -1177,7 +1213,7 @@ static int enqueue_prefill_f32(rlh_model *m, rlh_caches *c, const int32_t *token
     if (span) {
         HIP_TRY(hipMemcpyAsync(S.x, span->x_in, sizeof(float) * (size_t)n * d, hipMemcpyHostToDevice, st));
     } else {
-        HIP_TRY(hipMemcpyAsync(m->prompt_dev, tokens, sizeof(int32_t) * (size_t)n, hipMemcpyHostToDevice, st));
+        HIP_TRY(stage_upload(m->ctx, m->prompt_dev, tokens, sizeof(int32_t) * (size_t)n));
         HIP_TRY(launch_set_state(m->state, n - 1, tokens[n - 1], 1, st));
         HIP_TRY(launch_embed_rows(m->tok_emb.p, m->tok_emb.f16, m->prompt_dev, n, d, S.x, st));
     }
@@ -1347,7 +1383,7 @@ static int enqueue_forward(rlh_model *m, rlh_caches *c, const int32_t *tokens, i
         if (m->prm.force_f16) return enqueue_prefill(m, c, tokens, n);
         if (prefill_f32_supported(m)) return enqueue_prefill_f32(m, c, tokens, n);
     }
-    HIP_TRY(hipMemcpyAsync(m->prompt_dev, tokens, sizeof(int32_t) * (size_t)n, hipMemcpyHostToDevice, st));
+    if (n > 1) HIP_TRY(stage_upload(m->ctx, m->prompt_dev, tokens, sizeof(int32_t) * (size_t)n)); // (one token travels as a kernel argument)
     HIP_TRY(launch_set_state(m->state, start_pos, tokens[0], 1, st));
     for (int i = 0; i < n; i++) {
         int rc = enqueue_token_step(m, c, start_pos + i + 1, i == n - 1);
@@ -1364,8 +1400,7 @@ extern "C" int rlh_forward(rlh_model *m, rlh_caches *c, const int32_t *tokens, i
     CtxLock lock(m->ctx);
     rc = enqueue_forward(m, c, tokens, n, start_pos);
     if (rc != RLH_OK) return rc;
-    HIP_TRY(hipMemcpyAsync(logits_out, m->logits, sizeof(float) * (size_t)m->prm.vocab_size, hipMemcpyDeviceToHost, m->ctx->stream));
-    HIP_TRY(hipStreamSynchronize(m->ctx->stream));
+    HIP_TRY(stage_download(m->ctx, logits_out, m->logits, sizeof(float) * (size_t)m->prm.vocab_size));
     return RLH_OK;
 }
 

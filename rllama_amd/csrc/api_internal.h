@@ -61,6 +61,8 @@ bool tunables_set(Tunables &t, const char *name, const char *value);
 void tunables_from_env(Tunables &t);
 } // namespace rlh
 
+constexpr size_t kStageBytes = (size_t)1 << 20;
+
 struct rlh_ctx {
     int device = 0;
     int verbose = 0;
@@ -74,6 +76,10 @@ struct rlh_ctx {
     rlh::TensorPool pool;
     Tunables tun;
     unsigned tun_version = 0;        // bumped by rlh_set_option: captured decode steps of an older version are dropped
+    // Page-locked staging of small host transfers, [0, kStageBytes) for uploads and as much again for downloads: a call holds mu from its first
+    // transfer until the stream is idle, so one call uses it at a time.  Null until the first use, or where it could not be allocated.
+    char *stage = nullptr;
+    bool stage_busy = false; // an upload from it may still be queued
     void *noalloc_scratch = nullptr; // this device's address of the library's static work memory (api_ops.hip)
 };
 
@@ -100,6 +106,10 @@ struct CtxLock {
 };
 
 namespace rlh {
+// Transfers between the caller's pageable memory and the device with the context locked, through page-locked staging where they fit.
+// stage_upload: `host` is the caller's again at once.  stage_download: waits for the stream.
+hipError_t stage_upload(rlh_ctx *ctx, void *dev, const void *host, size_t bytes);
+hipError_t stage_download(rlh_ctx *ctx, void *host, const void *dev, size_t bytes);
 void pool_release(rlh_ctx *ctx); // waits for the stream and frees the kept buffers
 // hipMalloc for everything the library holds on the device: when memory runs out, the context's kept buffers are freed first
 hipError_t device_alloc(rlh_ctx *ctx, void **p, size_t bytes);

@@ -64,6 +64,10 @@ extern "C" int rlh_tensor_download(rlh_tensor *t, void *host, int cols_capacity,
     if (!t || !host || cols_capacity < t->cols) return fail(RLH_ERR_INVALID, "rlh_tensor_download: bad argument");
     CtxLock lock(t->ctx);
     const size_t es = t->esize();
+    if (t->cols == cols_capacity && !ev) { // (with an event the caller's memory is written after this call returns)
+        HIP_TRY(stage_download(t->ctx, host, t->p, t->count() * es));
+        return RLH_OK;
+    }
     if (t->cols == cols_capacity) HIP_TRY(hipMemcpyAsync(host, t->p, t->count() * es, hipMemcpyDeviceToHost, t->ctx->stream));
     else
         HIP_TRY(hipMemcpy2DAsync(host, (size_t)cols_capacity * es, t->p, (size_t)t->cols * es, (size_t)t->cols * es, (size_t)t->rows, hipMemcpyDeviceToHost,
