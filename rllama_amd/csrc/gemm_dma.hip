@@ -727,69 +727,71 @@ __global__ void gemm_split_finish_kernel(GemmParams p, const float *partial, int
 }
 
 // The same second step for the residual epilogue with the row RMSNorm that follows it: one workgroup per row of C adds the
-// partial sums in the order of the splits, applies the epilogue, keeps the row in registers, and writes the normalised row
-// rounded to f16 as well (the loop structure and the order of additions of rmsnorm_rows_f16_kernel, prefill.hip).
-constexpr int kFinishNormVecs = 8; // rows of up to 256 x 4 x 8 floats
-__global__ __launch_bounds__(256) void gemm_split_finish_norm_kernel(GemmParams p, const float *partial, int splits) {
+// partial sums in the order of the splits, applies the epilogue, and writes the normalised row rounded to f16 as well.
+// Bound by latency: few rows, and per element a chain of loads.  So a thread has one or two pieces of the row and requests four partial
+// sums at a time, and the residual and the weights with the first of them (256 threads with up to eight pieces of the row each, one partial
+// sum after the other: 6.9 us for 131 rows of 4096 in four splits, 5.4 like this).  The sum of squares is taken by the first 256 threads in the
+// order of rmsnorm_rows_f16_kernel (prefill.hip), from LDS.
+constexpr int kFinishThreads = 1024, kFinishVecs = 2, kFinishNormVecs = 8; // rows of up to 1024 x 2 x 4 = 256 x 8 x 4 floats
+__global__ __launch_bounds__(kFinishThreads) void gemm_split_finish_norm_kernel(GemmParams p, const float *partial, int splits) {
     __shared__ float red[16];
+    __shared__ float4_t xrow[kFinishThreads * kFinishVecs];
     const size_t per = (size_t)p.m * p.n;
     const int r = blockIdx.x, tid = threadIdx.x, n4 = p.n / 4;
     const size_t row = (size_t)r * p.ldc, wrow = (size_t)r * p.n;
-    const float4_t *w4 = reinterpret_cast<const float4_t *>(p.norm_w);
-    float4_t xv[kFinishNormVecs];
+    float4_t res[kFinishVecs], wn[kFinishVecs], sum[kFinishVecs];
+#pragma unroll
+    for (int j = 0; j < kFinishVecs; j++) {
+        const int i = tid + j * kFinishThreads;
+        if (i < n4) {
+            res[j] = *reinterpret_cast<const float4_t *>(p.residual + row + (size_t)i * 4);
+            wn[j] = reinterpret_cast<const float4_t *>(p.norm_w)[i];
+            const float *src = partial + wrow + (size_t)i * 4;
+            for (int z = 0; z < splits; z += 4) {
+                float4_t part[4];
+#pragma unroll
+                for (int q = 0; q < 4; q++)
+                    if (z + q < splits) part[q] = *reinterpret_cast<const float4_t *>(src + (size_t)(z + q) * per);
+#pragma unroll
+                for (int q = 0; q < 4; q++)
+                    if (z + q < splits) sum[j] = z + q == 0 ? part[q] : sum[j] + part[q];
+            }
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < kFinishVecs; j++) {
+        const int i = tid + j * kFinishThreads;
+        if (i < n4) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) sum[j][e] = res[j][e] + f16r(sum[j][e]);
+            *reinterpret_cast<float4_t *>(reinterpret_cast<float *>(p.c) + row + (size_t)i * 4) = sum[j];
+            xrow[i] = sum[j];
+        }
+    }
+    __syncthreads();
     float ss = 0.0f;
-    // the pieces outermost, so that a thread's loads of one piece are all in flight together (per element the partial sums are
-    // still added in the order of the pieces)
-#pragma unroll
-    for (int j = 0; j < kFinishNormVecs; j++) {
-        const int i = tid + j * 256;
-        xv[j] = i < n4 ? *reinterpret_cast<const float4_t *>(partial + wrow + (size_t)i * 4) : float4_t{0.0f, 0.0f, 0.0f, 0.0f};
-    }
-    float4_t res[kFinishNormVecs];
-#pragma unroll
-    for (int j = 0; j < kFinishNormVecs; j++) {
-        const int i = tid + j * 256;
-        res[j] = i < n4 ? *reinterpret_cast<const float4_t *>(p.residual + row + (size_t)i * 4) : float4_t{0.0f, 0.0f, 0.0f, 0.0f};
-    }
-    for (int z = 1; z < splits; z++) {
-        float4_t part[kFinishNormVecs];
+    if (tid < 256) {
 #pragma unroll
         for (int j = 0; j < kFinishNormVecs; j++) {
             const int i = tid + j * 256;
-            part[j] = i < n4 ? *reinterpret_cast<const float4_t *>(partial + z * per + wrow + (size_t)i * 4) : float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+            if (i < n4) {
+                const float4_t v = xrow[i];
+#pragma unroll
+                for (int e = 0; e < 4; e++) ss = fmaf(v[e], v[e], ss);
+            }
         }
-#pragma unroll
-        for (int j = 0; j < kFinishNormVecs; j++) xv[j] += part[j];
     }
-#pragma unroll
-    for (int j = 0; j < kFinishNormVecs; j++) {
-        const int i = tid + j * 256;
-        if (i < n4) {
-#pragma unroll
-            for (int e = 0; e < 4; e++) xv[j][e] = res[j][e] + f16r(xv[j][e]);
-            *reinterpret_cast<float4_t *>(reinterpret_cast<float *>(p.c) + row + (size_t)i * 4) = xv[j];
-        }
-#pragma unroll
-        for (int e = 0; e < 4; e++) ss = fmaf(xv[j][e], xv[j][e], ss);
-    }
-    float4_t wn[kFinishNormVecs]; // requested before the row sum, not after it
-#pragma unroll
-    for (int j = 0; j < kFinishNormVecs; j++) {
-        const int i = tid + j * 256;
-        wn[j] = i < n4 ? w4[i] : float4_t{0.0f, 0.0f, 0.0f, 0.0f};
-    }
-    ss = block_sum(ss, red);
+    ss = block_sum(ss, red); // (wavefronts 4 to 15 add zeros)
     const float rs = 1.0f / sqrtf(ss / (float)p.n + p.norm_eps);
     half_t *yr = p.norm_out + (size_t)r * p.n;
 #pragma unroll
-    for (int j = 0; j < kFinishNormVecs; j++) {
-        const int i = tid + j * 256;
+    for (int j = 0; j < kFinishVecs; j++) {
+        const int i = tid + j * kFinishThreads;
         if (i < n4) {
-            const float4_t wv = wn[j];
             typedef __attribute__((ext_vector_type(4))) _Float16 half4_t;
             half4_t o;
 #pragma unroll
-            for (int e = 0; e < 4; e++) o[e] = to_f16((xv[j][e] * rs) * wv[e]);
+            for (int e = 0; e < 4; e++) o[e] = to_f16((sum[j][e] * rs) * wn[j][e]);
             *reinterpret_cast<half4_t *>(yr + i * 4) = o;
         }
     }
@@ -1028,7 +1030,7 @@ hipError_t launch_gemm_f16_dma(const GemmParams &p_in, int epilogue, hipStream_t
         if (e != hipSuccess) return e;
         if (epilogue == kGemmEpiResAddF32 && p_in.norm_w != nullptr && p_in.norm_out != nullptr && p_in.norm_done != nullptr &&
             p_in.n <= 256 * 4 * kFinishNormVecs && !p_in.tune.no_finish_norm) {
-            hipLaunchKernelGGL(gemm_split_finish_norm_kernel, dim3(p_in.m), dim3(256), 0, s, p_in, (const float *)p_in.workspace, splits);
+            hipLaunchKernelGGL(gemm_split_finish_norm_kernel, dim3(p_in.m), dim3(kFinishThreads), 0, s, p_in, (const float *)p_in.workspace, splits);
             *p_in.norm_done = 1;
             return hipGetLastError();
         }
