@@ -341,7 +341,12 @@ __global__ __launch_bounds__(2 * kBK * kRH * kCH) void gemm_f16_rows_kernel(Gemm
     }
 }
 
-inline int rows_fragments(const GemmParams &p) { return p.f32_operands && p.m > 64 ? 6 : (p.m + 15) / 16; }
+// 16-row fragments of a product's tile.  From 65 rows on an even number (fp32: 6): their wavefronts split the rows in two, and two wavefronts per
+// SIMD cover for each other's waits (7B shape, 131 rows: pieces of wo and w2 25.3 us on nine fragments and four wavefronts, 23.0 on ten and eight).
+inline int rows_fragments(const GemmParams &p) {
+    const int needed = (p.m + 15) / 16;
+    return needed <= 4 ? needed : p.f32_operands ? 6 : (needed + 1) / 2 * 2;
+}
 
 // Microseconds per 1024 values of k that the workgroups of a product of `pieces` pieces take on nf x 16 columns each: rounds of
 // workgroups x what a compute unit stages at 45 GB/s, or (fp32) what its matrix cores take at 0.45 TFLOP/s, whichever is longer.
@@ -405,11 +410,8 @@ hipError_t launch_rows_epi(const GemmParams &p, hipStream_t s) {
     case 2: return launch_rows_mf<kEpi, 2>(p, s);
     case 3: return launch_rows_mf<kEpi, 3>(p, s);
     case 4: return launch_rows_mf<kEpi, 4>(p, s);
-    case 5: return launch_rows_mf<kEpi, 5>(p, s);
     case 6: return launch_rows_mf<kEpi, 6>(p, s);
-    case 7: return launch_rows_mf<kEpi, 7>(p, s);
     case 8: return launch_rows_mf<kEpi, 8>(p, s);
-    case 9: return launch_rows_mf<kEpi, 9>(p, s);
     case 10: return launch_rows_mf<kEpi, 10>(p, s);
     default: return hipErrorInvalidValue;
     }
