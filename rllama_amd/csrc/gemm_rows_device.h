@@ -11,9 +11,9 @@
 // What bounds it: few rows, memory (8 rows, us: wq|wk|wv 12288 x 4096 24.8 -> 18.3, w1|w3 11008 x 4096 39.5 -> 31.8 = 5.7 TB/s, w2 4096 x 11008
 // 20.3 + 5.6 for adding the pieces -> 17.3); many rows, what a compute unit takes from L2 into LDS, 50 to 70 GB/s here (131 rows:
 // wq|wk|wv 44 -> 33, w1|w3 58 -> 44; spreading the requests over the MFMAs, wavefronts of their own for them and units of 64 change
-// nothing there).  Time to the first token, former kernels -> this: 7B shape 8 / 131 rows 3.61 -> 3.03 / 5.27 -> 4.85 ms; dim 2304,
-// 10 layers, 8 / 24 / 64 / 128 / 160 rows 754 / 908 / 1001 / 1090 / 1083 -> 564 / 632 / 735 / 890 / 994 us; dim 5120, 4 layers, 8 / 64 / 160 rows
-// 754 / 932 / 1069 -> 649 / 763 / 1035.  Beyond 160 rows the operand of activations alone fills the LDS.
+// nothing there).  Time to the first token, former kernels -> this: 7B shape 8 / 131 rows 3.61 -> 3.03 / 5.83 -> 4.72 ms; dim 2304, 10 layers,
+// 8 / 24 / 64 rows 754 / 908 / 1001 -> 564 / 632 / 735 us; dim 2816, 8 layers, 112 / 144 rows 1095 / 1128 -> 832 / 910; dim 5120, 4 layers,
+// 8 / 64 / 144 rows 754 / 932 / 1060 -> 649 / 763 / 982.  Beyond 160 rows the operand of activations alone fills the LDS.
 //
 // Weights are the first operand of v_mfma_f32_16x16x32_f16, so a lane ends up with four consecutive columns of one row.
 #pragma once
