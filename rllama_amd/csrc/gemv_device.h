@@ -221,7 +221,11 @@ __device__ __forceinline__ void gemv_body(const GemvParams &p, uint4_t *smem_raw
     wmat[0] = reinterpret_cast<const WT *>(p.w);
     if constexpr (kMats == 2) wmat[1] = reinterpret_cast<const WT *>(p.w_b);
     const int unit_first = blockIdx.x * kGemvWaves + wave;
-    uint4_t wpre[kBurst] = {};
+    uint4_t wpre[kBurst];
+    if constexpr (kGroup > 0) { // units past the end are not loaded, their sums not used
+#pragma unroll
+        for (int i = 0; i < kBurst; i++) wpre[i] = uint4_t{0, 0, 0, 0};
+    }
     bool have_pre = false;
     auto preload = [&]() {
         if constexpr (kGroup > 0) {
