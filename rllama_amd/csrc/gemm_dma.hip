@@ -132,6 +132,13 @@ __global__ __launch_bounds__(128 * kWavesM) void gemm_f16_dma_kernel(GemmParams 
             }
         }
     };
+    auto issue = [&](int kt) {
+        const unsigned dst = lds_base + (unsigned)(kt % kStages) * kStageBytes + (unsigned)wave * 1024;
+#pragma unroll
+        for (int i = 0; i < kLoadsMax; i++)
+            if (i < kLoadsMin || !short_wave) dma16(gsrc[i] + (src_is_b[i] ? iss_kb : iss_ka), dst + i * (kWaves * 1024));
+        issue_done(kt);
+    };
 
     constexpr int kNTs = kP * kNT;                       // column tiles of a wavefront over all products (product q: j / kNT)
     float16_t acc[kIT][kNTs];
@@ -206,7 +213,8 @@ __global__ __launch_bounds__(128 * kWavesM) void gemm_f16_dma_kernel(GemmParams 
     // memory path until the last is taken, its fragment reads and MFMAs behind it.  With four stages or more they are spread over the
     // MFMAs instead, one per kDmaEvery fragment pairs and in a fixed order (7B shape, 131 rows: wq|wk|wv on 128 x 64 44.4 -> 39.9 us, w1|w3 on 192 x 64 58.2 -> 54.4).
     // With two or three, K-tile t + 1 has to arrive while K-tile t is consumed, and what counts is that it is requested early (256 x 192, 7B
-    // wq|wk|wv of 1024 rows 107 us at once, 114 - 117 spread).
+    // wq|wk|wv of 1024 rows 107 us at once, 114 - 117 spread).  Their loop stays a plain one: written with the fixed order's helpers
+    // the compiler prepares the addresses between the requests, and wo / w2 on 256 x 128 (1500 rows of 4608) take 182.1 us instead of 179.1.
     constexpr bool kSpread = kStages >= 4;
     constexpr int kKS = kBK / 16;
     constexpr int kSplitJ = kNTs / 2; // column tiles of the last K-step whose MFMAs run before the tile change (0 .. kNT measured alike)
@@ -227,6 +235,13 @@ __global__ __launch_bounds__(128 * kWavesM) void gemm_f16_dma_kernel(GemmParams 
         const int lc = ks * 2 + fch;
         if (r < kIT) af[set][r] = *reinterpret_cast<const half8_t *>(stage + a_off[r] + ((lc ^ a_sw[r]) << 4));
         else bf[set][r - kIT] = *reinterpret_cast<const half8_t *>(stage + b_off[r - kIT] + ((lc ^ b_sw[r - kIT]) << 4));
+    };
+    auto read_frags = [&](int set, const unsigned char *stage, int ks) {
+        const int lc = ks * 2 + fch;
+#pragma unroll
+        for (int i = 0; i < kIT; i++) af[set][i] = *reinterpret_cast<const half8_t *>(stage + a_off[i] + ((lc ^ a_sw[i]) << 4));
+#pragma unroll
+        for (int j = 0; j < (kDual ? 0 : kNT); j++) bf[set][j] = *reinterpret_cast<const half8_t *>(stage + b_off[j] + ((lc ^ b_sw[j]) << 4));
     };
     if constexpr (kDual) {
         // Two products: 192 accumulator registers of the 256 a wavefront has here, so everything else is kept small.  Staging
@@ -272,187 +287,225 @@ __global__ __launch_bounds__(128 * kWavesM) void gemm_f16_dma_kernel(GemmParams 
             const int c = ((ks * 2 + fch) ^ sw) << 4;
             b[j] = *reinterpret_cast<const half8_t *>(stage + xb + (q * kBN + j * 32) * kRowBytes + c);
         };
-        constexpr int kSlots = kIT * kNT, kReads = kIT + kNT;  // per product and K-step
-        constexpr int kDmaSlots = (kKS - 1) * 2 * kSlots + kSlots; // up to the tile change
-        constexpr int kSpan = kDmaSlots < kDmaEvery * kLoads ? kDmaSlots : kDmaEvery * kLoads;
-        for (int t = 0; t < kStages; t++) {
+        auto issue2 = [&](int kt) {
+            const unsigned dst = lds_base + (unsigned)(kt % kStages) * kStageBytes + (unsigned)wave * 1024;
 #pragma unroll
-            for (int i = 0; i < kLoads; i++) issue2_load(t, i);
-            issue2_done(t);
-        }
+            for (int i = 0; i < kLA; i++) dma16_base(s_a + iss_k, voff_a[i], dst + i * (kWaves * 1024));
+#pragma unroll
+            for (int i = 0; i < kLB; i++) dma16_base(s_b + iss_k, voff_b[i], dst + (kLA + i) * (kWaves * 1024));
+#pragma unroll
+            for (int i = 0; i < kLB; i++) dma16_base(s_b2 + iss_k, voff_b[i], dst + (kLA + kLB + i) * (kWaves * 1024));
+            issue2_done(kt);
+        };
+        auto read_as = [&](int set, const unsigned char *stage, int ks) {
+            const int c = ((ks * 2 + fch) ^ sw) << 4;
+#pragma unroll
+            for (int i = 0; i < kIT; i++) af[set][i] = *reinterpret_cast<const half8_t *>(stage + xa + i * (32 * kRowBytes) + c);
+        };
+        auto read_bs = [&](half8_t (&b)[kNT], const unsigned char *stage, int ks, int q) {
+            const int c = ((ks * 2 + fch) ^ sw) << 4;
+#pragma unroll
+            for (int j = 0; j < kNT; j++) b[j] = *reinterpret_cast<const half8_t *>(stage + xb + (q * kBN + j * 32) * kRowBytes + c);
+        };
+        constexpr int kSlots = kIT * kNT, kReads = kIT + kNT;  // per product and K-step
+        auto mmas = [&](int set, const half8_t (&b)[kNT], int q) { // the MFMAs of product q
+#pragma unroll
+            for (int j = 0; j < kNT; j++)
+#pragma unroll
+                for (int i = 0; i < kIT; i++) mma(af[set][i], b[j], acc[i][q * kNT + j]);
+        };
+#pragma unroll
+        for (int t = 0; t < kStages; t++) issue2(t);
         wait_vmcnt<(kStages - 1) * kLoads>();
         __syncthreads();
+        read_as(0, lds_raw, 0);
+        read_bs(b0, lds_raw, 0, 0);
+        if constexpr (kSpread) {
+            constexpr int kDmaSlots = (kKS - 1) * 2 * kSlots + kSlots; // up to the tile change
+            constexpr int kSpan = kDmaSlots < kDmaEvery * kLoads ? kDmaSlots : kDmaEvery * kLoads;
+            for (int kt = 0; kt < n_kt; kt++) {
+                const unsigned char *stage = lds_raw + (kt % kStages) * kStageBytes;
+                const int kt_in = kt + kStages - 1; // the K-tile requested during this one, into the stage that the tile change before freed
+                auto dma_at = [&](auto atc) {
+                    constexpr int at = decltype(atc)::value;
+                    if constexpr (at < kSpan) {
+                        constexpr int lo = at * kLoads / kSpan, hi = (at + 1) * kLoads / kSpan;
+                        if constexpr (hi > lo) {
+                            if (kt > 0) {
 #pragma unroll
-        for (int i = 0; i < kIT; i++) read_a(0, lds_raw, 0, i);
-#pragma unroll
-        for (int j = 0; j < kNT; j++) read_b(b0, lds_raw, 0, 0, j);
-        for (int kt = 0; kt < n_kt; kt++) {
-            const unsigned char *stage = lds_raw + (kt % kStages) * kStageBytes;
-            const int kt_in = kt + kStages - 1; // the K-tile requested during this one, into the stage that the tile change before freed
-            auto dma_at = [&](auto atc) {
-                constexpr int at = decltype(atc)::value;
-                if constexpr (at < kSpan) {
-                    constexpr int lo = at * kLoads / kSpan, hi = (at + 1) * kLoads / kSpan;
-                    if constexpr (hi > lo) {
-                        if (kt > 0) {
-#pragma unroll
-                            for (int i = lo; i < hi; i++) issue2_load(kt_in, i);
-                            if constexpr (hi == kLoads) issue2_done(kt_in);
+                                for (int i = lo; i < hi; i++) issue2_load(kt_in, i);
+                                if constexpr (hi == kLoads) issue2_done(kt_in);
+                            }
                         }
                     }
-                }
-                __builtin_amdgcn_sched_barrier(0);
-            };
-            static_for<kKS>([&](auto ksc) {
-                constexpr int ks = decltype(ksc)::value, cur = ks & 1, nxt = cur ^ 1;
-                if constexpr (kSpread) {
+                    __builtin_amdgcn_sched_barrier(0);
+                };
+                static_for<kKS>([&](auto ksc) {
+                    constexpr int ks = decltype(ksc)::value, cur = ks & 1, nxt = cur ^ 1;
                     static_for<kSlots>([&](auto slc) {
                         constexpr int sl = decltype(slc)::value;
                         mma(af[cur][sl % kIT], b0[sl / kIT], acc[sl % kIT][sl / kIT]);
                         if constexpr (sl < kNT) read_b(b1, stage, ks, 1, sl);
                         dma_at(std::integral_constant<int, ks * 2 * kSlots + sl>{});
                     });
-                } else {
+                    if constexpr (ks + 1 < kKS) {
+                        static_for<kSlots>([&](auto slc) {
+                            constexpr int sl = decltype(slc)::value;
+                            mma(af[cur][sl % kIT], b1[sl / kIT], acc[sl % kIT][kNT + sl / kIT]);
+                            if constexpr (sl < kIT) read_a(nxt, stage, ks + 1, sl);
+                            else if constexpr (sl < kReads) read_b(b0, stage, ks + 1, 0, sl - kIT);
+                            if constexpr (sl + 1 == kSlots && kReads > kSlots) {
 #pragma unroll
-                    for (int j = 0; j < kNT; j++) read_b(b1, stage, ks, 1, j);
+                                for (int r = kSlots; r < kReads; r++) {
+                                    if (r < kIT) read_a(nxt, stage, ks + 1, r);
+                                    else read_b(b0, stage, ks + 1, 0, r - kIT);
+                                }
+                            }
+                            dma_at(std::integral_constant<int, (ks * 2 + 1) * kSlots + sl>{});
+                        });
+                    } else {
+                        wait_vmcnt<(kStages - 2) * kLoads>();
+                        __syncthreads(); // K-tile kt + 1 is in LDS for everybody, and nobody reads K-tile kt any more
+                        const unsigned char *next = lds_raw + ((kt + 1) % kStages) * kStageBytes;
+                        read_as(nxt, next, 0);
+                        read_bs(b0, next, 0, 0);
+                        __builtin_amdgcn_sched_barrier(0);
+                        mmas(cur, b1, 1);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                });
+            }
+        } else {
+            for (int kt = 0; kt < n_kt; kt++) {
+                const unsigned char *stage = lds_raw + (kt % kStages) * kStageBytes;
 #pragma unroll
-                    for (int sl = 0; sl < kSlots; sl++) mma(af[cur][sl % kIT], b0[sl / kIT], acc[sl % kIT][sl / kIT]);
+                for (int ks = 0; ks < kKS; ks++) {
+                    const int cur = ks & 1, nxt = cur ^ 1;
+                    read_bs(b1, stage, ks, 1);
+                    mmas(cur, b0, 0);
 #pragma unroll
                     for (int r = 0; r < kNT; r++) {
                         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0); // MFMA
                         __builtin_amdgcn_sched_group_barrier(0x100, 1, 0); // DS read
                     }
                     if constexpr (kSlots > kNT) __builtin_amdgcn_sched_group_barrier(0x008, kSlots - kNT, 0);
-                }
-                if constexpr (ks + 1 < kKS && kSpread) {
-                    static_for<kSlots>([&](auto slc) {
-                        constexpr int sl = decltype(slc)::value;
-                        mma(af[cur][sl % kIT], b1[sl / kIT], acc[sl % kIT][kNT + sl / kIT]);
-                        if constexpr (sl < kIT) read_a(nxt, stage, ks + 1, sl);
-                        else if constexpr (sl < kReads) read_b(b0, stage, ks + 1, 0, sl - kIT);
-                        if constexpr (sl + 1 == kSlots && kReads > kSlots) {
+                    if (ks + 1 < kKS) {
+                        read_as(nxt, stage, ks + 1);
+                        read_bs(b0, stage, ks + 1, 0);
+                        mmas(cur, b1, 1);
+                        constexpr int kPairs = kSlots < kReads ? kSlots : kReads;
 #pragma unroll
-                            for (int r = kSlots; r < kReads; r++) {
-                                if (r < kIT) read_a(nxt, stage, ks + 1, r);
-                                else read_b(b0, stage, ks + 1, 0, r - kIT);
-                            }
+                        for (int r = 0; r < kPairs; r++) {
+                            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
                         }
-                        dma_at(std::integral_constant<int, (ks * 2 + 1) * kSlots + sl>{});
-                    });
-                } else if constexpr (ks + 1 < kKS) {
-#pragma unroll
-                    for (int i = 0; i < kIT; i++) read_a(nxt, stage, ks + 1, i);
-#pragma unroll
-                    for (int j = 0; j < kNT; j++) read_b(b0, stage, ks + 1, 0, j);
-#pragma unroll
-                    for (int sl = 0; sl < kSlots; sl++) mma(af[cur][sl % kIT], b1[sl / kIT], acc[sl % kIT][kNT + sl / kIT]);
-                    constexpr int kPairs = kSlots < kReads ? kSlots : kReads;
-#pragma unroll
-                    for (int r = 0; r < kPairs; r++) {
-                        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                        if constexpr (kSlots > kPairs) __builtin_amdgcn_sched_group_barrier(0x008, kSlots - kPairs, 0);
+                        if constexpr (kReads > kPairs) __builtin_amdgcn_sched_group_barrier(0x100, kReads - kPairs, 0);
+                    } else {
+                        __builtin_amdgcn_sched_barrier(0);
+                        wait_vmcnt<(kStages - 2) * kLoads>();
+                        __syncthreads(); // K-tile kt + 1 is in LDS for everybody, and nobody reads K-tile kt any more
+                        issue2(kt + kStages);
+                        const unsigned char *next = lds_raw + ((kt + 1) % kStages) * kStageBytes;
+                        read_as(nxt, next, 0);
+                        read_bs(b0, next, 0, 0);
+                        __builtin_amdgcn_sched_barrier(0);
+                        mmas(cur, b1, 1);
                     }
-                    if constexpr (kSlots > kPairs) __builtin_amdgcn_sched_group_barrier(0x008, kSlots - kPairs, 0);
-                    if constexpr (kReads > kPairs) __builtin_amdgcn_sched_group_barrier(0x100, kReads - kPairs, 0);
-                } else {
-                    __builtin_amdgcn_sched_barrier(0);
-                    wait_vmcnt<(kStages - 2) * kLoads>();
-                    __syncthreads(); // K-tile kt + 1 is in LDS for everybody, and nobody reads K-tile kt any more
-                    if constexpr (!kSpread) {
-#pragma unroll
-                        for (int i = 0; i < kLoads; i++) issue2_load(kt + kStages, i);
-                        issue2_done(kt + kStages);
-                    }
-                    const unsigned char *next = lds_raw + ((kt + 1) % kStages) * kStageBytes;
-#pragma unroll
-                    for (int i = 0; i < kIT; i++) read_a(nxt, next, 0, i);
-#pragma unroll
-                    for (int j = 0; j < kNT; j++) read_b(b0, next, 0, 0, j);
-                    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                    for (int sl = 0; sl < kSlots; sl++) mma(af[cur][sl % kIT], b1[sl / kIT], acc[sl % kIT][kNT + sl / kIT]);
-                    __builtin_amdgcn_sched_barrier(0);
                 }
-            });
+            }
         }
     } else {
         constexpr int kSlots = kIT * kNTs, kReads = kIT + kNTs; // fragment pairs and fragments of a K-step
-        constexpr int kDmaSlots = (kKS - 1) * kSlots;           // of the K-steps in front of the tile change
-        constexpr int kSpan = kDmaSlots < kDmaEvery * kLoadsMax ? kDmaSlots : kDmaEvery * kLoadsMax;
-        auto slot_mma = [&](int set, int sl) { mma(af[set][sl % kIT], bf[set][sl / kIT], acc[sl % kIT][sl / kIT]); };
-        for (int t = 0; t < kStages; t++) {
+        auto mmas = [&](int set, int j0, int j1) {
 #pragma unroll
-            for (int i = 0; i < kLoadsMax; i++) issue_load(t, i);
-            issue_done(t);
-        }
+            for (int j = j0; j < j1; j++)
+#pragma unroll
+                for (int i = 0; i < kIT; i++) mma(af[set][i], bf[set][j], acc[i][j]);
+        };
+        auto wait_next = [&]() {
+            if (short_wave) wait_vmcnt<(kStages - 2) * kLoadsMin>();
+            else wait_vmcnt<(kStages - 2) * kLoadsMax>();
+            __syncthreads(); // the next K-tile is in LDS for everybody, and nobody reads this one any more
+        };
+#pragma unroll
+        for (int t = 0; t < kStages; t++) issue(t);
         if (short_wave) wait_vmcnt<(kStages - 1) * kLoadsMin>();
         else wait_vmcnt<(kStages - 1) * kLoadsMax>();
         __syncthreads();
+        read_frags(0, lds_raw, 0);
+        if constexpr (kSpread) {
+            constexpr int kDmaSlots = (kKS - 1) * kSlots; // of the K-steps in front of the tile change
+            constexpr int kSpan = kDmaSlots < kDmaEvery * kLoadsMax ? kDmaSlots : kDmaEvery * kLoadsMax;
+            for (int kt = 0; kt < n_kt; kt++) {
+                const unsigned char *stage = lds_raw + (kt % kStages) * kStageBytes;
+                const int kt_in = kt + kStages - 1; // the K-tile requested during this one, into the stage that the tile change before freed
+                static_for<kKS>([&](auto ksc) {
+                    constexpr int ks = decltype(ksc)::value, cur = ks & 1, nxt = cur ^ 1;
+                    if constexpr (ks + 1 < kKS) {
+                        static_for<kSlots>([&](auto slc) {
+                            constexpr int sl = decltype(slc)::value, at = ks * kSlots + sl;
+                            mma(af[cur][sl % kIT], bf[cur][sl / kIT], acc[sl % kIT][sl / kIT]);
+                            if constexpr (sl < kReads) read_frag(nxt, stage, ks + 1, sl);
+                            if constexpr (sl + 1 == kSlots && kReads > kSlots) {
 #pragma unroll
-        for (int r = 0; r < kReads; r++) read_frag(0, lds_raw, 0, r);
-        for (int kt = 0; kt < n_kt; kt++) {
-            const unsigned char *stage = lds_raw + (kt % kStages) * kStageBytes;
-            const int kt_in = kt + kStages - 1; // the K-tile requested during this one, into the stage that the tile change before freed
-            static_for<kKS>([&](auto ksc) {
-                constexpr int ks = decltype(ksc)::value, cur = ks & 1, nxt = cur ^ 1;
-                if constexpr (ks + 1 < kKS && kSpread) {
-                    static_for<kSlots>([&](auto slc) {
-                        constexpr int sl = decltype(slc)::value, at = ks * kSlots + sl;
-                        slot_mma(cur, sl);
-                        if constexpr (sl < kReads) read_frag(nxt, stage, ks + 1, sl);
-                        if constexpr (sl + 1 == kSlots && kReads > kSlots) {
+                                for (int r = kSlots; r < kReads; r++) read_frag(nxt, stage, ks + 1, r);
+                            }
+                            if constexpr (at < kSpan) {
+                                constexpr int lo = at * kLoadsMax / kSpan, hi = (at + 1) * kLoadsMax / kSpan;
+                                if constexpr (hi > lo) {
+                                    if (kt > 0) {
 #pragma unroll
-                            for (int r = kSlots; r < kReads; r++) read_frag(nxt, stage, ks + 1, r);
-                        }
-                        if constexpr (at < kSpan) {
-                            constexpr int lo = at * kLoadsMax / kSpan, hi = (at + 1) * kLoadsMax / kSpan;
-                            if constexpr (hi > lo) {
-                                if (kt > 0) {
-#pragma unroll
-                                    for (int i = lo; i < hi; i++) issue_load(kt_in, i);
-                                    if constexpr (hi == kLoadsMax) issue_done(kt_in);
+                                        for (int i = lo; i < hi; i++) issue_load(kt_in, i);
+                                        if constexpr (hi == kLoadsMax) issue_done(kt_in);
+                                    }
                                 }
                             }
-                        }
+                            __builtin_amdgcn_sched_barrier(0);
+                        });
+                    } else {
+                        mmas(cur, 0, kSplitJ);
                         __builtin_amdgcn_sched_barrier(0);
-                    });
-                } else if constexpr (ks + 1 < kKS) {
-#pragma unroll
-                    for (int r = 0; r < kReads; r++) read_frag(nxt, stage, ks + 1, r);
-#pragma unroll
-                    for (int sl = 0; sl < kSlots; sl++) slot_mma(cur, sl);
-                    // an LDS fragment read of the next step behind each of the first MFMAs of this one, so that the reads are in flight under
-                    // the matrix pipe (left to itself the scheduler issues them at the end of the step and the MFMAs wait for them)
-                    constexpr int kPerMma = kF32 ? 4 : 1; // MFMA instructions per fragment pair
-                    constexpr int kPairs = kSlots < kReads ? kSlots : kReads;
-#pragma unroll
-                    for (int r = 0; r < kPairs; r++) {
-                        __builtin_amdgcn_sched_group_barrier(0x008, kPerMma, 0); // MFMA
-                        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);       // DS read
+                        wait_next();
+                        read_frags(nxt, lds_raw + ((kt + 1) % kStages) * kStageBytes, 0);
+                        __builtin_amdgcn_sched_barrier(0);
+                        mmas(cur, kSplitJ, kNTs);
+                        __builtin_amdgcn_sched_barrier(0);
                     }
-                    if constexpr (kSlots > kPairs) __builtin_amdgcn_sched_group_barrier(0x008, (kSlots - kPairs) * kPerMma, 0);
-                    if constexpr (kReads > kPairs) __builtin_amdgcn_sched_group_barrier(0x100, kReads - kPairs, 0);
-                } else {
+                });
+            }
+        } else {
+            for (int kt = 0; kt < n_kt; kt++) {
+                const unsigned char *stage = lds_raw + (kt % kStages) * kStageBytes;
 #pragma unroll
-                    for (int sl = 0; sl < kSplitJ * kIT; sl++) slot_mma(cur, sl);
-                    __builtin_amdgcn_sched_barrier(0);
-                    if (short_wave) wait_vmcnt<(kStages - 2) * kLoadsMin>();
-                    else wait_vmcnt<(kStages - 2) * kLoadsMax>();
-                    __syncthreads(); // K-tile kt + 1 is in LDS for everybody, and nobody reads K-tile kt any more
-                    if constexpr (!kSpread) {
+                for (int ks = 0; ks < kKS; ks++) {
+                    const int cur = ks & 1, nxt = cur ^ 1;
+                    if (ks + 1 < kKS) {
+                        read_frags(nxt, stage, ks + 1);
+                        mmas(cur, 0, kNTs);
+                        // order within the step: an LDS fragment read of the next step behind each of the first MFMAs of this one,
+                        // so that the reads are in flight under the matrix pipe and none is left to wait for when the next step
+                        // begins (left to itself the scheduler issues the reads at the end of the step and the MFMAs wait for them)
+                        constexpr int kPerMma = kF32 ? 4 : 1; // MFMA instructions per fragment pair
+                        constexpr int kPairs = kSlots < kReads ? kSlots : kReads;
 #pragma unroll
-                        for (int i = 0; i < kLoadsMax; i++) issue_load(kt + kStages, i);
-                        issue_done(kt + kStages);
+                        for (int r = 0; r < kPairs; r++) {
+                            __builtin_amdgcn_sched_group_barrier(0x008, kPerMma, 0); // MFMA
+                            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);       // DS read
+                        }
+                        if constexpr (kSlots > kPairs) __builtin_amdgcn_sched_group_barrier(0x008, (kSlots - kPairs) * kPerMma, 0);
+                        if constexpr (kReads > kPairs) __builtin_amdgcn_sched_group_barrier(0x100, kReads - kPairs, 0);
+                    } else {
+                        mmas(cur, 0, kSplitJ);
+                        __builtin_amdgcn_sched_barrier(0);
+                        wait_next();
+                        issue(kt + kStages);
+                        read_frags(nxt, lds_raw + ((kt + 1) % kStages) * kStageBytes, 0);
+                        __builtin_amdgcn_sched_barrier(0);
+                        mmas(cur, kSplitJ, kNTs);
                     }
-                    const unsigned char *next = lds_raw + ((kt + 1) % kStages) * kStageBytes;
-#pragma unroll
-                    for (int r = 0; r < kReads; r++) read_frag(nxt, next, 0, r);
-                    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                    for (int sl = kSplitJ * kIT; sl < kSlots; sl++) slot_mma(cur, sl);
-                    __builtin_amdgcn_sched_barrier(0);
                 }
-            });
+            }
         }
     }
     wait_vmcnt<0>(); // drain the clamped tail loads before the block's LDS is released
