@@ -273,13 +273,14 @@ extern "C" int rlh_device_info(rlh_ctx *ctx, char *name, int cap, int *compute_u
     return RLH_OK;
 }
 
-// A copy to or from pageable memory goes through staging of the runtime's own, which it waits for; through memory of ours the copy is one
-// command of the stream and the wait at the end of the call is the only one.  With the upload of a single token gone (it is a kernel argument
-// anyway): decode step of dim 1024, 8 layers 238 -> 219 us (f32 mode 367 -> 313), 7B shape, 8 layers 715 -> 700; results of 630 KB to 2.4 MB
-// of op-level tensors 114 -> 112 and, above the staging, unchanged.  1 MiB: larger copies are no faster through it.
+// Token ids of prompts, logits and op-level results of at most 1 MiB.  A copy to or from pageable memory goes through staging of the runtime's
+// own, which it waits for; through memory of ours the copy is one launch on the stream and the wait at the end of the call is the only one.
+// It is a kernel's copy: a copy command is slower (decode step of dim 1024, 4 layers, us: pageable 196, command 146, kernel 134; prompt
+// of 8 rows 295, 182, 167) and stands in line with the driver's clearing of freed memory (dim 3328, 4 layers, within 0.2 s of freeing a model of 5 GB:
+// pageable 372, command 435, kernel 305; 345, 309 and 300 otherwise).  Larger copies are no faster through it.
 namespace rlh {
-static bool stage_ready(rlh_ctx *ctx, size_t bytes) {
-    if (bytes > kStageBytes) return false;
+static bool stage_ready(rlh_ctx *ctx, const void *dev, size_t bytes) {
+    if (bytes > kStageBytes || reinterpret_cast<uintptr_t>(dev) % 16 != 0) return false;
     if (ctx->stage == nullptr && hipHostMalloc((void **)&ctx->stage, 2 * kStageBytes, hipHostMallocDefault) != hipSuccess) {
         ctx->stage = nullptr;
         (void)hipGetLastError();
@@ -288,19 +289,19 @@ static bool stage_ready(rlh_ctx *ctx, size_t bytes) {
 }
 
 hipError_t stage_upload(rlh_ctx *ctx, void *dev, const void *host, size_t bytes) {
-    if (!stage_ready(ctx, bytes)) return hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, ctx->stream);
+    if (!stage_ready(ctx, dev, bytes)) return hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, ctx->stream);
     if (ctx->stage_busy) { // the call before ended without stage_download, maybe with an error
         const hipError_t e = hipStreamSynchronize(ctx->stream);
         if (e != hipSuccess) return e;
     }
     memcpy(ctx->stage, host, bytes);
     ctx->stage_busy = true;
-    return hipMemcpyAsync(dev, ctx->stage, bytes, hipMemcpyHostToDevice, ctx->stream);
+    return launch_copy_bytes(dev, ctx->stage, bytes, ctx->stream);
 }
 
 hipError_t stage_download(rlh_ctx *ctx, void *host, const void *dev, size_t bytes) {
-    const bool staged = stage_ready(ctx, bytes);
-    hipError_t e = hipMemcpyAsync(staged ? ctx->stage + kStageBytes : host, dev, bytes, hipMemcpyDeviceToHost, ctx->stream);
+    const bool staged = stage_ready(ctx, dev, bytes);
+    hipError_t e = staged ? launch_copy_bytes(ctx->stage + kStageBytes, dev, bytes, ctx->stream) : hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, ctx->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
     if (e == hipSuccess) ctx->stage_busy = false;
     if (e == hipSuccess && staged) memcpy(host, ctx->stage + kStageBytes, bytes);

@@ -184,6 +184,23 @@ hipError_t launch_advance_pos(DecodeState *state, const int32_t *tokens_dev, int
 }
 
 // ------------------------------------------------------------------------------------------------
+// Copies between device memory and page-locked host memory
+// ------------------------------------------------------------------------------------------------
+// Bound by the link.  A kernel and not a copy command: the copy engines are not ours alone (api.hip has the figures).
+__global__ __launch_bounds__(256) void copy_bytes_kernel(unsigned char *dst, const unsigned char *src, size_t bytes) {
+    const size_t n16 = bytes / 16, first = (size_t)blockIdx.x * 256 + threadIdx.x;
+    for (size_t i = first; i < n16; i += (size_t)gridDim.x * 256) reinterpret_cast<uint4_t *>(dst)[i] = reinterpret_cast<const uint4_t *>(src)[i];
+    if (first < bytes % 16) dst[n16 * 16 + first] = src[n16 * 16 + first];
+}
+
+hipError_t launch_copy_bytes(void *dst, const void *src, size_t bytes, hipStream_t s) {
+    if (((reinterpret_cast<uintptr_t>(dst) | reinterpret_cast<uintptr_t>(src)) & 15) != 0) return hipErrorInvalidValue;
+    const size_t blocks = (bytes / 16 + 255) / 256;
+    hipLaunchKernelGGL(copy_bytes_kernel, dim3((unsigned)(blocks < 1 ? 1 : blocks > 256 ? 256 : blocks)), dim3(256), 0, s, (unsigned char *)dst, (const unsigned char *)src, bytes);
+    return hipGetLastError();
+}
+
+// ------------------------------------------------------------------------------------------------
 // Synthetic fills
 // ------------------------------------------------------------------------------------------------
 template <typename ET>
