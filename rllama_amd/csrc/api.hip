@@ -273,7 +273,7 @@ extern "C" int rlh_device_info(rlh_ctx *ctx, char *name, int cap, int *compute_u
     return RLH_OK;
 }
 
-// Token ids of prompts, logits and op-level results of at most 1 MiB.  A copy to or from pageable memory goes through staging of the runtime's
+// Token ids of prompts and greedy picks, logits and op-level results of at most 1 MiB.  A copy to or from pageable memory goes through staging of the runtime's
 // own, which it waits for; through memory of ours the copy is one launch on the stream and the wait at the end of the call is the only one.
 // It is a kernel's copy: a copy command is slower (decode step of dim 1024, 4 layers, us: pageable 196, command 146, kernel 134; prompt
 // of 8 rows 295, 182, 167) and stands in line with the driver's clearing of freed memory (dim 3328, 4 layers, within 0.2 s of freeing a model of 5 GB:
@@ -281,7 +281,7 @@ extern "C" int rlh_device_info(rlh_ctx *ctx, char *name, int cap, int *compute_u
 namespace rlh {
 static bool stage_ready(rlh_ctx *ctx, const void *dev, size_t bytes) {
     if (bytes > kStageBytes || reinterpret_cast<uintptr_t>(dev) % 16 != 0) return false;
-    if (ctx->stage == nullptr && hipHostMalloc((void **)&ctx->stage, 2 * kStageBytes, hipHostMallocDefault) != hipSuccess) {
+    if (ctx->stage == nullptr && hipHostMalloc((void **)&ctx->stage, 2 * kStageBytes, hipHostMallocCoherent) != hipSuccess) {
         ctx->stage = nullptr;
         (void)hipGetLastError();
     }
@@ -290,7 +290,7 @@ static bool stage_ready(rlh_ctx *ctx, const void *dev, size_t bytes) {
 
 hipError_t stage_upload(rlh_ctx *ctx, void *dev, const void *host, size_t bytes) {
     if (!stage_ready(ctx, dev, bytes)) return hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, ctx->stream);
-    if (ctx->stage_busy) { // the call before ended without stage_download, maybe with an error
+    if (ctx->stage_busy) { // the call before ended with an error
         const hipError_t e = hipStreamSynchronize(ctx->stream);
         if (e != hipSuccess) return e;
     }
@@ -1415,8 +1415,7 @@ static int forward_greedy_scaled(rlh_model *m, rlh_caches *c, const int32_t *tok
     rc = enqueue_forward(m, c, tokens, n, start_pos);
     if (rc != RLH_OK) return rc;
     HIP_TRY(launch_argmax_advance(m->logits, m->prm.vocab_size, m->state, m->out_tokens, m->out_cap, st, scale));
-    HIP_TRY(hipMemcpyAsync(next_token, m->out_tokens, sizeof(int32_t), hipMemcpyDeviceToHost, st));
-    HIP_TRY(hipStreamSynchronize(st));
+    HIP_TRY(stage_download(m->ctx, next_token, m->out_tokens, sizeof(int32_t)));
     m->next_pos = start_pos + n;
     m->greedy_caches = c;
     return RLH_OK;
@@ -1563,8 +1562,7 @@ extern "C" int rlh_generate_greedy(rlh_model *m, rlh_caches *c, const int32_t *p
         rc = enqueue_decode_step(m, c, n_prompt + i);
     }
     if (rc == RLH_OK && e == hipSuccess) e = hipEventRecord(e2, st);
-    if (rc == RLH_OK && e == hipSuccess) e = hipMemcpyAsync(out_tokens, m->out_tokens, sizeof(int32_t) * (size_t)n_new, hipMemcpyDeviceToHost, st);
-    if (rc == RLH_OK && e == hipSuccess) e = hipStreamSynchronize(st);
+    if (rc == RLH_OK && e == hipSuccess) e = stage_download(m->ctx, out_tokens, m->out_tokens, sizeof(int32_t) * (size_t)n_new);
     if (rc == RLH_OK && e == hipSuccess) {
         float a = 0.0f, b = 0.0f;
         (void)hipEventElapsedTime(&a, e0, e1);

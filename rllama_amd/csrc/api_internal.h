@@ -79,7 +79,7 @@ struct rlh_ctx {
     // Page-locked staging of small host transfers, [0, kStageBytes) for uploads and as much again for downloads: a call holds mu from its first
     // transfer until the stream is idle, so one call uses it at a time.  Null until the first use, or where it could not be allocated.
     char *stage = nullptr;
-    bool stage_busy = false; // an upload from it may still be queued
+    bool stage_busy = false; // an upload from it may still be queued; every call that uploads ends with stage_download, unless it fails
     void *noalloc_scratch = nullptr; // this device's address of the library's static work memory (api_ops.hip)
 };
 
