@@ -782,10 +782,12 @@ __global__ void gemm_split_finish_kernel(GemmParams p, const float *partial, int
 // The same second step for the residual epilogue with the row RMSNorm that follows it: one workgroup per row of C adds the
 // partial sums in the order of the splits, applies the epilogue, and writes the normalised row rounded to f16 as well.
 // Bound by latency: few rows, and per element a chain of loads.  So a thread has one or two pieces of the row and requests four partial
-// sums at a time, and the residual and the weights with the first of them (256 threads with up to eight pieces of the row each, one partial
-// sum after the other: 6.9 us for 131 rows of 4096 in four splits, 5.4 like this).  The sum of squares is taken by the first 256 threads in the
-// order of rmsnorm_rows_f16_kernel (prefill.hip), from LDS.
-constexpr int kFinishThreads = 1024, kFinishVecs = 2, kFinishNormVecs = 8; // rows of up to 1024 x 2 x 4 = 256 x 8 x 4 floats
+// sums at a time, and the residual and the weights with the first of them.  As many threads as the row has pieces, at most 1024: more would
+// only leave a compute unit fewer rows.  us, 256 threads with up to eight pieces each, one partial sum after the other -> 1024 threads -> this:
+// 1500 rows of 1024 7.6 -> 8.8 -> 6.4, 1024 rows of 1920 7.7 -> 8.4 -> 7.2, 600 of 2048 6.0 -> 6.6 -> 5.7, 200 of 4096 6.9 -> 6.1, 256 of 8192
+// 10.0 -> 8.6.  The sum of squares is taken by the first 256 threads in the order of rmsnorm_rows_f16_kernel (prefill.hip), from LDS.
+constexpr int kFinishVecs = 2, kFinishNormVecs = 8; // rows of up to 1024 x 2 x 4 = 256 x 8 x 4 floats
+template <int kFinishThreads>
 __global__ __launch_bounds__(kFinishThreads) void gemm_split_finish_norm_kernel(GemmParams p, const float *partial, int splits) {
     __shared__ float red[16];
     __shared__ float4_t xrow[kFinishThreads * kFinishVecs];
@@ -1083,7 +1085,10 @@ hipError_t launch_gemm_f16_dma(const GemmParams &p_in, int epilogue, hipStream_t
         if (e != hipSuccess) return e;
         if (epilogue == kGemmEpiResAddF32 && p_in.norm_w != nullptr && p_in.norm_out != nullptr && p_in.norm_done != nullptr &&
             p_in.n <= 256 * 4 * kFinishNormVecs && !p_in.tune.no_finish_norm) {
-            hipLaunchKernelGGL(gemm_split_finish_norm_kernel, dim3(p_in.m), dim3(kFinishThreads), 0, s, p_in, (const float *)p_in.workspace, splits);
+            const float *partial = reinterpret_cast<const float *>(p_in.workspace);
+            if (p_in.n <= 1024) hipLaunchKernelGGL(gemm_split_finish_norm_kernel<256>, dim3(p_in.m), dim3(256), 0, s, p_in, partial, splits);
+            else if (p_in.n <= 2048) hipLaunchKernelGGL(gemm_split_finish_norm_kernel<512>, dim3(p_in.m), dim3(512), 0, s, p_in, partial, splits);
+            else hipLaunchKernelGGL(gemm_split_finish_norm_kernel<1024>, dim3(p_in.m), dim3(1024), 0, s, p_in, partial, splits);
             *p_in.norm_done = 1;
             return hipGetLastError();
         }
