@@ -874,6 +874,8 @@ static int choose_narrow(const GemmParams &p) {
     return -1;
 }
 
+bool gemm_f16_narrow(const GemmParams &p) { return choose_narrow(p) >= 0; }
+
 // Products with few output tiles (few prompt rows) leave most compute units without a workgroup, and what bounds them is
 // streaming the weights once: the K range is then cut into split_k pieces that run as separate workgroups (more weight bytes
 // in flight, every compute unit busy), their fp32 partial sums go to the caller's workspace and a second small kernel adds

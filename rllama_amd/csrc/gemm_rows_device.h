@@ -1,8 +1,8 @@
 // gemm_rows_device.h -- C = A * B^T (f16 operands, fp32 accumulate) for prompts of up to 160 rows, one row tile for all of them.
 //
 // With so few rows the product is one pass over the weights B, and what a compute unit can take in bounds it: from memory while the rows
-// are few, from L2 (every workgroup stages all of A) when they are many.  So a workgroup owns all rows and 16 to 64 columns, few
-// enough that all workgroups run in one round; its wavefronts split K (K-group g takes the g-th 32 halves of every unit of K), so that
+// are few, from L2 (every workgroup stages all of A) when they are many.  So a workgroup owns all rows and 16 to 64 columns, as
+// many as let all workgroups run in one round up to 16384 columns (more take more rounds); its wavefronts split K (K-group g takes the g-th 32 halves of every unit of K), so that
 // an operand byte is written to LDS once and read back once or twice; and the weights are swept in whole 256-byte pieces
 // of rows.  Every workgroup starts at another unit of K: workgroups in step ask for the same columns of all rows, i.e. for
 // addresses a whole row apart, and those meet in few memory channels (8 rows, 12288 x 4096: 21.3 us in step, 18.2 apart).  The
@@ -27,6 +27,7 @@
 namespace rlh {
 
 constexpr int kRowsMax = 160, kRowsF32Max = 96;
+constexpr int kRowsFrags128 = 13; // fragments (rows and columns) of a workgroup up to which three units of 128 halves fit the LDS
 
 // kMF x kNF: 16 x 16 fragments of a workgroup's tile (rows x columns of one product; kGemmEpiSiluGateF16 computes two products).
 // kBK: halves of K per unit; K-group g of the kBK / 32 takes K-step g of every unit.  kRH x kCH: wavefronts of one K-group, over rows
@@ -376,7 +377,7 @@ hipError_t launch_rows(const GemmParams &p, hipStream_t s) {
         if (p.k >= 6144 && p.k % 256 == 0) return launch_rows<kEpi, kMF, kNF, kF32, 256>(p, s);
     }
     constexpr int kFrags = kMF + kNF * (kEpi == kGemmEpiSiluGateF16 || kEpi == kGemmEpiSiluGateF32 ? 2 : 1);
-    constexpr int kBK = kBKFixed > 0 ? kBKFixed : kFrags <= 13 ? 128 : 64;
+    constexpr int kBK = kBKFixed > 0 ? kBKFixed : kFrags <= kRowsFrags128 ? 128 : 64;
     constexpr int kFit = (kMF == 1 && kFrags <= 5 ? 80 : 160) * 32 / (kFrags * kBK); // units of kFrags * 32 * kBK bytes
     constexpr int kStages = kFit > 8 ? 8 : kFit > 6 && kMF > 1 ? 6 : kFit;
     constexpr int kCH = kEpi == kGemmEpiSiluGateF16 || (kBK == 64 && kEpi != kGemmEpiSiluGateF32) ? 2 : 1;

@@ -202,6 +202,8 @@ hipError_t launch_gemm_f16_skinny(const GemmParams &p, int epilogue, hipStream_t
 int gemm_f16_rows_pieces(const GemmParams &p, int epilogue);
 // whether w1 and w3 are better as two products, each cut along K, than in one pass (gemm_dma.hip)
 bool gemm_f16_gate_cut(const GemmParams &p);
+// whether 64-column tiles of a product make one round that is worth it, so that it is not cut along K (gemm_dma.hip)
+bool gemm_f16_narrow(const GemmParams &p);
 hipError_t launch_gemm_f16_rows(const GemmParams &p, int epilogue, hipStream_t s); // p: one that gemm_f16_rows_pieces takes, or its pieces
 // the same for fp32 operands (gemm_rows_f32.hip); 0: the product is for the other kernels
 int gemm_f32_rows_pieces(const GemmParams &p, int epilogue);

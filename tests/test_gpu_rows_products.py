@@ -47,6 +47,21 @@ def test_what_stays_on_the_other_kernels(ctx):
         assert np.array_equal(got, want) == same
 
 
+# (rows, columns, K, whether the kernels for any number of rows take it): more than one round of workgroups; cut where their tiles make one round; A beyond an L2;
+# each beside sizes on the other side of the line
+@pytest.mark.parametrize("m,n,k,other", [(65, 16448, 256, True), (64, 16448, 256, False), (65, 16384, 256, False), (112, 32000, 256, True), (96, 1536, 1536, True),
+                                         (64, 1536, 1536, False), (96, 768, 1536, False), (97, 3072, 2560, True), (96, 3072, 2560, False),
+                                         (160, 1024, 10752, True), (160, 1024, 10624, False)])
+def test_what_the_other_kernels_do_better(ctx, m, n, k, other):
+    rng = np.random.default_rng(m + n + k)
+    a, b = _f16(rng, m, k, 1.0), _f16(rng, n, k, 0.05)
+    A, B = Tensor.from_numpy(ctx, a), Tensor.from_numpy(ctx, b)
+    got = A.matrix_mul_transposed(B).to_numpy()
+    _check(got, a, b)
+    with options(ctx, GEMM_ROWS="0"):
+        assert np.array_equal(got, A.matrix_mul_transposed(B).to_numpy()) == other
+
+
 # whole prompts and the token behind them: residual, SiLU-gate and RoPE / cache / V^T epilogues, whole sums and pieces (ffn 6144), head dimensions
 # 16 to 128, V^T read past the last row by the next attention kernel's tiles
 @pytest.mark.parametrize("dim,heads,ffn", [(1024, 16, 2816), (1152, 9, 3072), (1024, 64, 1024), (2048, 64, 6144)])
