@@ -5,7 +5,7 @@
 // many as let all workgroups run in one round up to 16384 columns (more take more rounds); its wavefronts split K (K-group g takes the g-th 32 halves of every unit of K), so that
 // an operand byte is written to LDS once and read back once or twice; and the weights are swept in whole 256-byte pieces
 // of rows.  Every workgroup starts at another unit of K: workgroups in step ask for the same columns of all rows, i.e. for
-// addresses a whole row apart, and those meet in few memory channels (8 rows, 12288 x 4096: 21.3 us in step, 18.2 apart).  The
+// addresses a whole row apart, and those meet in few memory channels.  The
 // partial sums of the K-groups are added through LDS in the order of the groups: deterministic, whole sums in the epilogue.
 //
 // What bounds it: few rows, memory (8 rows, us: wq|wk|wv 12288 x 4096 24.8 -> 18.3, w1|w3 11008 x 4096 39.5 -> 31.8 = 5.7 TB/s, w2 4096 x 11008
@@ -74,7 +74,11 @@ __global__ __launch_bounds__(2 * kBK * kRH * kCH) void gemm_f16_rows_kernel(Gemm
         cnt = q + (z < r ? 1 : 0);
         u0 = z * q + min(z, r);
     }
-    const int rot = (int)(((unsigned)(bx >> 3) * 5u + (unsigned)(bx & 7)) % (unsigned)cnt); // 8 XCDs: the workgroups of one L2 are 8 apart
+    // Where a workgroup starts: apart from those of its XCD, which are 8 launches apart, and from the other XCDs.  Chosen by time: among bx, bx >> 3 and bx & 7
+    // plus 1, 3, 5 or 7 times bx >> 3 all are within 1.2 % over 15 products of 2 to 131 rows (in step 3.5 % slower, apart by XCD only 2.8), and 5 is the
+    // fastest where it matters, long rows (8 rows, us, in step / bx / 1 / 3 / 5 / 7: 4096 x 11008 21.0 / 18.9 / 18.8 / 17.7 / 17.4 / 18.2, 24576 x 8192
+    // 77.6 / 72.9 / 70.4 / 68.9 / 68.5 / 70.1).  It decides the order of the fp32 sums; any order is as good.
+    const int rot = (int)(((unsigned)(bx >> 3) * 5u + (unsigned)(bx & 7)) % (unsigned)cnt);
 
     // ---- staging: rows of B (then of B2), then of A, 16-byte chunk c of row r at chunk c ^ swz(r): conflict-free fragment reads, and free
     //      here because every lane names its own global address.  Groups of kRpl rows (1 KiB) are dealt round-robin to the wavefronts.
