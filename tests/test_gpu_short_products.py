@@ -1,5 +1,6 @@
 """f16 products of short prompts: the kernel for at most 16 rows, and the row heights of the 64-column tiles that keep a product
-(or w1 and w3 in one pass) in one round of workgroups."""
+(or w1 and w3 in one pass) in one round of workgroups.  The kernel for at most 160 rows takes many of these sizes (test_gpu_rows_products.py); GEMM_ROWS=0
+keeps it away where another one is meant."""
 import numpy as np
 import pytest
 
@@ -58,33 +59,42 @@ def test_product_of_few_rows(ctx, m, n, k):
 @pytest.mark.parametrize("m,n,k", [(16, 2048, 5632), (2, 1024, 11008), (12, 6144, 2560), (8, 16384, 1408), (8, 5120, 1280), (3, 2048, 6912)])
 def test_few_rows_that_the_tiled_kernels_do_better(ctx, m, n, k):
     rng = np.random.default_rng(m + n + k)
-    A, B = (Tensor.from_numpy(ctx, _f16(rng, r, k, std)) for r, std in ((m, 1.0), (n, 0.05)))
-    got = A.matrix_mul_transposed(B).to_numpy()
-    with options(ctx, GEMM_SKINNY="0"):
+    a, b = _f16(rng, m, k, 1.0), _f16(rng, n, k, 0.05)
+    A, B = Tensor.from_numpy(ctx, a), Tensor.from_numpy(ctx, b)
+    with options(ctx, GEMM_ROWS="0"):
+        got = A.matrix_mul_transposed(B).to_numpy()
+    _check(got, a, b)
+    with options(ctx, GEMM_ROWS="0", GEMM_SKINNY="0"):
         assert np.array_equal(got, A.matrix_mul_transposed(B).to_numpy())
 
 
 def test_two_products_of_few_rows_on_more_workgroups_than_compute_units(ctx):
     rng = np.random.default_rng(95)
-    A, W1, W3 = (Tensor.from_numpy(ctx, _f16(rng, r, 2048, std)) for r, std in ((16, 1.0), (5632, 0.05), (5632, 0.05)))
-    got = A.ffn_gate(W1, W3).to_numpy()
-    with options(ctx, GEMM_SKINNY="0"):
+    a, w1, w3 = _f16(rng, 16, 2048, 1.0), _f16(rng, 5632, 2048, 0.05), _f16(rng, 5632, 2048, 0.05)
+    A, W1, W3 = (Tensor.from_numpy(ctx, t) for t in (a, w1, w3))
+    with options(ctx, GEMM_ROWS="0"):
+        got = A.ffn_gate(W1, W3).to_numpy()
+    _check_gate(got, a, w1, w3)
+    with options(ctx, GEMM_ROWS="0", GEMM_SKINNY="0"):
         assert np.array_equal(got, A.ffn_gate(W1, W3).to_numpy())
 
 
-@pytest.mark.parametrize("dim,heads,ffn", [(1024, 16, 2816), (1024, 8, 1024), (1024, 64, 1056)])
+# 17 heads of 64: K that only this kernel takes
+@pytest.mark.parametrize("dim,heads,ffn", [(1024, 16, 2816), (1024, 8, 1024), (1024, 64, 1056), (1088, 17, 2880)])
 @pytest.mark.parametrize("n", [2, 15, 16, 17])
-def test_prompt_of_few_rows(ctx, dim, heads, ffn, n):
+@pytest.mark.parametrize("rows", ["1", "0"])
+def test_prompt_of_few_rows(ctx, dim, heads, ffn, n, rows):
     """A whole prompt and the token behind it, head dimensions 64, 128 and 16: residual, SiLU-gate and RoPE / cache / V^T epilogues."""
     shape = Shape(dim=dim, n_layers=2, n_heads=heads, ffn_hidden=ffn, vocab_size=64, max_seq_len=80)
     W = synth_weights(shape, seed=91, std=0.05, norm_ones=False)
     toks = np.random.default_rng(92).integers(0, shape.vocab_size, 71)
     om, gm = make_oracle(shape, W, True), make_gpu(ctx, shape, W, True)
     gc, oc = gm.make_caches(), om.make_caches()
-    gm.forward(toks[:70], 0, gc)  # leaves other rows' values in the work buffers
-    gc = gm.make_caches()
-    assert max_rel_err(gm.forward(toks[:n], 0, gc), om.forward(toks[:n], 0, oc)) < TOL_F16
-    assert max_rel_err(gm.forward(toks[n:n + 1], n, gc), om.forward(toks[n:n + 1], n, oc)) < TOL_F16
+    with options(ctx, GEMM_ROWS=rows):
+        gm.forward(toks[:70], 0, gc)  # leaves other rows' values in the work buffers
+        gc = gm.make_caches()
+        assert max_rel_err(gm.forward(toks[:n], 0, gc), om.forward(toks[:n], 0, oc)) < TOL_F16
+        assert max_rel_err(gm.forward(toks[n:n + 1], n, gc), om.forward(toks[n:n + 1], n, oc)) < TOL_F16
     gm.free()
 
 
@@ -95,7 +105,8 @@ def test_lowest_row_tile_in_one_round(ctx, m, n, k):
     rng = np.random.default_rng(m + n + k)
     a, b, w3 = _f16(rng, m, k, 1.0), _f16(rng, n, k, 0.05), _f16(rng, n, k, 0.05)
     A, B, W3 = (Tensor.from_numpy(ctx, t) for t in (a, b, w3))
-    _check(A.matrix_mul_transposed(B).to_numpy(), a, b)
+    with options(ctx, GEMM_ROWS="0"):
+        _check(A.matrix_mul_transposed(B).to_numpy(), a, b)
     got = A.ffn_gate(B, W3).to_numpy()
     with options(ctx, GEMM_DUAL="1"):  # another tile, the same order of additions
         assert np.array_equal(got, A.ffn_gate(B, W3).to_numpy())
@@ -125,6 +136,7 @@ def test_prompt_on_narrow_tiles(ctx, dim, heads, ffn, rows):
     om, gm = make_oracle(shape, W, True), make_gpu(ctx, shape, W, True)
     for n in rows:
         gc, oc = gm.make_caches(), om.make_caches()
-        assert max_rel_err(gm.forward(toks[:n], 0, gc), om.forward(toks[:n], 0, oc)) < TOL_F16, n
+        with options(ctx, GEMM_ROWS="0"):
+            assert max_rel_err(gm.forward(toks[:n], 0, gc), om.forward(toks[:n], 0, oc)) < TOL_F16, n
         assert max_rel_err(gm.forward(toks[n:n + 1], n, gc), om.forward(toks[n:n + 1], n, oc)) < TOL_F16, n
     gm.free()
