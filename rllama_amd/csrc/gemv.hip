@@ -44,7 +44,7 @@ __global__ __launch_bounds__(kGemvThreads) void gemv_kernel(GemvParams p) {
     // 4096 x 11008 17.6 -> 16.9; 13B shape: wq|wk|wv 27.3 -> 27.05, wo 10.8 -> 10.6, w2 24.3 -> 24.15; w1|w3 has done it since
     // it was worth 1.6 % there.  (Issued behind the first of w2's two batches of x it cost 0.4 us instead: the second batch
     // waits behind the burst.  With a test for it inside the main loop the 13B wq|wk|wv lost 0.6 us.)  The output head with the
-    // greedy pick gains nothing from it and does not do it.
+    // greedy pick gains nothing from it on long rows and does not do it there; short rows (kGroup > 0) always do.
     // (The stamped measurement build keeps the burst behind the prologue, so that "x staged" and "first burst" stay two phases.)
     constexpr int kPre = (!kStamp && ((RLH_GEMV_PRELOAD_EPIS >> kEpi) & 1)) ? kPreSelf : kPreNone;
     gemv_body<WT, XT, kEpi, kStream, kPre, kBurst, kEmbed, kStamp, kGroup, kPV>(p, smem_raw, red, rope_f);
@@ -136,10 +136,13 @@ static hipError_t launch_gemv_t(GemvParams p, hipStream_t s) {
 
 template <int kEpi>
 static hipError_t launch_gemv_e(const GemvParams &p, hipStream_t s) {
-    if (p.w_is_f16) {
-        return p.x_f16 ? launch_gemv_t<half_t, half_t, kEpi>(p, s) : launch_gemv_t<half_t, float, kEpi>(p, s);
+    if (p.w_is_f16 && p.x_f16) return launch_gemv_t<half_t, half_t, kEpi>(p, s);
+    if (!p.w_is_f16 && !p.x_f16) return launch_gemv_t<float, float, kEpi>(p, s);
+    if constexpr (kEpi == kEpiStore) { // (a layer's fused products round x where its weights are f16, and only there)
+        if (p.w_is_f16) return launch_gemv_t<half_t, float, kEpi>(p, s);
+        return launch_gemv_t<float, half_t, kEpi>(p, s);
     }
-    return p.x_f16 ? launch_gemv_t<float, half_t, kEpi>(p, s) : launch_gemv_t<float, float, kEpi>(p, s);
+    return hipErrorInvalidValue;
 }
 
 hipError_t launch_gemv_stamped(const GemvParams &p, hipStream_t s, int stamps_capacity_waves, int *n_waves) {
