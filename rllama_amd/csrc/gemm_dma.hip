@@ -858,6 +858,7 @@ __global__ __launch_bounds__(kFinishThreads) void gemm_split_finish_norm_kernel(
 // this, us: 3072 x 1024 weights, 40 / 131 / 300 / 600 rows: 11.8 / 13.8 / 15.5 / 20.4 -> 7.4 / 7.8 / 9.4 / 11.0; 6144 x 2048, 20 / 40 / 80 / 200:
 // 17.2 / 22.0 / 26.0 / 18.4 -> 11.8 / 12.0 / 13.8 / 16.8; 3072 x 3072, 20 / 131 / 300: 19.5 / 25.8 / 20.3 -> 15.5 / 16.5 / 19.9; 1024 x 2816, 131 / 300:
 // 15.4 / 26.2 -> 14.6 / 15.0, but 20 / 40 rows (16 / 32 workgroups): 11.3 / 13.5 against 14.5 / 14.6; 4096 x 4096, 80 rows: 18.7 against 20.2.
+// (Up to 160 rows most products whose K is a multiple of 128 go to gemm_rows_device.h; the figures compare the kernels for the others.)
 static int choose_narrow(const GemmParams &p) {
     if (p.f32_operands || p.batch != 1 || p.split_k > 1 || p.k_seg != 0 || p.causal != 0 || p.b2 != nullptr || p.k % 64 != 0 || p.k < 1024 || p.k > 3072) return -1; // (measured from 1024 on)
     if (p.tune.tile_plus1 != 0 || p.tune.split_k > 1) return -1;
@@ -973,7 +974,7 @@ static int choose_dual(const GemmParams &p, int *cut_cols = nullptr) {
     // 2816 x 1024 weights, 40 / 80 / 131 / 200 / 300 / 600 rows: 11.3 / 12.1 / 27.0 / 30.1 / 30.7 / 37.7 -> 10.4 / 10.3 / 10.4 / 12.1 / 12.5 / 14.1;
     // 5632 x 2048, 131 / 200 / 400 rows: 36.7 / 38.7 / 48.1 -> 22.4 / 22.6 / 36.7; 7B shape, 131 / 160 / 192 / 256: 96 / 95 / 95 / 97 -> 62 / 60 /
     // 65 / 80; 13B shape: 124 / 123 / 129 / 132 -> 91 / 91 / 96 / 115.  Beyond one round (65B shape, 344 workgroups) it gains 4 % up to
-    // 192 rows and loses 16 % at 256.
+    // 192 rows and loses 16 % at 256.  (Of these, prompts of at most 160 rows with K a multiple of 128 go to gemm_rows_device.h now; rlh_ffn_gate beyond 16 rows comes here.)
     if (gemm_f16_gate_cut(p)) return 0;
     const int n_cu = p.compute_units;
     const int heights[5] = {32, 64, 128, 192, 256};

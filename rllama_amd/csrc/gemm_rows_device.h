@@ -1,16 +1,16 @@
 // gemm_rows_device.h -- C = A * B^T (f16 operands, fp32 accumulate) for prompts of up to 160 rows, one row tile for all of them.
 //
 // With so few rows the product is one pass over the weights B, and what a compute unit can take in bounds it: from memory while the rows
-// are few, from L2 (every workgroup stages all of A) when they are many.  So a workgroup owns all rows and 16 to 64 columns, as
-// many as let all workgroups run in one round up to 16384 columns (more take more rounds); its wavefronts split K (K-group g takes the g-th 32 halves of every unit of K), so that
-// an operand byte is written to LDS once and read back once or twice; and the weights are swept in whole 256-byte pieces
-// of rows.  Every workgroup starts at another unit of K: workgroups in step ask for the same columns of all rows, i.e. for
-// addresses a whole row apart, and those meet in few memory channels.  The
-// partial sums of the K-groups are added through LDS in the order of the groups: deterministic, whole sums in the epilogue.
+// are few, from L2 (every workgroup stages all of A) when they are many.  So a workgroup owns all rows and 16 to 64 columns: few
+// enough that every compute unit has work, and up to 16384 columns enough that all workgroups run in one round (more columns take more rounds, where
+// gemm_rows.hip compares with the other kernels).  Its wavefronts split K (K-group g takes the g-th 32 halves of every unit of K), so that an operand
+// byte is written to LDS once and read back once or twice; and the weights are swept in whole 256-byte pieces of rows.  Every workgroup starts
+// at another unit of K: workgroups in step ask for the same columns of all rows, i.e. for addresses a whole row apart, and those meet in few memory
+// channels.  The partial sums of the K-groups are added through LDS in the order of the groups: deterministic, whole sums in the epilogue.
 //
-// What bounds it: few rows, memory (8 rows, us: wq|wk|wv 12288 x 4096 24.8 -> 18.3, w1|w3 11008 x 4096 39.5 -> 31.8 = 5.7 TB/s, w2 4096 x 11008
-// 20.3 + 5.6 for adding the pieces -> 17.3); many rows, what a compute unit takes from L2 into LDS, 50 to 70 GB/s here (131 rows:
-// wq|wk|wv 44 -> 33, w1|w3 58 -> 44; spreading the requests over the MFMAs, wavefronts of their own for them and units of 64 change
+// What bounds it: few rows, memory (inside a prompt of 8 rows, us: wq|wk|wv 12288 x 4096 24.8 -> 20.0, w1|w3 11008 x 4096 39.5 -> 33.2 = 5.4 TB/s, w2
+// 4096 x 11008 20.3 + 5.6 for adding the pieces -> 17.2); many rows, what a compute unit takes from L2 into LDS, 45 to 50 GB/s here (131 rows:
+// wq|wk|wv 44 -> 35.8, w1|w3 58 -> 44; spreading the requests over the MFMAs, wavefronts of their own for them and units of 64 change
 // nothing there).  Time to the first token, former kernels -> this: 7B shape 8 / 131 rows 3.61 -> 3.03 / 5.83 -> 4.72 ms; dim 2304, 10 layers,
 // 8 / 24 / 64 rows 754 / 908 / 1001 -> 564 / 632 / 735 us; dim 2816, 8 layers, 112 / 144 rows 1095 / 1128 -> 832 / 910; dim 5120, 4 layers,
 // 8 / 64 / 144 rows 754 / 932 / 1060 -> 649 / 763 / 982.  Beyond 160 rows the operand of activations alone fills the LDS.

@@ -10,7 +10,9 @@
 // whole sums: no second kernel.
 //
 // Products whose K is a multiple of 128 and whose columns are a multiple of 8 go to gemm_rows_device.h instead, which sweeps whole
-// 256-byte pieces of rows and is faster (dim 2304, 10 layers, 8 rows: 754 -> 564 us to the first token); the figures here are of the others.
+// 256-byte pieces of rows and is faster (dim 2304, 10 layers, 8 rows: 754 -> 564 us to the first token).  Left here are other K, such as an odd
+// number of heads of 64 (f16 prompts of dim 1088), other numbers of columns, and what GEMM_ROWS=0 sends here; the figures below, taken in part at multiples of
+// 128, compare this kernel with the tiled ones.
 //
 // What bounds it: small products by the latency of their launches, larger ones by what the memory path takes in 64-byte pieces.
 // Time to the first token at 2 / 8 / 16 rows, ms, tiled kernels -> this: dim 1024, 8 layers 0.50 / 0.52 / 0.53 -> 0.41 / 0.43 / 0.44; dim 2048,
