@@ -375,8 +375,10 @@ inline int rows_columns(const GemmParams &p, int pieces) {
 template <int kEpi, int kMF, int kNF, bool kF32, int kBKFixed = 0>
 hipError_t launch_rows(const GemmParams &p, hipStream_t s) {
     // Units of 128 halves (whole 256-byte pieces of rows) while at least three fit the LDS, else of 64.  One fragment of rows and few
-    // columns: 80 KB, so that two workgroups share a compute unit, and for long rows units of 256, i.e. twice the wavefronts (8 rows,
-    // 4096 x 4096: 9.1 us with units of 128, 10.8 with 256; 4096 x 11008: 19.7 and 17.2).
+    // columns: 80 KB, so that two workgroups share a compute unit, and for long rows units of 256, i.e. twice the wavefronts.  2 to 16
+    // rows of 1024 to 8192 columns, K = 6144 to 22016, units of 256 against 128: 0.86 to 1.07 of the time, mean 0.98, but 5120 columns (a quarter more
+    // than one workgroup per compute unit) 1.0 to 1.13 up to K = 11008.  Below 6144 it depends on the columns alike (0.87 to 1.0 up to 4096 of them, 1.0 to 1.15 at
+    // 5120 and 6656); with the residual and its norm, 4096 x 4096 of 8 rows: 9.1 us with units of 128, 10.8 with 256.
     if constexpr (kMF == 1 && kNF <= 2 && kBKFixed == 0 && !kF32 && kEpi != kGemmEpiSiluGateF16) {
         if (p.k >= 6144 && p.k % 256 == 0) return launch_rows<kEpi, kMF, kNF, kF32, 256>(p, s);
     }
