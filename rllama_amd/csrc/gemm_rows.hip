@@ -13,7 +13,7 @@ static bool rows_beyond_l2(const GemmParams &p, int pieces, long rounds) { retur
 // Microseconds of a product in `pieces` pieces with what has to follow it: a launch, then what one compute unit stages at 45 GB/s (twice that
 // where at most an eighth of them work) or all of the weights at 5.6 TB/s.  Units of 128 halves are staged slower where A is beyond the L2
 // (8192 x 22016, 128 rows: one round of 2 pieces 149 us, two rounds of 4 pieces 108).  Partial sums are written and read back at 2.5 TB/s, all in
-// all (taken as 4.7, 12288 x 6144 of 160 rows ran in 4 pieces, 65 us, and 512 x 4096 of 2 rows in 8, 9.2 us; 56 and 5.0 in one).
+// all (taken as 4.7, 12288 x 6144 of 160 rows ran in 4 pieces, 65 us, and 512 x 4096 of 2 rows in 8, 9.2 us; 47 and 5.0 in one).
 // The kernel that adds the pieces brings the RMSNorm behind a residual product along.
 static double rows_us(const GemmParams &p, int epilogue, int pieces) {
     const double k = ((p.k / 128 + pieces - 1) / pieces) * 128.0;
